@@ -261,15 +261,18 @@ HBTX_HD uint64_t key_prefix(uint64_t k, int l)
 // Softened pair potential inside the kernel radius h, in units where the final
 // sum is multiplied by G/a: the GADGET-2 cubic-spline polynomial of
 // src/gravity_tree.cpp:150-162 (outside h the term is -m/r).  rinv = 1/sqrt(r2).
+// (the fused multiply-adds are written out, so that every kernel rounds alike)
 HBTX_DEV float spline_near(float r2, float rinv, float m, float hinv)
 {
+#pragma clang fp contract(off)
   const float r = (r2 > 0.f) ? r2 * rinv : 0.f;
   const float u = r * hinv;
   const float u2 = u * u;
-  const float inner = -2.8f + u2 * (5.333333333333f + u2 * (6.4f * u - 9.6f));
-  const float outer = -3.2f + 0.066666666667f * __builtin_amdgcn_rcpf(u) +
-                      u2 * (10.666666666667f + u * (-16.0f + u * (9.6f - 2.133333333333f * u)));
-  return m * hinv * ((u < 0.5f) ? inner : outer);
+  const float inner = __builtin_fmaf(u2, __builtin_fmaf(u2, __builtin_fmaf(u, 6.4f, -9.6f), 5.333333333333f), -2.8f);
+  const float po = __builtin_fmaf(u, __builtin_fmaf(u, __builtin_fmaf(u, -2.133333333333f, 9.6f), -16.0f),
+                                  10.666666666667f);
+  const float outer = __builtin_fmaf(u2, po, __builtin_fmaf(__builtin_amdgcn_rcpf(u), 0.066666666667f, -3.2f));
+  return (m * hinv) * ((u < 0.5f) ? inner : outer);
 }
 
 // Kahan-compensated accumulation of FP32 terms.
@@ -283,6 +286,7 @@ struct Kahan
   }
   HBTX_DEV void add(float x)
   {
+#pragma clang fp contract(off)
     float y = x - c;
     float t = s + y;
     c = (t - s) - y;

@@ -1656,6 +1656,27 @@ void build_tree(hbtx_ctx *c, const hbtx_params &prm, int64_t n, const float *pos
   B.ran = false;
 }
 
+// Potentials at A's targets: the tree walk, or the exact sum over the records.
+// The exact sum takes several waves per 64 targets up to DS_ITEMS_PER_CU times 64
+// targets a CU; beyond that one wave per 64 targets keeps the chip as full, without
+// the exchange (20,011 sources, one wave against several: 30,001 targets 2087 and
+// 241 us, 131,072 targets 1382 and 1035 us, 262,144 targets 1765 and 1971 us).
+#define DS_ITEMS_PER_CU 12
+template <bool PERIODIC, bool STATS>
+void launch_points(hbtx_ctx *c, const PointArgs &A)
+{
+  const int64_t nt = A.ntgt;
+  const int64_t items = (nt + HBTX_WAVE - 1) / HBTX_WAVE;
+  if (!A.treemode && items <= (int64_t)DS_ITEMS_PER_CU * c->num_cu)
+  {
+    k_points_direct<PERIODIC, STATS>
+      <<<(unsigned)std::max<int64_t>(1, items), DS_THREADS, 0, c->stream>>>(A);
+    return;
+  }
+  const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(nt / HBTX_WAVE + 1, 32 * c->num_cu) / HBTX_WALK_WG_WAVES);
+  k_points_potential<PERIODIC, STATS><<<grid, WALK_WG_THREADS, 0, c->stream>>>(A);
+}
+
 void tree_points(hbtx_ctx *c, hbtx_tree *T, int64_t nt, const float *tpos, const float *tmass, double *out)
 {
   REQUIRE(nt >= 0 && nt < (int64_t)0x20000000, HBTX_E_INVALID, "bad target count");
@@ -1702,23 +1723,11 @@ void tree_points(hbtx_ctx *c, hbtx_tree *T, int64_t nt, const float *tpos, const
   A.overflow = counter.p + 1;
   A.P = T->P;
   HIPCHK(hipMemsetAsync(c->stats.p, 0, NSTATS * sizeof(unsigned long long), st));
-  const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(nt / HBTX_WAVE + 1, 32 * c->num_cu) /
-                                                 HBTX_WALK_WG_WAVES);
   HIPCHK(hipEventRecord(c->wev0, st));
   if (T->P.periodic)
-  {
-    if (c->count_work)
-      k_points_potential<true, true><<<grid, WALK_WG_THREADS, 0, st>>>(A);
-    else
-      k_points_potential<true, false><<<grid, WALK_WG_THREADS, 0, st>>>(A);
-  }
+    c->count_work ? launch_points<true, true>(c, A) : launch_points<true, false>(c, A);
   else
-  {
-    if (c->count_work)
-      k_points_potential<false, true><<<grid, WALK_WG_THREADS, 0, st>>>(A);
-    else
-      k_points_potential<false, false><<<grid, WALK_WG_THREADS, 0, st>>>(A);
-  }
+    c->count_work ? launch_points<false, true>(c, A) : launch_points<false, false>(c, A);
   HIPCHK(hipEventRecord(c->wev1, st));
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(out, phid.p, nt * sizeof(double), hipMemcpyDeviceToHost, st));
@@ -2202,12 +2211,7 @@ int hbtx_direct_potential_noalloc(hbtx_ctx *c, const hbtx_params *prm, int64_t n
       A.stats = nullptr;
       A.overflow = nullptr; // direct sums only
       A.P = P;
-      const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(n_tgt / HBTX_WAVE + 1, 32 * c->num_cu) /
-                                                     HBTX_WALK_WG_WAVES);
-      if (P.periodic)
-        k_points_potential<true, false><<<grid, WALK_WG_THREADS, 0, st>>>(A);
-      else
-        k_points_potential<false, false><<<grid, WALK_WG_THREADS, 0, st>>>(A);
+      P.periodic ? launch_points<true, false>(c, A) : launch_points<false, false>(c, A);
     }
     HIPCHK(hipGetLastError());
   });

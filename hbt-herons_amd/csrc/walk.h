@@ -15,6 +15,7 @@
 // correction update (src/subhalo_unbind.cpp:577-589).
 #pragma once
 #include "common.h"
+#include <type_traits>
 
 namespace hbtx
 {
@@ -64,9 +65,12 @@ HBTX_DEV uint64_t wave_mask(bool p)
   return __builtin_amdgcn_ballot_w64(p);
 }
 
-template <bool PERIODIC>
+// Squared distance with the fused multiply-adds written out, so that every kernel
+// rounds alike: the x square first where XFIRST, else the y square.
+template <bool PERIODIC, bool XFIRST>
 HBTX_DEV float sep2(float ex, float ey, float ez, float px, float py, float pz, const DevParams &P)
 {
+#pragma clang fp contract(off)
   float dx, dy, dz;
   if (PERIODIC)
   {
@@ -80,7 +84,7 @@ HBTX_DEV float sep2(float ex, float ey, float ez, float px, float py, float pz, 
     dy = ey - py;
     dz = ez - pz;
   }
-  return dx * dx + dy * dy + dz * dz;
+  return __builtin_fmaf(dz, dz, XFIRST ? __builtin_fmaf(dy, dy, dx * dx) : __builtin_fmaf(dx, dx, dy * dy));
 }
 
 // Per-wave work counters of one walk (uniform values, kept only in the stats
@@ -239,15 +243,19 @@ HBTX_DEV void tree_walk_stack(const uint2 *wt, int ub, int ue, bool valid, float
     // or the spline where N; the sum runs under the accepting lanes' exec mask,
     // so that a lane that does not accept never uses its 1/r (infinite where the
     // record is the target itself).  A cell's visit returns the lanes that opened it.
+    using XF = std::true_type;
+    using YF = std::false_type;
     float4 rn = rec[0];
     float2 wn = aw[0];
-    auto visit = [&](int j, bool is_cell) -> uint64_t {
+    // (xf: the first of a group of four and the records past the last group square x
+    // first, the others y)
+    auto visit = [&](int j, bool is_cell, auto xf) -> uint64_t {
       // record j was read ahead; read record j + 1 while it is evaluated
       const float4 r = rn;
       const float2 w = wn;
       rn = rec[j + 1];
       wn = aw[2 * (j + 1)];
-      const float r2 = sep2<PERIODIC>(r.x, r.y, r.z, px, py, pz, P);
+      const float r2 = sep2<PERIODIC, decltype(xf)::value>(r.x, r.y, r.z, px, py, pz, P);
       const uint64_t rm = __builtin_amdgcn_uicmp(__float_as_uint(w.y) & bit, 0u, 33 /* ne */);
       const uint64_t lm = is_cell ? __builtin_amdgcn_fcmpf(r2, w.x, 4 /* ordered < */) : 0ull;
       const uint64_t nm = __builtin_amdgcn_fcmpf(r2, P.h2, 4 /* ordered < */);
@@ -288,8 +296,8 @@ HBTX_DEV void tree_walk_stack(const uint2 *wt, int ub, int ue, bool valid, float
     int j = 0;
     for (; j + 4 <= ncell; j += 4)
     {
-      const uint64_t o0 = visit(j, true), o1 = visit(j + 1, true), o2 = visit(j + 2, true),
-                     o3 = visit(j + 3, true);
+      const uint64_t o0 = visit(j, true, XF()), o1 = visit(j + 1, true, YF()),
+                     o2 = visit(j + 2, true, YF()), o3 = visit(j + 3, true, YF());
       if (lane == 0)
       {
         omw[2 * j] = make_uint2((uint32_t)o0, (uint32_t)(o0 >> 32));
@@ -301,7 +309,7 @@ HBTX_DEV void tree_walk_stack(const uint2 *wt, int ub, int ue, bool valid, float
     }
     for (; j < ncell; j++)
     {
-      const uint64_t o = visit(j, true);
+      const uint64_t o = visit(j, true, XF());
       if (lane == 0)
         omw[2 * j] = make_uint2((uint32_t)o, (uint32_t)(o >> 32));
       block_end(1);
@@ -309,15 +317,15 @@ HBTX_DEV void tree_walk_stack(const uint2 *wt, int ub, int ue, bool valid, float
     // particles
     for (; j + 4 <= nb; j += 4)
     {
-      visit(j, false);
-      visit(j + 1, false);
-      visit(j + 2, false);
-      visit(j + 3, false);
+      visit(j, false, XF());
+      visit(j + 1, false, YF());
+      visit(j + 2, false, YF());
+      visit(j + 3, false, YF());
       block_end(4);
     }
     for (; j < nb; j++)
     {
-      visit(j, false);
+      visit(j, false, XF());
       block_end(1);
     }
     // push the chains' rests and the opened cells' children
@@ -351,7 +359,8 @@ HBTX_DEV void tree_walk_stack(const uint2 *wt, int ub, int ue, bool valid, float
 template <bool PERIODIC>
 HBTX_DEV float direct_term(const float4 e, float px, float py, float pz, const DevParams &P, bool &near)
 {
-  const float r2 = sep2<PERIODIC>(e.x, e.y, e.z, px, py, pz, P);
+#pragma clang fp contract(off)
+  const float r2 = sep2<PERIODIC, false>(e.x, e.y, e.z, px, py, pz, P);
   const float rinv = __builtin_amdgcn_rsqf(r2);
   float term = -e.w * rinv;
   const bool nr = r2 < P.h2;
@@ -376,28 +385,78 @@ HBTX_DEV void const_load_4rec(const uint2 *p, float4 r[4])
                        __int_as_float(a[4 * k + 3]));
 }
 
+// One group of four records against every lane's target: their terms' sum.
+template <bool PERIODIC>
+HBTX_DEV float direct_group(const float4 r[4], float px, float py, float pz, const DevParams &P, bool &nr)
+{
+#pragma clang fp contract(off)
+  float part = direct_term<PERIODIC>(r[0], px, py, pz, P, nr);
+  part += direct_term<PERIODIC>(r[1], px, py, pz, P, nr);
+  part += direct_term<PERIODIC>(r[2], px, py, pz, P, nr);
+  part += direct_term<PERIODIC>(r[3], px, py, pz, P, nr);
+  return part;
+}
+
+// The sums of groups [g0, g1) of a particle record list, in order, to emit(group,
+// sum).  The records come through scalar loads, AHEAD groups (64 bytes each) ahead:
+// a wave waits for its groups, sends the loads of the next ones and then evaluates
+// (scalar loads return in any order, so a wait covers every load in flight: it
+// has to come before the next ones go out).  Loading each group just before its use
+// left a wave waiting for the L2 once per group.
+template <bool PERIODIC, int AHEAD, class Emit>
+HBTX_DEV void direct_groups(const uint2 *ent, int g0, int g1, float px, float py, float pz, const DevParams &P,
+                            WalkCounts &wc, Emit emit)
+{
+  if (g0 >= g1)
+    return;
+  float4 a[AHEAD][4], b[AHEAD][4];
+  auto load = [&](int g, float4(&u)[AHEAD][4]) {
+#pragma unroll
+    for (int k = 0; k < AHEAD; k++)
+      const_load_4rec(ent + 8 * (int64_t)min(g + k, g1 - 1), u[k]); // (past the last group: the last again, unused)
+  };
+  auto arrived = [] {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt(0)
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto eval = [&](int g, float4(&u)[AHEAD][4]) {
+#pragma unroll
+    for (int k = 0; k < AHEAD; k++)
+    {
+      if (g + k >= g1)
+        break;
+      bool nr = false;
+      emit(g + k, direct_group<PERIODIC>(u[k], px, py, pz, P, nr));
+      wc.nnear += nr;
+    }
+  };
+  load(g0, a);
+  for (int g = g0; g < g1; g += 2 * AHEAD)
+  {
+    arrived();
+    load(g + AHEAD, b);
+    __builtin_amdgcn_sched_barrier(0);
+    eval(g, a);
+    if (g + AHEAD >= g1)
+      break;
+    arrived();
+    load(g + 2 * AHEAD, a);
+    __builtin_amdgcn_sched_barrier(0);
+    eval(g + AHEAD, b);
+  }
+}
+
 // Direct mode: the records are particles only (two units each), summed in
-// groups of four (one scalar load each), Kahan-compensated across groups.
+// groups of four, Kahan-compensated across groups.
 template <bool PERIODIC>
 HBTX_DEV void direct_sum(const uint2 *wt, int ub, int ue, float px, float py, float pz, const DevParams &P,
                          Kahan &acc, WalkCounts &wc)
 {
   const uint2 *ent = wt + ub;
   const int ee = (ue - ub) / 2;
-  int i = 0;
-  for (; i + 4 <= ee; i += 4)
-  {
-    float4 r[4];
-    const_load_4rec(ent + 2 * i, r);
-    bool nr = false;
-    float part = direct_term<PERIODIC>(r[0], px, py, pz, P, nr);
-    part += direct_term<PERIODIC>(r[1], px, py, pz, P, nr);
-    part += direct_term<PERIODIC>(r[2], px, py, pz, P, nr);
-    part += direct_term<PERIODIC>(r[3], px, py, pz, P, nr);
-    wc.nnear += nr;
-    acc.add(part);
-  }
-  for (; i < ee; i++)
+  direct_groups<PERIODIC, 1>(ent, 0, ee / 4, px, py, pz, P, wc, [&](int, float part) { acc.add(part); });
+  for (int i = ee & ~3; i < ee; i++)
   {
     bool nr = false;
     acc.add(direct_term<PERIODIC>(const_load_f4u(ent + 2 * i), px, py, pz, P, nr));
