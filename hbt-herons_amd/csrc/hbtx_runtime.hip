@@ -1660,7 +1660,7 @@ void build_tree(hbtx_ctx *c, const hbtx_params &prm, int64_t n, const float *pos
 // The exact sum takes several waves per 64 targets up to DS_ITEMS_PER_CU times 64
 // targets a CU; beyond that one wave per 64 targets keeps the chip as full, without
 // the exchange (20,011 sources, one wave against several: 30,001 targets 2087 and
-// 241 us, 131,072 targets 1382 and 1035 us, 262,144 targets 1765 and 1971 us).
+// 227 us, 131,072 targets 1382 and 957 us, 262,144 targets 1753 and 1971 us).
 #define DS_ITEMS_PER_CU 12
 template <bool PERIODIC, bool STATS>
 void launch_points(hbtx_ctx *c, const PointArgs &A)

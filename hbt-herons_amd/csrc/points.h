@@ -99,10 +99,12 @@ __global__ __launch_bounds__(WALK_WG_THREADS, 8) void k_points_potential(PointAr
 // stage, and one more wave adds them in order (four dependent operations a group,
 // about an eighth of a group's work) while the others form the next stage's.
 // 20,011 sources on 30,001 targets: 3104 us with one wave waiting for each group's
-// records, 2087 us with the records loaded ahead (direct_groups), 241 us here (2.5e12
-// pairs/s; the vector units alone allow about 3.0e12).
+// records, 2087 us with the records loaded ahead (direct_groups), 227 us here (2.6e12
+// pairs/s; the vector units alone allow about 3.0e12).  With 4 groups a wave and
+// stage it took 241 us, and 192 instead of 158 us on 8,000 targets: a stage starts
+// with its records not yet loaded, so longer stages wait less.
 #define DS_WAVES 8
-#define DS_GROUPS 4
+#define DS_GROUPS 8
 #define DS_THREADS (HBTX_WAVE * (DS_WAVES + 1))
 template <bool PERIODIC, bool STATS>
 __global__ __launch_bounds__(DS_THREADS) void k_points_direct(PointArgs A)
@@ -140,19 +142,19 @@ __global__ __launch_bounds__(DS_THREADS) void k_points_direct(PointArgs A)
       {
         const int n = min(DS_WAVES * DS_GROUPS, ng - (st - 1) * DS_WAVES * DS_GROUPS);
         const float(*b)[HBTX_WAVE] = parts[(st - 1) & 1];
-        if (n == DS_WAVES * DS_GROUPS)
+        int k0 = 0;
+        for (; k0 + 32 <= n; k0 += 32)
         {
-          float v[DS_WAVES * DS_GROUPS];
+          float v[32];
 #pragma unroll
-          for (int k = 0; k < DS_WAVES * DS_GROUPS; k++)
-            v[k] = b[k][lane];
+          for (int k = 0; k < 32; k++)
+            v[k] = b[k0 + k][lane];
 #pragma unroll
-          for (int k = 0; k < DS_WAVES * DS_GROUPS; k++)
+          for (int k = 0; k < 32; k++)
             acc.add(v[k]);
         }
-        else
-          for (int k = 0; k < n; k++)
-            acc.add(b[k][lane]);
+        for (int k = k0; k < n; k++)
+          acc.add(b[k][lane]);
       }
       __syncthreads();
     }

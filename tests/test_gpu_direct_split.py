@@ -10,10 +10,10 @@ import hbtx
 pytestmark = pytest.mark.gpu
 
 
-# source counts around a group (4 sources) and a stage (128 sources), targets around a wave
+# source counts around a group (4 sources), the adder's batch (128) and a stage (256), targets around a wave
 @pytest.mark.parametrize("periodic", [False, True])
 @pytest.mark.parametrize("ns,nt", [(1, 1), (3, 64), (4, 65), (5, 63), (127, 2), (128, 64), (129, 130), (131, 65),
-                                   (255, 7), (4099, 129)])
+                                   (255, 7), (256, 64), (257, 65), (4099, 129)])
 def test_split_sum_equals_the_wave_sum(ctx, ns, nt, periodic):
     rng = np.random.default_rng(ns * 1000 + nt)
     src = (rng.normal(0, 0.05, (ns, 3)) + 2.0).astype(np.float32)
