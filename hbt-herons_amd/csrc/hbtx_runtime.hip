@@ -15,6 +15,8 @@
 #include "tiles.h"
 #include "profile.h"
 #include "reassign.h"
+#include "load.h"
+#include "transfer.h"
 
 #define WALK_MAX_CHUNKS 16
 // entries whose walk records (at most 3 units each) keep unit offsets in int32
@@ -155,12 +157,15 @@ struct Batch
   bool has_type = false;
   bool has_u = false;
   bool has_proposal = false;
+  bool has_id = false;
   std::vector<int64_t> h_off;
-  std::vector<int64_t> h_id;
   std::vector<int32_t> h_count;
   // particles
   DArr<float4> posm, velu;
   DArr<int8_t> ptype;
+  DArr<int64_t> ids;     // particle ids (has_id), else a particle's id is its index in its subhalo
+  DArr<char> raw;        // the upload, where the walk records' buffer is too small for it
+  DArr<int32_t> load_bad;
   DArr<int32_t> sub_of, sub_zero, off, off_pairs, order, order_zero;
   DArr<int32_t> state, cur, cur2, src, src_sub, fvals, ford;
   DArr<float> energy, esl, selfm, fenergy, fpot, eref;
@@ -215,6 +220,7 @@ struct View
   SubArrays S;
   PartArrays Q;
   const int32_t *order;
+  const int64_t *ids; // null: a particle's id is its index in its subhalo
   int64_t p0; // first particle of the view in the batch
   int32_t s0; // first subhalo of the view
   int32_t *ford;
@@ -287,6 +293,7 @@ struct hbtx_ctx
   DArr<int4> red_tiles;
   DArr<double> red_partial;
   DArr<unsigned long long> stats;
+  Staging staging;
   hipEvent_t ev0 = nullptr, ev1 = nullptr, wev0 = nullptr, wev1 = nullptr;
   int64_t walk_items_hint = INT64_MAX; // work items of the previous round of the running view
   double walk_ms = 0.0;
@@ -300,7 +307,20 @@ struct hbtx_ctx
   int graph_rounds = 0, graph_captures = 0;
   int64_t tree_entries = 0, tree_entries_first = 0; // octree entries built, all rounds / first round
   Batch B;
-  // particle reassignment buffers (grow-only, reused across calls)
+  // workspaces of the calls that take host arrays (grow-only, reused across calls)
+  struct
+  {
+    DArr<float> raw;            // the arrays as uploaded
+    DArr<float4> tgt, posm;
+    DArr<double> phi;
+    DArr<uint64_t> keys;
+    DArr<int32_t> vals, seg, counter, off, sub_of, local;
+    DArr<hbtx_sub_result> res;
+    DArr<float> rc, mc, X;
+    DArr<uint8_t> y;
+    DArr<hbtx_sub_profile> prof;
+  } ws;
+  // particle reassignment buffers (likewise)
   struct
   {
     DArr<float> pos, radii;
@@ -570,13 +590,13 @@ int64_t entry_bound(int64_t n)
   int64_t e = n, w = 1;
   if (n < 2)
     return e;
-  for (int l = 0; l <= HBTX_KEY_LEVELS; l++)
-  {
-    e += std::min(w, n / 2);
-    w = std::min<int64_t>(w * 8, (int64_t)1 << 40);
-  }
-  return e;
+  int l = 0;
+  for (; l <= HBTX_KEY_LEVELS && w < n / 2; l++, w *= 8)
+    e += w;
+  return e + (HBTX_KEY_LEVELS + 1 - l) * (n / 2);
 }
+
+void grow_entries(Batch &B, int64_t need, bool slack);
 
 void batch_reserve(hbtx_ctx *c, Batch &B)
 {
@@ -585,6 +605,9 @@ void batch_reserve(hbtx_ctx *c, Batch &B)
   B.posm.alloc(n);
   B.velu.alloc(n);
   B.ptype.alloc(n);
+  if (B.has_id)
+    B.ids.alloc(n);
+  B.load_bad.alloc(1);
   B.sub_of.alloc(n);
   B.sub_zero.alloc(std::max<int64_t>(B.max_count, 1));
   B.off.alloc(ns + 1);
@@ -612,12 +635,7 @@ void batch_reserve(hbtx_ctx *c, Batch &B)
   B.flag64.alloc(n + 1);
   B.keys.alloc(n);
   B.lev.alloc(n + 1);
-  B.ent_cap = (int32_t)std::min<int64_t>(3 * n + 64, WREC_MAX_ENTRIES);
-  B.ent.alloc((int64_t)B.ent_cap + 1);
-  B.eskip.alloc((int64_t)B.ent_cap + 1);
-  B.ent_depth.alloc(((int64_t)B.ent_cap + 16) & ~(int64_t)15);
-  B.wt.alloc(3 * (int64_t)B.ent_cap + 4);
-  B.cell_u.alloc((int64_t)B.ent_cap + 1);
+  grow_entries(B, std::min<int64_t>(3 * n + 64, WREC_MAX_ENTRIES), false);
   B.items.alloc(n / HBTX_WAVE + ns + 1);
   B.icnt.alloc(ns + 1);
   B.iscan.alloc(ns + 1);
@@ -718,6 +736,7 @@ View make_view(Batch &B, int64_t p0, int64_t n, int32_t s0, int32_t nsub, bool w
   Q.cur2 = B.cur2.p + p0;
   Q.proposal = B.has_proposal ? B.proposal.p + p0 : nullptr;
   V.order = whole ? B.order.p : B.order_zero.p;
+  V.ids = B.has_id ? B.ids.p + p0 : nullptr;
   V.ford = B.ford.p + p0;
   V.fenergy = B.fenergy.p + p0;
   V.fpot = B.fpot.p + p0;
@@ -767,19 +786,15 @@ int32_t *round_ptr(Batch &B)
   return B.misc.p + 5;
 }
 
-// entry buffers for at least `need` entries (slack: a quarter more, for the next rounds)
-void grow_entries(Batch &B, int64_t need, bool slack = true)
+// entry buffers for at least `need` entries (slack: a quarter more, for the next
+// rounds); buffers that are large enough already stay
+void grow_entries(Batch &B, int64_t need, bool slack)
 {
   const int64_t cap = std::min<int64_t>(slack ? need + need / 4 + 64 : need, WREC_MAX_ENTRIES);
   REQUIRE(cap >= need, HBTX_E_CAPACITY, "tree entry count exceeds the walk-record range");
-  B.ent.release();
-  B.eskip.release();
-  B.ent_depth.release();
   B.ent.alloc(cap + 1);
   B.eskip.alloc(cap + 1);
   B.ent_depth.alloc((cap + 16) & ~(int64_t)15);
-  B.wt.release();
-  B.cell_u.release();
   B.wt.alloc(3 * cap + 4);
   B.cell_u.alloc(cap + 1);
   B.ent_cap = (int32_t)cap;
@@ -872,7 +887,7 @@ void build_sources_tree(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, cons
     REQUIRE(etot >= 0, HBTX_E_CAPACITY, "tree entry count overflows int32");
     if (etot > B.ent_cap)
     {
-      grow_entries(B, etot);
+      grow_entries(B, etot, true);
       T = tree_args(B, V, P);
     }
   }
@@ -1047,7 +1062,7 @@ __global__ void k_final_local(SubArrays S, int64_t n, const int32_t *vals, const
 
 __global__ void k_final_sub(SubArrays S, PartArrays Q, DevParams P, const int32_t *vals, const double *kin,
                             const double *core, const int32_t *first_tracer, const float *ref_in,
-                            hbtx_sub_result *out)
+                            const int64_t *ids, hbtx_sub_result *out)
 {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= S.nsub)
@@ -1129,6 +1144,11 @@ __global__ void k_final_sub(SubArrays S, PartArrays Q, DevParams P, const int32_
   }
   else
     R.tracer_index = 0;
+  if (nb > 0)
+  {
+    const int p = vals[S.off[s] + (int)R.tracer_index];
+    R.mostbound_id = ids ? ids[p] : (int64_t)(p - S.off[s]);
+  }
   const double *c = core + (int64_t)RED_NV * s;
   const double msum = c[0];
   double s2r = 0., s2v = 0.;
@@ -1192,7 +1212,7 @@ void run_final(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, bool want_pot
   k_first_tracer<<<gw, 256, 0, st>>>(V.S, V.Q, P, V.fvals, V.first_tracer);
   k_core_wave<<<gw, 256, 0, st>>>(V.S, V.Q, P, V.fvals, V.red2);
   k_final_sub<<<gs, 256, 0, st>>>(V.S, V.Q, P, V.fvals, V.red, V.red2, V.first_tracer, B.ref_in.p + 6 * V.s0,
-                                  V.dres);
+                                  V.ids, V.dres);
   if (want_pot)
     k_potential_energy<<<gb, 256, 0, st>>>(V.S, V.Q, P, n, V.fvals, V.fpot);
   HIPCHK(hipGetLastError());
@@ -1434,94 +1454,115 @@ void check_layout(int64_t n, int64_t nsub, const int64_t *offsets)
   }
 }
 
+// Subhaloes by particle count, largest first, equal counts in input order (three
+// counting passes over the 27 bits of a count).
+void size_order(const std::vector<int32_t> &count, std::vector<int32_t> &order)
+{
+  const size_t n = count.size();
+  std::vector<int32_t> tmp(n);
+  order.resize(n);
+  std::iota(order.begin(), order.end(), 0);
+  for (int pass = 0; pass < 3; pass++)
+  {
+    auto digit = [&](int32_t s) { return 511 - ((count[s] >> (9 * pass)) & 511); };
+    size_t start[513] = {0};
+    for (size_t i = 0; i < n; i++)
+      start[digit((int32_t)i) + 1]++;
+    for (int d = 0; d < 512; d++)
+      start[d + 1] += start[d];
+    for (size_t i = 0; i < n; i++)
+      tmp[start[digit(order[i])]++] = order[i];
+    order.swap(tmp);
+  }
+}
+
+// The caller's arrays as they are through pinned staging (transfer.h) into one
+// device block, and from there into the batch's layout (load.h).  vel, u, type, id,
+// mb_pos and mb_vel may be null.
 void upload_batch(hbtx_ctx *c, Batch &B, int64_t n, const float *pos, const float *vel, const float *mass,
                   const float *u, const int32_t *type, const int64_t *id, int64_t nsub, const int64_t *offsets,
                   const float *ref_pos, const float *ref_vel, const float *mb_pos, const float *mb_vel)
 {
   check_layout(n, nsub, offsets);
-  REQUIRE(pos && vel && mass && ref_pos && ref_vel, HBTX_E_INVALID, "null input array");
+  REQUIRE(pos && mass && ref_pos && ref_vel, HBTX_E_INVALID, "null input array");
   B.n = n;
   B.nsub = (int32_t)nsub;
   B.has_type = type != nullptr;
   B.has_u = u != nullptr;
+  B.has_id = id != nullptr;
   B.has_proposal = false;
   B.has_prev = false;
   B.egroups_min = -1;
   B.feat_full = false;
+  B.ran = false;
   B.h_off.assign(offsets, offsets + nsub + 1);
   B.h_count.resize(nsub);
   B.max_count = 0;
+  B.ent_bound = 0;
   for (int64_t s = 0; s < nsub; s++)
   {
     B.h_count[s] = (int32_t)(offsets[s + 1] - offsets[s]);
     B.max_count = std::max(B.max_count, B.h_count[s]);
-  }
-  B.ent_bound = 0;
-  for (int64_t s = 0; s < nsub; s++)
     B.ent_bound += entry_bound(B.h_count[s]);
-  if (id)
-    B.h_id.assign(id, id + n);
-  else
-  {
-    B.h_id.resize(n);
-    for (int64_t s = 0; s < nsub; s++)
-      for (int64_t i = offsets[s]; i < offsets[s + 1]; i++)
-        B.h_id[i] = i - offsets[s];
   }
   batch_reserve(c, B);
-  std::vector<float4> hp(n), hv(n);
-  std::vector<int32_t> hsub(n);
-  for (int64_t i = 0; i < n; i++)
+  std::vector<int32_t> horder;
+  size_order(B.h_count, horder);
+
+  std::vector<XferPart> parts;
+  size_t end = 0;
+  auto place = [&](size_t bytes) {
+    const size_t at = end;
+    end = (at + bytes + 15) & ~(size_t)15;
+    return at;
+  };
+  auto array = [&](const void *src, size_t bytes) {
+    const size_t at = place(src ? bytes : 0);
+    if (src && bytes)
+      parts.push_back(xfer_from(at, src, bytes));
+    return at;
+  };
+  const size_t a_off = place((nsub + 1) * sizeof(int32_t));
+  parts.push_back({a_off, nullptr, (nsub + 1) * sizeof(int32_t), [offsets](char *slot, size_t off, size_t len) {
+                     for (size_t i = 0; i < len / 4; i++)
+                       ((int32_t *)slot)[i] = (int32_t)offsets[off / 4 + i];
+                   }});
+  const size_t a_order = array(horder.data(), nsub * sizeof(int32_t));
+  const size_t a_rp = array(ref_pos, 3 * nsub * sizeof(float)), a_rv = array(ref_vel, 3 * nsub * sizeof(float));
+  const size_t a_mp = array(mb_pos, 3 * nsub * sizeof(float)), a_mv = array(mb_vel, 3 * nsub * sizeof(float));
+  const size_t a_mass = array(mass, n * sizeof(float)), a_pos = array(pos, 3 * n * sizeof(float));
+  const size_t a_vel = array(vel, 3 * n * sizeof(float)), a_u = array(u, n * sizeof(float));
+  const size_t a_type = array(type, n * sizeof(int32_t)), a_id = array(id, n * sizeof(int64_t));
+  // the walk records' buffer (72 bytes a particle, idle between runs) takes the block
+  char *raw = (char *)B.wt.p;
+  if (end > B.wt.n * sizeof(uint2))
   {
-    // (the walk records mark cells by the sign bit of the mass)
-    REQUIRE(mass[i] >= 0.f, HBTX_E_INVALID, "particle masses must be non-negative");
-    hp[i] = make_float4(pos[3 * i], pos[3 * i + 1], pos[3 * i + 2], mass[i]);
-    hv[i] = make_float4(vel[3 * i], vel[3 * i + 1], vel[3 * i + 2], u ? u[i] : 0.f);
+    B.raw.alloc(end);
+    raw = B.raw.p;
   }
-  for (int64_t s = 0; s < nsub; s++)
-    for (int64_t i = offsets[s]; i < offsets[s + 1]; i++)
-      hsub[i] = (int32_t)s;
-  std::vector<int32_t> hoff(nsub + 1), hpairs(2 * nsub + 2, 0), horder(nsub);
-  for (int64_t s = 0; s <= nsub; s++)
-    hoff[s] = (int32_t)offsets[s];
-  for (int64_t s = 0; s < nsub; s++)
-    hpairs[2 * s + 1] = B.h_count[s];
-  std::iota(horder.begin(), horder.end(), 0);
-  std::stable_sort(horder.begin(), horder.end(),
-                   [&](int32_t a, int32_t b) { return B.h_count[a] > B.h_count[b]; });
-  std::vector<float> hr(6 * nsub), hm(6 * nsub);
-  for (int64_t s = 0; s < nsub; s++)
-    for (int k = 0; k < 3; k++)
-    {
-      hr[6 * s + k] = ref_pos[3 * s + k];
-      hr[6 * s + 3 + k] = ref_vel[3 * s + k];
-      hm[6 * s + k] = mb_pos ? mb_pos[3 * s + k] : ref_pos[3 * s + k];
-      hm[6 * s + 3 + k] = mb_vel ? mb_vel[3 * s + k] : ref_vel[3 * s + k];
-    }
   hipStream_t st = c->stream;
-  HIPCHK(hipMemcpyAsync(B.posm.p, hp.data(), n * sizeof(float4), hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(B.velu.p, hv.data(), n * sizeof(float4), hipMemcpyHostToDevice, st));
-  if (type)
-  {
-    std::vector<int8_t> ht(n);
-    for (int64_t i = 0; i < n; i++)
-    {
-      REQUIRE(type[i] >= 0 && type[i] < 6, HBTX_E_INVALID, "particle type out of range [0,6)");
-      ht[i] = (int8_t)type[i];
-    }
-    HIPCHK(hipMemcpyAsync(B.ptype.p, ht.data(), n, hipMemcpyHostToDevice, st));
-    HIPCHK(hipStreamSynchronize(st));
-  }
-  HIPCHK(hipMemcpyAsync(B.sub_of.p, hsub.data(), n * sizeof(int32_t), hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemsetAsync(B.sub_zero.p, 0, std::max<int64_t>(B.max_count, 1) * sizeof(int32_t), st));
-  HIPCHK(hipMemsetAsync(B.order_zero.p, 0, sizeof(int32_t), st));
-  HIPCHK(hipMemcpyAsync(B.off.p, hoff.data(), (nsub + 1) * sizeof(int32_t), hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(B.off_pairs.p, hpairs.data(), (2 * nsub + 2) * sizeof(int32_t), hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(B.order.p, horder.data(), nsub * sizeof(int32_t), hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(B.ref_in.p, hr.data(), 6 * nsub * sizeof(float), hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(B.mb_in.p, hm.data(), 6 * nsub * sizeof(float), hipMemcpyHostToDevice, st));
+  HIPCHK(c->staging.up(c->device, st, raw, parts));
+  auto dev = [&](const void *given, size_t at) { return given ? (const float *)(raw + at) : nullptr; };
+  k_fill_i32<<<1, 64, 0, st>>>(B.load_bad.p, 1, 0);
+  k_fill_i32<<<blocks_for(B.max_count), 256, 0, st>>>(B.sub_zero.p, std::max<int64_t>(B.max_count, 1), 0);
+  k_fill_i32<<<1, 64, 0, st>>>(B.order_zero.p, 1, 0);
+  k_load_subs<<<blocks_for(nsub + 1, 256, 1 << 24), 256, 0, st>>>(
+    (const int32_t *)(raw + a_off), (const int32_t *)(raw + a_order), dev(ref_pos, a_rp), dev(ref_vel, a_rv),
+    dev(mb_pos, a_mp), dev(mb_vel, a_mv), (int32_t)nsub, B.off.p, B.off_pairs.p, B.order.p, B.ref_in.p, B.mb_in.p);
+  k_load_particles<<<blocks_for(n), 256, 0, st>>>(dev(pos, a_pos), dev(vel, a_vel), dev(mass, a_mass), dev(u, a_u),
+                                                  (const int32_t *)dev(type, a_type), (const int64_t *)dev(id, a_id), n,
+                                                  B.posm.p, B.velu.p, B.ptype.p, B.ids.p, B.load_bad.p);
+  k_load_sub_of<<<blocks_for((n + 3) / 4), 256, 0, st>>>(B.off.p, (int32_t)nsub, n, B.sub_of.p, nullptr);
+  HIPCHK(hipGetLastError());
+  int32_t bad = 0;
+  HIPCHK(hipMemcpyAsync(&bad, B.load_bad.p, sizeof(bad), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
-  B.ran = false;
+  B.raw.release();
+  if (bad)
+    B.n = B.nsub = 0; // nothing is loaded
+  // (the walk records mark cells by the sign bit of the mass)
+  REQUIRE(!(bad & LOAD_BAD_MASS), HBTX_E_INVALID, "particle masses must be non-negative");
+  REQUIRE(!(bad & LOAD_BAD_TYPE), HBTX_E_INVALID, "particle type out of range [0,6)");
 }
 
 void run_batch(hbtx_ctx *c, const hbtx_params &prm, uint32_t flags, double *elapsed_ms)
@@ -1573,34 +1614,22 @@ void fetch_batch(hbtx_ctx *c, int64_t *out_order, float *out_energy, float *out_
 {
   Batch &B = c->B;
   REQUIRE(B.ran, HBTX_E_INVALID, "batch has not been run");
-  hipStream_t st = c->stream;
   const int64_t n = B.n;
-  std::vector<int32_t> ford(n);
-  HIPCHK(hipMemcpyAsync(ford.data(), B.ford.p, n * sizeof(int32_t), hipMemcpyDeviceToHost, st));
+  std::vector<XferPart> parts;
+  if (out_order)
+    parts.push_back({0, B.ford.p, n * sizeof(int32_t), [out_order](char *slot, size_t off, size_t len) {
+                       const int32_t *v = (const int32_t *)slot;
+                       int64_t *o = out_order + off / 4;
+                       for (size_t i = 0; i < len / 4; i++)
+                         o[i] = v[i];
+                     }});
   if (out_energy)
-    HIPCHK(hipMemcpyAsync(out_energy, B.fenergy.p, n * sizeof(float), hipMemcpyDeviceToHost, st));
+    parts.push_back(xfer_to(out_energy, B.fenergy.p, n * sizeof(float)));
   if (out_potential)
-    HIPCHK(hipMemcpyAsync(out_potential, B.fpot.p, n * sizeof(float), hipMemcpyDeviceToHost, st));
-  std::vector<hbtx_sub_result> res(B.nsub);
-  HIPCHK(hipMemcpyAsync(res.data(), B.dres.p, B.nsub * sizeof(hbtx_sub_result), hipMemcpyDeviceToHost, st));
-  HIPCHK(hipStreamSynchronize(st));
-  for (int64_t s = 0; s < B.nsub; s++)
-  {
-    const int64_t a = B.h_off[s];
-    for (int64_t k = 0; k < B.h_count[s]; k++)
-      if (out_order)
-        out_order[a + k] = ford[a + k];
-    hbtx_sub_result &R = res[s];
-    if (R.nbound > 0 && !R.disrupted)
-    {
-      const int64_t ti = R.tracer_index;
-      R.mostbound_id = B.h_id[a + ford[a + ti]];
-    }
-    else
-      R.mostbound_id = -1;
-    if (out_res)
-      out_res[s] = R;
-  }
+    parts.push_back(xfer_to(out_potential, B.fpot.p, n * sizeof(float)));
+  if (out_res)
+    parts.push_back(xfer_to(out_res, B.dres.p, B.nsub * sizeof(hbtx_sub_result)));
+  HIPCHK(c->staging.down(c->device, c->stream, parts));
 }
 
 // ---------------------------------------------------------------------------
@@ -1611,10 +1640,9 @@ void build_tree(hbtx_ctx *c, const hbtx_params &prm, int64_t n, const float *pos
 {
   REQUIRE(n >= 1, HBTX_E_INVALID, "a tree needs at least one source");
   Batch &B = c->B;
-  std::vector<float> vel(3 * n, 0.f);
   const int64_t off[2] = {0, n};
   float zero3[3] = {0.f, 0.f, 0.f};
-  upload_batch(c, B, n, pos, vel.data(), mass, nullptr, nullptr, nullptr, 1, off, zero3, zero3, nullptr, nullptr);
+  upload_batch(c, B, n, pos, nullptr, mass, nullptr, nullptr, nullptr, 1, off, zero3, zero3, nullptr, nullptr);
   hbtx_params p = prm;
   p.direct_cutoff = treemode ? 0 : ((int64_t)1 << 40);
   p.max_sample_size = 0;
@@ -1683,44 +1711,37 @@ void tree_points(hbtx_ctx *c, hbtx_tree *T, int64_t nt, const float *tpos, const
   if (nt == 0)
     return;
   hipStream_t st = c->stream;
-  DArr<float4> dt;
-  DArr<float> phi;
-  DArr<double> phid;
-  DArr<uint64_t> keys;
-  DArr<int32_t> vals, segb, segl, counter;
-  dt.alloc(nt);
-  phi.alloc(nt);
-  phid.alloc(nt);
-  keys.alloc(nt);
-  vals.alloc(nt);
-  segb.alloc(1);
-  segl.alloc(1);
-  counter.alloc(2); // [0] work counter, [1] overflow word
-  std::vector<float4> h(nt);
-  for (int64_t i = 0; i < nt; i++)
-    h[i] = make_float4(tpos[3 * i], tpos[3 * i + 1], tpos[3 * i + 2], tmass ? tmass[i] : 0.f);
-  HIPCHK(hipMemcpyAsync(dt.p, h.data(), nt * sizeof(float4), hipMemcpyHostToDevice, st));
+  auto &W = c->ws;
+  W.raw.alloc(4 * nt);
+  W.tgt.alloc(nt);
+  W.phi.alloc(nt);
+  W.keys.alloc(nt);
+  W.vals.alloc(nt);
+  W.seg.alloc(2);
+  W.counter.alloc(2); // [0] work counter, [1] overflow word
+  std::vector<XferPart> parts{xfer_from(0, tpos, 3 * nt * sizeof(float))};
+  if (tmass)
+    parts.push_back(xfer_from(3 * nt * sizeof(float), tmass, nt * sizeof(float)));
+  HIPCHK(c->staging.up(c->device, st, W.raw.p, parts));
+  k_pack_points<<<blocks_for(nt), 256, 0, st>>>(W.raw.p, tmass ? W.raw.p + 3 * nt : nullptr, (int32_t)nt, W.tgt.p);
+  k_points_begin<<<1, 64, 0, st>>>(W.counter.p, W.seg.p, (int32_t)nt);
   // walk order: targets sorted by their key in the tree cube
-  k_point_keys<<<blocks_for(nt), 256, 0, st>>>(dt.p, (int32_t)nt, T->cube.p, keys.p, vals.p);
-  int32_t hb = 0, hl = (int32_t)nt;
-  HIPCHK(hipMemcpyAsync(segb.p, &hb, 4, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(segl.p, &hl, 4, hipMemcpyHostToDevice, st));
+  k_point_keys<<<blocks_for(nt), 256, 0, st>>>(W.tgt.p, (int32_t)nt, T->cube.p, W.keys.p, W.vals.p);
   if (T->treemode)
-    seg_sort(c, keys.p, vals.p, 1, segb.p, segl.p, nt, 63);
-  HIPCHK(hipMemsetAsync(counter.p, 0, 8, st));
+    seg_sort(c, W.keys.p, W.vals.p, 1, W.seg.p, W.seg.p + 1, nt, 63);
   PointArgs A;
-  A.tgt = dt.p;
-  A.tgt_order = vals.p;
+  A.tgt = W.tgt.p;
+  A.tgt_order = W.vals.p;
   A.ntgt = (int32_t)nt;
   A.eb = 0;
   A.ee = T->nw;
   A.treemode = T->treemode;
   A.wt = T->wt.p;
-  A.phi = phi.p;
-  A.phi_d = phid.p;
-  A.counter = counter.p;
+  A.phi = nullptr;
+  A.phi_d = W.phi.p;
+  A.counter = W.counter.p;
   A.stats = c->stats.p;
-  A.overflow = counter.p + 1;
+  A.overflow = W.counter.p + 1;
   A.P = T->P;
   HIPCHK(hipMemsetAsync(c->stats.p, 0, NSTATS * sizeof(unsigned long long), st));
   HIPCHK(hipEventRecord(c->wev0, st));
@@ -1730,10 +1751,8 @@ void tree_points(hbtx_ctx *c, hbtx_tree *T, int64_t nt, const float *tpos, const
     c->count_work ? launch_points<false, true>(c, A) : launch_points<false, false>(c, A);
   HIPCHK(hipEventRecord(c->wev1, st));
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(out, phid.p, nt * sizeof(double), hipMemcpyDeviceToHost, st));
   int32_t ov = 0;
-  HIPCHK(hipMemcpyAsync(&ov, counter.p + 1, 4, hipMemcpyDeviceToHost, st));
-  HIPCHK(hipStreamSynchronize(st));
+  HIPCHK(c->staging.down(c->device, st, {xfer_to(out, W.phi.p, nt * sizeof(double)), xfer_to(&ov, W.counter.p + 1, 4)}));
   REQUIRE(ov == 0, HBTX_E_CAPACITY, "tree walk stack capacity exceeded");
   float wms = 0.f;
   HIPCHK(hipEventElapsedTime(&wms, c->wev0, c->wev1));
@@ -1935,6 +1954,8 @@ int hbtx_batch_load(hbtx_ctx *c, int64_t n, const float *pos, const float *vel, 
     return HBTX_E_INVALID;
   API_GUARD(c, {
     HIPCHK(hipSetDevice(c->device));
+    check_layout(n, nsub, offsets);
+    REQUIRE(vel, HBTX_E_INVALID, "null input array");
     upload_batch(c, c->B, n, pos, vel, mass, u, type, id, nsub, offsets, ref_pos, ref_vel, mb_pos, mb_vel);
   });
 }
@@ -1945,8 +1966,8 @@ int hbtx_batch_set_proposal(hbtx_ctx *c, const uint8_t *proposal)
     return HBTX_E_INVALID;
   API_GUARD(c, {
     REQUIRE(proposal, HBTX_E_INVALID, "null proposal");
-    HIPCHK(hipMemcpyAsync(c->B.proposal.p, proposal, c->B.n, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    HIPCHK(hipSetDevice(c->device));
+    HIPCHK(c->staging.up(c->device, c->stream, c->B.proposal.p, {xfer_from(0, proposal, c->B.n)}));
     c->B.has_proposal = true;
   });
 }
@@ -2022,6 +2043,8 @@ int hbtx_unbind_batch(hbtx_ctx *c, const hbtx_params *prm, int64_t n, const floa
     return HBTX_E_INVALID;
   API_GUARD(c, {
     HIPCHK(hipSetDevice(c->device));
+    check_layout(n, nsub, offsets);
+    REQUIRE(vel, HBTX_E_INVALID, "null input array");
     upload_batch(c, c->B, n, pos, vel, mass, u, type, id, nsub, offsets, ref_pos, ref_vel, mb_pos, mb_vel);
     run_batch(c, *prm, flags, nullptr);
     fetch_batch(c, out_order, out_energy, out_potential, out_res);
@@ -2237,8 +2260,7 @@ int hbtx_batch_profiles(hbtx_ctx *c, const hbtx_params *prm, hbtx_sub_profile *o
     A.rc = B.prof_r.p;
     A.mc = B.prof_m.p;
     run_profiles(c, *prm, A, B.n, B.nsub, B.sub_of.p, B.seg_begin.p, B.seg_len.p, B.keys.p, B.src.p, B.dprof.p);
-    HIPCHK(hipMemcpyAsync(out, B.dprof.p, B.nsub * sizeof(hbtx_sub_profile), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    HIPCHK(c->staging.down(c->device, c->stream, {xfer_to(out, B.dprof.p, B.nsub * sizeof(hbtx_sub_profile))}));
   });
 }
 
@@ -2252,11 +2274,8 @@ int hbtx_profiles(hbtx_ctx *c, const hbtx_params *prm, int64_t n, const float *p
     REQUIRE(n < (int64_t)0x20000000 && nsub < (int64_t)0x7fffffff, HBTX_E_INVALID, "too large");
     REQUIRE(offsets[0] == 0 && offsets[nsub] == n, HBTX_E_INVALID, "offsets must start at 0 and end at n");
     hipStream_t st = c->stream;
-    std::vector<float4> hp(std::max<int64_t>(n, 1));
-    std::vector<int32_t> hoff(nsub + 1), hsub(std::max<int64_t>(n, 1)), hord(std::max<int64_t>(n, 1));
+    std::vector<int32_t> hoff(nsub + 1);
     std::vector<hbtx_sub_result> hres(nsub);
-    for (int64_t i = 0; i < n; i++)
-      hp[i] = make_float4(pos[3 * i], pos[3 * i + 1], pos[3 * i + 2], mass[i]);
     for (int64_t s = 0; s < nsub; s++)
     {
       const int64_t a = offsets[s], e = offsets[s + 1];
@@ -2270,47 +2289,39 @@ int hbtx_profiles(hbtx_ctx *c, const hbtx_params *prm, int64_t n, const float *p
       if (nbound[s] > 0)
         for (int k = 0; k < 3; k++)
           R.mostbound_pos[k] = pos[3 * a + k];
-      for (int64_t i = a; i < e; i++)
-      {
-        hsub[i] = (int32_t)s;
-        hord[i] = (int32_t)(i - a);
-      }
     }
     hoff[nsub] = (int32_t)n;
-    DArr<float4> dp;
-    DArr<int32_t> doff, dsub, dord, sb, sl, vals;
-    DArr<uint64_t> keys;
-    DArr<hbtx_sub_result> dres;
-    DArr<float> rc, mc;
-    DArr<hbtx_sub_profile> dout;
-    dp.alloc(hp.size());
-    doff.alloc(nsub + 1);
-    dsub.alloc(hsub.size());
-    dord.alloc(hord.size());
-    sb.alloc(nsub + 1);
-    sl.alloc(nsub + 1);
-    vals.alloc(hsub.size());
-    keys.alloc(hsub.size());
-    dres.alloc(nsub);
-    rc.alloc(hsub.size());
-    mc.alloc(hsub.size());
-    dout.alloc(nsub);
-    HIPCHK(hipMemcpyAsync(dp.p, hp.data(), hp.size() * sizeof(float4), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(doff.p, hoff.data(), (nsub + 1) * sizeof(int32_t), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dsub.p, hsub.data(), hsub.size() * sizeof(int32_t), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dord.p, hord.data(), hord.size() * sizeof(int32_t), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dres.p, hres.data(), nsub * sizeof(hbtx_sub_result), hipMemcpyHostToDevice, st));
+    auto &W = c->ws;
+    const int64_t n1 = std::max<int64_t>(n, 1);
+    W.raw.alloc(4 * n1);
+    W.posm.alloc(n1);
+    W.off.alloc(nsub + 1);
+    W.sub_of.alloc(n1);
+    W.local.alloc(n1);
+    W.seg.alloc(2 * (nsub + 1));
+    W.vals.alloc(n1);
+    W.keys.alloc(n1);
+    W.res.alloc(nsub);
+    W.rc.alloc(n1);
+    W.mc.alloc(n1);
+    W.prof.alloc(nsub);
+    HIPCHK(c->staging.up(c->device, st, W.raw.p,
+                         {xfer_from(0, pos, 3 * n * sizeof(float)), xfer_from(3 * n * sizeof(float), mass, n * sizeof(float))}));
+    HIPCHK(c->staging.up(c->device, st, W.off.p, {xfer_from(0, hoff.data(), (nsub + 1) * sizeof(int32_t))}));
+    HIPCHK(c->staging.up(c->device, st, W.res.p, {xfer_from(0, hres.data(), nsub * sizeof(hbtx_sub_result))}));
+    if (n > 0)
+      k_pack_points<<<blocks_for(n), 256, 0, st>>>(W.raw.p, W.raw.p + 3 * n, (int32_t)n, W.posm.p);
+    k_load_sub_of<<<blocks_for((n + 3) / 4), 256, 0, st>>>(W.off.p, (int32_t)nsub, n, W.sub_of.p, W.local.p);
     ProfArgs A;
-    A.off = doff.p;
-    A.ford = dord.p;
-    A.posm = dp.p;
-    A.res = dres.p;
-    A.seg_len = sl.p;
-    A.rc = rc.p;
-    A.mc = mc.p;
-    run_profiles(c, *prm, A, n, (int32_t)nsub, dsub.p, sb.p, sl.p, keys.p, vals.p, dout.p);
-    HIPCHK(hipMemcpyAsync(out, dout.p, nsub * sizeof(hbtx_sub_profile), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+    A.off = W.off.p;
+    A.ford = W.local.p;
+    A.posm = W.posm.p;
+    A.res = W.res.p;
+    A.seg_len = W.seg.p + nsub + 1;
+    A.rc = W.rc.p;
+    A.mc = W.mc.p;
+    run_profiles(c, *prm, A, n, (int32_t)nsub, W.sub_of.p, W.seg.p, W.seg.p + nsub + 1, W.keys.p, W.vals.p, W.prof.p);
+    HIPCHK(c->staging.down(c->device, st, {xfer_to(out, W.prof.p, nsub * sizeof(hbtx_sub_profile))}));
   });
 }
 
@@ -2370,11 +2381,11 @@ int hbtx_reassign_targets(hbtx_ctx *c, const hbtx_params *prm, int64_t n, const 
     R.trec.alloc(n);
     R.lbase.alloc(RS_LEVELS);
     hipStream_t st = c->stream;
-    HIPCHK(hipMemcpyAsync(R.pos.p, pos, 3 * n * sizeof(float), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(R.tracer.p, is_tracer, n, hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(R.sub.p, sub, n * sizeof(int32_t), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(R.goff.p, hoff.data(), (G + 1) * sizeof(int32_t), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(R.radii.p, rad.data(), RS_RADII * sizeof(float), hipMemcpyHostToDevice, st));
+    HIPCHK(c->staging.up(c->device, st, R.pos.p, {xfer_from(0, pos, 3 * n * sizeof(float))}));
+    HIPCHK(c->staging.up(c->device, st, R.tracer.p, {xfer_from(0, is_tracer, n)}));
+    HIPCHK(c->staging.up(c->device, st, R.sub.p, {xfer_from(0, sub, n * sizeof(int32_t))}));
+    HIPCHK(c->staging.up(c->device, st, R.goff.p, {xfer_from(0, hoff.data(), (G + 1) * sizeof(int32_t))}));
+    HIPCHK(c->staging.up(c->device, st, R.radii.p, {xfer_from(0, rad.data(), RS_RADII * sizeof(float))}));
     RsArgs A;
     A.n = (int32_t)n;
     A.ngroups = G;
@@ -2451,8 +2462,7 @@ int hbtx_reassign_targets(hbtx_ctx *c, const hbtx_params *prm, int64_t n, const 
     }
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(c->ev1, st));
-    HIPCHK(hipMemcpyAsync(out_target, R.out.p, n * sizeof(int32_t), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+    HIPCHK(c->staging.down(c->device, st, {xfer_to(out_target, R.out.p, n * sizeof(int32_t))}));
     if (elapsed_ms)
     {
       float ms = 0.f;
@@ -2484,8 +2494,8 @@ int hbtx_segmented_sort(hbtx_ctx *c, int64_t n, uint64_t *keys, int32_t *vals, i
       hb[s] = (int32_t)seg_offsets[s];
       hl[s] = (int32_t)(seg_offsets[s + 1] - seg_offsets[s]);
     }
-    HIPCHK(hipMemcpyAsync(dk.p, keys, n * 8, hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dv.p, vals, n * 4, hipMemcpyHostToDevice, st));
+    HIPCHK(c->staging.up(c->device, st, dk.p, {xfer_from(0, keys, n * 8)}));
+    HIPCHK(c->staging.up(c->device, st, dv.p, {xfer_from(0, vals, n * 4)}));
     HIPCHK(hipMemcpyAsync(sb.p, hb.data(), nseg * 4, hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(sl.p, hl.data(), nseg * 4, hipMemcpyHostToDevice, st));
     // digit passes only over the bits the keys use
@@ -2496,9 +2506,7 @@ int hbtx_segmented_sort(hbtx_ctx *c, int64_t n, uint64_t *keys, int32_t *vals, i
     while (bits < 64 && (any >> bits) != 0)
       bits++;
     seg_sort(c, dk.p, dv.p, (int32_t)nseg, sb.p, sl.p, n, bits);
-    HIPCHK(hipMemcpyAsync(keys, dk.p, n * 8, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(vals, dv.p, n * 4, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+    HIPCHK(c->staging.down(c->device, st, {xfer_to(keys, dk.p, n * 8), xfer_to(vals, dv.p, n * 4)}));
   });
 }
 
@@ -2539,6 +2547,18 @@ void mlp_upload(hbtx_ctx *c, hbtx_mlp *M, const float *master)
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(st));
   M->step = 0;
+}
+
+// samples of a call (labels may be null) into the context's workspace
+void mlp_samples(hbtx_ctx *c, int64_t n, const float *X, const uint8_t *y)
+{
+  auto &W = c->ws;
+  W.X.alloc(n * MLP_IN);
+  HIPCHK(c->staging.up(c->device, c->stream, W.X.p, {xfer_from(0, X, n * MLP_IN * sizeof(float))}));
+  if (!y)
+    return;
+  W.y.alloc(n);
+  HIPCHK(c->staging.up(c->device, c->stream, W.y.p, {xfer_from(0, y, n)}));
 }
 
 // forward+backward of nb samples (rows idx[0..nb) of dX, or rows 0..nb) -> M->grad, M->loss
@@ -2625,12 +2645,9 @@ int hbtx_mlp_gradient(hbtx_ctx *c, hbtx_mlp *M, int64_t n, const float *X, const
   API_GUARD(c, {
     HIPCHK(hipSetDevice(c->device));
     hipStream_t st = c->stream;
-    DArr<float> dX;
-    DArr<uint8_t> dy;
-    dX.alloc(n * MLP_IN);
-    dy.alloc(n);
-    HIPCHK(hipMemcpyAsync(dX.p, X, n * MLP_IN * sizeof(float), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dy.p, y, n, hipMemcpyHostToDevice, st));
+    mlp_samples(c, n, X, y);
+    auto &dX = c->ws.X;
+    auto &dy = c->ws.y;
     mlp_grad_device(c, M, dX.p, dy.p, nullptr, n);
     double l = 0.0;
     if (grad)
@@ -2651,14 +2668,11 @@ int hbtx_mlp_train(hbtx_ctx *c, hbtx_mlp *M, int64_t n, const float *X, const ui
     HIPCHK(hipSetDevice(c->device));
     REQUIRE(n < (int64_t)0x7fffffff, HBTX_E_INVALID, "too many training samples");
     hipStream_t st = c->stream;
-    DArr<float> dX;
-    DArr<uint8_t> dy;
+    mlp_samples(c, n, X, y);
+    auto &dX = c->ws.X;
+    auto &dy = c->ws.y;
     DArr<int32_t> didx;
-    dX.alloc(n * MLP_IN);
-    dy.alloc(n);
     didx.alloc(n);
-    HIPCHK(hipMemcpyAsync(dX.p, X, n * MLP_IN * sizeof(float), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dy.p, y, n, hipMemcpyHostToDevice, st));
     std::vector<int32_t> perm(n);
     uint64_t rs = seed;
     const float b1 = 0.9f, b2 = 0.999f;
@@ -2708,14 +2722,13 @@ int hbtx_mlp_predict(hbtx_ctx *c, hbtx_mlp *M, int64_t n, const float *X, float 
     if (n == 0)
       return HBTX_OK;
     hipStream_t st = c->stream;
-    DArr<float> dX, dl;
-    dX.alloc(n * MLP_IN);
+    mlp_samples(c, n, X, nullptr);
+    auto &dX = c->ws.X;
+    auto &dl = c->ws.rc;
     dl.alloc(n);
-    HIPCHK(hipMemcpyAsync(dX.p, X, n * MLP_IN * sizeof(float), hipMemcpyHostToDevice, st));
     k_mlp_forward<<<mlp_forward_blocks(n), 256, 0, st>>>(M->wf.p, M->wb.p, dX.p, n, dl.p, nullptr, 0);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(logit, dl.p, n * sizeof(float), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+    HIPCHK(c->staging.down(c->device, st, {xfer_to(logit, dl.p, n * sizeof(float))}));
   });
 }
 
@@ -2745,13 +2758,15 @@ int hbtx_batch_set_previous(hbtx_ctx *c, const int32_t *prev_rank, const uint8_t
         com[6 * s + k] = prev_com_pos[3 * s + k];
         com[6 * s + 3 + k] = prev_com_vel[3 * s + k];
       }
-    HIPCHK(hipMemcpyAsync(B.prev_rank.p, prev_rank, n * sizeof(int32_t), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(B.prev_bound.p, prev_bound, n, hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(B.prev_energy.p, prev_energy, n * sizeof(float), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(B.prev_com.p, com.data(), 6 * ns * sizeof(float), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(B.prev_mb.p, prev_mbound, ns * sizeof(float), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(B.prev_rs.p, prev_rscale, ns * sizeof(float), hipMemcpyHostToDevice, st));
-    HIPCHK(hipStreamSynchronize(st));
+    auto up = [&](void *dst, const void *src, size_t bytes) {
+      HIPCHK(c->staging.up(c->device, st, dst, {xfer_from(0, src, bytes)}));
+    };
+    up(B.prev_rank.p, prev_rank, n * sizeof(int32_t));
+    up(B.prev_bound.p, prev_bound, n);
+    up(B.prev_energy.p, prev_energy, n * sizeof(float));
+    up(B.prev_com.p, com.data(), 6 * ns * sizeof(float));
+    up(B.prev_mb.p, prev_mbound, ns * sizeof(float));
+    up(B.prev_rs.p, prev_rscale, ns * sizeof(float));
     B.has_prev = true;
     B.feat_full = false;  // the features depend on the previous outputs
   });

@@ -176,6 +176,16 @@ __global__ __launch_bounds__(DS_THREADS) void k_points_direct(PointArgs A)
   }
 }
 
+// the walk's counters cleared, and one sort segment over the n targets
+__global__ void k_points_begin(int32_t *counter, int32_t *seg, int32_t n)
+{
+  if (blockIdx.x == 0 && threadIdx.x < 2)
+  {
+    counter[threadIdx.x] = 0;
+    seg[threadIdx.x] = (threadIdx.x == 0) ? 0 : n;
+  }
+}
+
 // keys of external target points in a tree's cube (walk order for coherence)
 __global__ void k_point_keys(const float4 *tgt, int32_t n, const double *cube, uint64_t *keys, int32_t *vals)
 {
