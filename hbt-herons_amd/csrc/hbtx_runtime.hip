@@ -13,6 +13,7 @@
 #include "subsample.h"
 #include "learn.h"
 #include "tiles.h"
+#include "lists.h"
 #include "profile.h"
 #include "reassign.h"
 #include "load.h"
@@ -184,7 +185,7 @@ struct Batch
   DArr<int32_t> icnt, iscan;
   // subhaloes
   DArr<int32_t> status, corr, iters, mode, treemode, nlast, nbound, nrem, nuns, ntgt, nsrc, src_off, ent_begin,
-    ent_end, nitems, bnd_cnt, bnd_tr, first_idx, seg_begin, seg_len, rbegin, rlen, type_cnt, first_tracer, aux32;
+    ent_end, nitems, bnd_cnt, bnd_tr, first_idx, seg_begin, seg_len, type_cnt, first_tracer, aux32;
   DArr<float> mlast, mbound, ref, oldref, mb, upscale, ref_in, mb_in, minit;
   DArr<int32_t> warm, npro, nadd, reset_;
   DArr<float> feat, logit;
@@ -217,6 +218,8 @@ struct View
 {
   int64_t n;
   int32_t nsub;
+  int32_t max_count; // particles of the largest subhalo
+  int64_t ent_bound; // entries of the largest trees its subhaloes can make
   SubArrays S;
   PartArrays Q;
   const int32_t *order;
@@ -294,6 +297,7 @@ struct hbtx_ctx
   DArr<double> red_partial;
   DArr<unsigned long long> stats;
   Staging staging;
+  int32_t *round_words = nullptr; // pinned: a round's words for the host
   hipEvent_t ev0 = nullptr, ev1 = nullptr, wev0 = nullptr, wev1 = nullptr;
   int64_t walk_items_hint = INT64_MAX; // work items of the previous round of the running view
   double walk_ms = 0.0;
@@ -344,6 +348,12 @@ namespace
 template <class T>
 void scan_excl(hbtx_ctx *c, const T *in, T *out, int64_t n, DArr<T> &part, const int32_t *n_dev = nullptr)
 {
+  if (n <= LIST_ONE_MAX)
+  {
+    k_scan_one<T><<<1, LIST_THREADS, 0, c->stream>>>(in, out, n, n_dev);
+    HIPCHK(hipGetLastError());
+    return;
+  }
   const int64_t nb = std::max<int64_t>(1, (n + SCAN_TILE - 1) / SCAN_TILE);
   part.alloc(nb);
   k_scan_reduce<T><<<(unsigned)nb, SCAN_THREADS, 0, c->stream>>>(in, n, n_dev, part.p);
@@ -361,9 +371,27 @@ void scan32_dev(hbtx_ctx *c, const int32_t *in, int32_t *out, int64_t n_max, con
 {
   scan_excl<int32_t>(c, in, out, n_max, c->part32, n_dev);
 }
-void scan64(hbtx_ctx *c, const int64_t *in, int64_t *out, int64_t n)
+
+// Tiles of `tile` slots over the ranges longer than `over` (lists.h); returns the
+// device-side tile count.  begin_out / len_out (may be null) receive the ranges.
+template <class R>
+const int32_t *list_tiles(hbtx_ctx *c, const R &r, int32_t ns, int tile, int over, bool first, int32_t *ntile,
+                          int32_t *toff, int4 *tiles, int32_t *begin_out = nullptr, int32_t *len_out = nullptr)
 {
-  scan_excl<int64_t>(c, in, out, n, c->part64);
+  const int gs = blocks_for(ns, 256, 1 << 24);
+  const bool whole = ns <= LIST_THREADS;
+  if (ns <= LIST_ONE_MAX)
+    k_list_one<<<1, LIST_THREADS, 0, c->stream>>>(r, ns, tile, over, first, ntile, toff, whole ? tiles : nullptr,
+                                                  begin_out, len_out);
+  else
+  {
+    k_list_counts<<<gs, 256, 0, c->stream>>>(r, ns, tile, over, ntile, begin_out, len_out);
+    scan32(c, ntile, toff, ns);
+  }
+  if (!whole)
+    k_list_tiles<<<gs, 256, 0, c->stream>>>(r, ns, tile, first, ntile, toff, tiles);
+  HIPCHK(hipGetLastError());
+  return toff + ns;
 }
 
 // Radix tiles of a segmented sort over n elements in nseg segments: a segment
@@ -386,28 +414,32 @@ void reserve_sort(hbtx_ctx *c, int64_t n, int32_t nseg)
   c->gchunk.alloc(maxt * RADIX_MAX_BINS); // chunk totals and bases, stored at the chunks' head tiles
 }
 
-// Sort (keys, vals) within each segment [seg_begin, seg_begin+seg_len); keys use
-// the low key_bits bits.
-// small_only: every segment is known to hold at most SORT_SMALL_MAX elements.
-void seg_sort(hbtx_ctx *c, uint64_t *keys, int32_t *vals, int32_t nseg, const int32_t *seg_begin,
-              const int32_t *seg_len, int64_t n_cap, int key_bits, bool small_only = false)
+// Sort (keys, vals) within each segment, given by r and written to [seg_begin,
+// seg_begin+seg_len) for the passes; keys use the low key_bits bits.
+// max_len: no segment is longer (the passes for longer segments are left out).
+template <class R>
+void seg_sort(hbtx_ctx *c, uint64_t *keys, int32_t *vals, int32_t nseg, const R &r, int32_t *seg_begin,
+              int32_t *seg_len, int64_t n_cap, int key_bits, int64_t max_len = INT64_MAX)
 {
   reserve_sort(c, n_cap, nseg);
+  const bool radix = max_len > SORT_SMALL_MAX;
+  if (radix)
+    list_tiles(c, r, nseg, SORT_TILE, SORT_SMALL_MAX, false, c->sort_ntile.p, c->sort_toff.p, c->sort_tiles.p, seg_begin,
+               seg_len);
+  else
+    k_list_counts<<<blocks_for(nseg, 256, 1 << 24), 256, 0, c->stream>>>(r, nseg, SORT_TILE, SORT_SMALL_MAX,
+                                                                         (int32_t *)nullptr, seg_begin, seg_len);
   k_sort_wave<<<std::max(1, std::min((nseg + 3) / 4, 16384)), SORT_THREADS, 0, c->stream>>>(keys, vals, seg_begin,
                                                                                             seg_len, nseg);
-  k_sort_wave4<<<std::max(1, std::min((nseg + 3) / 4, 16384)), SORT_THREADS, 0, c->stream>>>(keys, vals, seg_begin,
-                                                                                            seg_len, nseg);
-  k_sort_small<<<std::max(1, std::min(nseg, 16384)), SORT_THREADS, 0, c->stream>>>(keys, vals, seg_begin, seg_len,
-                                                                                    nseg);
-  if (small_only)
-  {
-    HIPCHK(hipGetLastError());
+  if (max_len > SORT_WAVE_MAX)
+    k_sort_wave4<<<std::max(1, std::min((nseg + 3) / 4, 16384)), SORT_THREADS, 0, c->stream>>>(keys, vals, seg_begin,
+                                                                                              seg_len, nseg);
+  if (max_len > SORT_WAVE4_MAX)
+    k_sort_small<<<std::max(1, std::min(nseg, 16384)), SORT_THREADS, 0, c->stream>>>(keys, vals, seg_begin, seg_len,
+                                                                                      nseg);
+  HIPCHK(hipGetLastError());
+  if (!radix)
     return;
-  }
-  k_sort_ntiles<<<blocks_for(nseg, 256, 1 << 20), 256, 0, c->stream>>>(seg_len, nseg, c->sort_ntile.p);
-  scan32(c, c->sort_ntile.p, c->sort_toff.p, nseg);
-  k_sort_tiles<<<blocks_for(nseg, 256, 1 << 20), 256, 0, c->stream>>>(seg_begin, seg_len, c->sort_toff.p, nseg,
-                                                                       c->sort_tiles.p);
   const int32_t *ntiles_p = c->sort_toff.p + nseg;
   const int64_t maxt = sort_tile_bound(n_cap, nseg);
   const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(maxt, 4 * c->num_cu));
@@ -447,19 +479,16 @@ void seg_sort(hbtx_ctx *c, uint64_t *keys, int32_t *vals, int32_t nseg, const in
   HIPCHK(hipGetLastError());
 }
 
-// Tiles of RED_TILE slots over [begin[s], begin[s]+len[s]); returns device pointer to tile count.
-const int32_t *red_tiles(hbtx_ctx *c, const int32_t *begin, const int32_t *len, int32_t nsub, int64_t n_cap)
+// Tiles of RED_TILE slots over the ranges; returns device pointer to tile count.
+template <class R>
+const int32_t *red_tiles(hbtx_ctx *c, const R &r, int32_t nsub, int64_t n_cap)
 {
   c->red_ntile.alloc(nsub + 1);
   c->red_toff.alloc(nsub + 1);
   const int64_t maxt = n_cap / RED_TILE + nsub + 1;
   c->red_tiles.alloc(maxt);
   c->red_partial.alloc(maxt * RED_NV);
-  k_red_ntiles<<<blocks_for(nsub, 256, 1 << 20), 256, 0, c->stream>>>(len, nsub, c->red_ntile.p);
-  scan32(c, c->red_ntile.p, c->red_toff.p, nsub);
-  k_red_tiles<<<blocks_for(nsub, 256, 1 << 20), 256, 0, c->stream>>>(begin, len, c->red_toff.p, nsub,
-                                                                      c->red_tiles.p);
-  return c->red_toff.p + nsub;
+  return list_tiles(c, r, nsub, RED_TILE, 0, false, c->red_ntile.p, c->red_toff.p, c->red_tiles.p);
 }
 
 int red_grid(hbtx_ctx *c, int64_t n_cap, int32_t nsub)
@@ -468,14 +497,13 @@ int red_grid(hbtx_ctx *c, int64_t n_cap, int32_t nsub)
 }
 
 DevParams make_dev_params(const hbtx_params &p);
-const int32_t *red_tiles(hbtx_ctx *c, const int32_t *begin, const int32_t *len, int32_t nsub, int64_t n_cap);
-int red_grid(hbtx_ctx *c, int64_t n_cap, int32_t nsub);
 
 // Profiles and shapes of the bound sets described by A (positions, final order,
 // results): sort by radius, tiled cumulative mass and candidates, per-subhalo
 // combination into out (device).
 void run_profiles(hbtx_ctx *c, const hbtx_params &prm, ProfArgs &A, int64_t n, int32_t nsub, const int32_t *sub_of,
-                  int32_t *seg_begin, int32_t *seg_len, uint64_t *keys, int32_t *vals, hbtx_sub_profile *out)
+                  int32_t *seg_begin, int32_t *seg_len, uint64_t *keys, int32_t *vals, hbtx_sub_profile *out,
+                  int64_t max_len)
 {
   hbtx_params p = prm;
   if (p.direct_cutoff < 0)
@@ -489,10 +517,11 @@ void run_profiles(hbtx_ctx *c, const hbtx_params &prm, ProfArgs &A, int64_t n, i
   A.vel_unit = G / a;
   hipStream_t st = c->stream;
   const int gs = blocks_for(nsub, 256, 1 << 20);
+  const RangeArray ranges{seg_begin, seg_len};
   k_prof_segments<<<gs, 256, 0, st>>>(nsub, A.off, A.res, seg_begin, seg_len);
   k_prof_keys<<<blocks_for(n), 256, 0, st>>>(A, n, sub_of, keys, vals);
-  seg_sort(c, keys, vals, nsub, seg_begin, seg_len, n, 32);
-  const int32_t *nt = red_tiles(c, seg_begin, seg_len, nsub, n);
+  seg_sort(c, keys, vals, nsub, ranges, seg_begin, seg_len, n, 32, max_len);
+  const int32_t *nt = red_tiles(c, ranges, nsub, n);
   A.part = c->red_partial.p;
   const int rg = red_grid(c, n, nsub);
   k_prof_tile_sum<<<rg, RED_THREADS, 0, st>>>(A, c->red_tiles.p, nt);
@@ -641,7 +670,7 @@ void batch_reserve(hbtx_ctx *c, Batch &B)
   B.iscan.alloc(ns + 1);
   DArr<int32_t> *i32s[] = {&B.status, &B.corr, &B.iters, &B.mode, &B.treemode, &B.nlast, &B.nbound, &B.nrem,
                            &B.nuns, &B.ntgt, &B.nsrc, &B.src_off, &B.ent_begin, &B.ent_end, &B.nitems, &B.bnd_cnt,
-                           &B.bnd_tr, &B.first_idx, &B.seg_begin, &B.seg_len, &B.rbegin, &B.rlen, &B.first_tracer,
+                           &B.bnd_tr, &B.first_idx, &B.seg_begin, &B.seg_len, &B.first_tracer,
                            &B.aux32};
   for (auto *a : i32s)
     a->alloc(ns + 1);
@@ -684,6 +713,8 @@ View make_view(Batch &B, int64_t p0, int64_t n, int32_t s0, int32_t nsub, bool w
   View V;
   V.n = n;
   V.nsub = nsub;
+  V.max_count = whole ? B.max_count : (int32_t)n;
+  V.ent_bound = whole ? B.ent_bound : entry_bound(n);
   V.p0 = p0;
   V.s0 = s0;
   SubArrays &S = V.S;
@@ -813,11 +844,7 @@ int tile_grid(hbtx_ctx *c, const View &V)
 // round's plan); returns the device-side tile count.
 const int32_t *build_slot_tiles(hbtx_ctx *c, Batch &B, View &V)
 {
-  const int gs = blocks_for(V.nsub, 256, 1 << 20);
-  k_slot_ntiles<<<gs, 256, 0, c->stream>>>(V.S, B.stile_n.p);
-  scan32(c, B.stile_n.p, B.stile_off.p, V.nsub);
-  k_slot_tiles<<<gs, 256, 0, c->stream>>>(V.S, B.stile_off.p, B.stiles.p);
-  return B.stile_off.p + V.nsub;
+  return list_tiles(c, RangeActive{V.S}, V.nsub, SLOT_TILE, 0, true, B.stile_n.p, B.stile_off.p, B.stiles.p);
 }
 
 // Sources of the round -> dense list, then (tree-mode subhaloes) the octree.
@@ -833,8 +860,7 @@ void round_sources_and_tree(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, 
     // candidate ranks in E-list order and the mass upscale factors (:290-391)
     k_mark_candidates<<<gb, 256, 0, st>>>(V.S, V.Q, n, B.flag.p);
     scan32(c, B.flag.p, B.crank.p, n);
-    k_upscale_ranges<<<gs, 256, 0, st>>>(V.S, B.rbegin.p, B.rlen.p);
-    const int32_t *nt = red_tiles(c, B.rbegin.p, B.rlen.p, V.nsub, n);
+    const int32_t *nt = red_tiles(c, RangeUpscale{V.S}, V.nsub, n);
     k_upscale_tiles<<<red_grid(c, n, V.nsub), 256, 0, st>>>(V.S, V.Q, P, c->red_tiles.p, nt, B.crank.p,
                                                             c->red_partial.p);
     k_red_finalize<<<red_finalize_blocks(V.nsub), 256, 0, st>>>(c->red_toff.p, c->red_ntile.p, V.nsub, c->red_partial.p, V.red2);
@@ -865,19 +891,27 @@ void build_sources_tree(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, cons
   const int32_t *s_total = B.tpre32.p + maxt;
   k_scatter_sources<<<tile_grid(c, V), SLOT_THREADS, 0, st>>>(V.S, B.stiles.p, nt, B.flag.p, B.tpre32.p, B.src.p,
                                                               B.src_sub.p, B.sub_first32.p);
+  if (level >= 2)
+  {
+    // direct sums only: the sources' records, in the dense list's order
+    TreeArgs T = tree_args(B, V, P);
+    k_sub_src_direct<<<gs, 256, 0, st>>>(V.S, B.sub_first32.p, s_total, B.misc.p + 3);
+    k_emit_direct<<<blocks_for(n, 256, 8 * 1024), 256, 0, st>>>(T);
+    HIPCHK(hipGetLastError());
+    return;
+  }
   k_sub_src<<<gs, 256, 0, st>>>(V.S, B.sub_first32.p);
-  k_tree_src_ranges<<<gs, 256, 0, st>>>(V.S, B.rbegin.p, B.rlen.p);
-  const int32_t *nbt = red_tiles(c, B.rbegin.p, B.rlen.p, V.nsub, n);
+  const int32_t *nbt = red_tiles(c, RangeTreeSrc{V.S}, V.nsub, n);
   k_bbox_tiles<<<red_grid(c, n, V.nsub), 256, 0, st>>>(V.S, V.Q.posm, B.src.p, c->red_tiles.p, nbt);
   k_cube<<<gs, 256, 0, st>>>(V.S);
   k_keys<<<gb, 256, 0, st>>>(V.S, P, V.Q.posm, B.src.p, B.src_sub.p, s_total, B.keys.p);
-  k_sort_segments<<<gs, 256, 0, st>>>(V.S, B.seg_begin.p, B.seg_len.p);
-  seg_sort(c, B.keys.p, B.src.p, V.nsub, B.seg_begin.p, B.seg_len.p, n, 63, level >= 1);
+  seg_sort(c, B.keys.p, B.src.p, V.nsub, RangeTreeSrc{V.S}, B.seg_begin.p, B.seg_len.p, n, 63,
+           level >= 1 ? SORT_SMALL_MAX : V.max_count);
   k_targets_from_sources<<<gb, 256, 0, st>>>(V.S, V.Q, B.src.p, B.src_sub.p, s_total);
   TreeArgs T = tree_args(B, V, P);
   k_tree_count<<<blocks_for(n, 256, 8 * 1024), 256, 0, st>>>(T, B.cnt.p);
   scan32_dev(c, B.cnt.p, B.cscan.p, n, s_total);
-  if (!graph)
+  if (!graph && B.ent_cap < V.ent_bound)
   {
     // exact entry count and depth of this round's trees; grow the entry buffers if needed
     k_entry_total<<<1, 1, 0, st>>>(s_total, B.cscan.p, B.misc.p + 3, 0x7fffffff, B.misc.p + 2);
@@ -891,16 +925,11 @@ void build_sources_tree(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, cons
       T = tree_args(B, V, P);
     }
   }
-  // (a captured round cannot wait for the count: its buffers are sized for the
-  // largest trees the batch can make)
+  // (buffers that hold the largest trees the view can make need no count; a captured
+  // round, which cannot wait for one, always has them)
   k_tree_emit<<<blocks_for(n, 256, 8 * 1024), 256, 0, st>>>(T);
   k_sub_entries<<<gs, 256, 0, st>>>(V.S, B.cscan.p, B.ent_cap, B.misc.p + 2);
   k_entry_total<<<1, 1, 0, st>>>(s_total, B.cscan.p, B.misc.p + 3, B.ent_cap, B.misc.p + 2);
-  if (level >= 2)
-  {
-    HIPCHK(hipGetLastError());
-    return; // direct sums only: no cells
-  }
   // moments bottom-up: LDS-staged windows, then one pass per level of window
   // groups (levels sized for the entry capacity; each pass reads the entry total)
   std::vector<int64_t> units{(std::max<int64_t>(B.ent_cap, 1) + MOM_WIN - 1) / MOM_WIN};
@@ -958,12 +987,17 @@ void round_items(hbtx_ctx *c, Batch &B, View &V)
 {
   hipStream_t st = c->stream;
   const int gs = blocks_for(V.nsub, 256, 1 << 20);
-  k_items_count<<<gs, 256, 0, st>>>(V.S, V.order, B.icnt.p);
-  scan32(c, B.icnt.p, B.iscan.p, V.nsub);
+  int32_t *total = B.misc.p + 7; // read after the round
+  if (V.nsub <= LIST_ONE_MAX)
+    k_items_one<<<1, LIST_THREADS, 0, st>>>(V.S, V.order, B.iscan.p, B.wctr.p, 16 * WALK_MAX_CHUNKS, total);
+  else
+  {
+    k_items_count<<<gs, 256, 0, st>>>(V.S, V.order, B.icnt.p);
+    scan32(c, B.icnt.p, B.iscan.p, V.nsub);
+    k_items_finish<<<1, 256, 0, st>>>(B.iscan.p + V.nsub, B.wctr.p, 16 * WALK_MAX_CHUNKS, total);
+  }
   k_items_emit<<<blocks_for((int64_t)V.nsub * HBTX_WAVE, 256, 1 << 24), 256, 0, st>>>(V.S, V.order, B.iscan.p,
                                                                                        B.items.p);
-  k_fill_i32<<<1, 256, 0, st>>>(B.wctr.p, 16 * WALK_MAX_CHUNKS, 0);
-  k_copy_i32<<<1, 64, 0, st>>>(B.iscan.p + V.nsub, B.misc.p + 7); // item count, read after the round
   HIPCHK(hipGetLastError());
 }
 
@@ -1027,13 +1061,12 @@ void round_partition(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, bool wa
     k_set_unsampled<<<gs, 256, 0, st>>>(V.S, B.aux32.p);
   }
   k_round_decide<<<gs, 256, 0, st>>>(V.S, P, B.sub_total64.p, warm_round ? B.aux32.p : nullptr);
-  k_com_ranges<<<gs, 256, 0, st>>>(V.S, B.rbegin.p, B.rlen.p);
   if (P.periodic)
   {
     k_fill_i32<<<gs, 256, 0, st>>>(V.S.first_idx, V.nsub, 0x7fffffff);
     k_first_index<<<gb, 256, 0, st>>>(V.S, V.Q, n);
   }
-  const int32_t *ntiles = red_tiles(c, B.rbegin.p, B.rlen.p, V.nsub, n);
+  const int32_t *ntiles = red_tiles(c, RangeCom{V.S}, V.nsub, n);
   k_red_tile<ComOp><<<red_grid(c, n, V.nsub), RED_THREADS, 0, st>>>(V.S, V.Q, P, c->red_tiles.p, ntiles,
                                                                      c->red_partial.p);
   k_red_finalize<<<red_finalize_blocks(V.nsub), 256, 0, st>>>(c->red_toff.p, c->red_ntile.p, V.nsub, c->red_partial.p, V.red);
@@ -1178,11 +1211,10 @@ void run_final(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, bool want_pot
   const int gb = blocks_for(n);
   const int gs = blocks_for(V.nsub, 256, 1 << 20);
   k_final_keys<<<gb, 256, 0, st>>>(V.S, V.Q, n, rounds, B.keys.p, V.fvals);
-  k_final_segments<<<gs, 256, 0, st>>>(V.S, B.seg_begin.p, B.seg_len.p);
   int gbits = 0;
   while ((1 << gbits) <= rounds)
     gbits++;
-  seg_sort(c, B.keys.p, V.fvals, V.nsub, B.seg_begin.p, B.seg_len.p, n, 32 + gbits);
+  seg_sort(c, B.keys.p, V.fvals, V.nsub, RangeConverged{V.S}, B.seg_begin.p, B.seg_len.p, n, 32 + gbits, V.max_count);
   if (P.refine)
   {
     // RefineBindingEnergyOrder (:395-425): tree over the most bound particles, true masses
@@ -1193,14 +1225,12 @@ void run_final(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, bool want_pot
     build_sources_tree(c, B, V, P, nt, false, 0, false);
     c->walk_items_hint = INT64_MAX; // (other targets than the rounds')
     round_walk(c, B, V, P);
-    k_refine_keys<<<gb, 256, 0, st>>>(V.S, n, V.fvals, B.eref.p + V.p0, B.keys.p, B.seg_begin.p, B.seg_len.p);
-    k_refine_segments<<<gs, 256, 0, st>>>(V.S, B.seg_begin.p, B.seg_len.p);
-    seg_sort(c, B.keys.p, V.fvals, V.nsub, B.seg_begin.p, B.seg_len.p, n, 32);
+    k_refine_keys<<<gb, 256, 0, st>>>(V.S, n, V.fvals, B.eref.p + V.p0, B.keys.p);
+    seg_sort(c, B.keys.p, V.fvals, V.nsub, RangeRefine{V.S}, B.seg_begin.p, B.seg_len.p, n, 32, V.max_count);
   }
   k_final_local<<<gb, 256, 0, st>>>(V.S, n, V.fvals, V.Q.energy, V.ford, V.fenergy);
   // kinematics / types over the bound particles (input order)
-  k_final_ranges<<<gs, 256, 0, st>>>(V.S, B.rbegin.p, B.rlen.p);
-  const int32_t *ntiles = red_tiles(c, B.rbegin.p, B.rlen.p, V.nsub, n);
+  const int32_t *ntiles = red_tiles(c, RangeConverged{V.S}, V.nsub, n);
   if (V.Q.ptype)
     k_final_tile<true><<<red_grid(c, n, V.nsub), RED_THREADS, 0, st>>>(V.S, V.Q, P, c->red_tiles.p, ntiles,
                                                                       c->red_partial.p);
@@ -1218,20 +1248,6 @@ void run_final(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, bool want_pot
   HIPCHK(hipGetLastError());
 }
 
-__global__ void k_all_ranges(SubArrays S, int32_t *begin, int32_t *len)
-{
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= S.nsub)
-    return;
-  begin[s] = S.off[s];
-  len[s] = S.off[s + 1] - S.off[s];
-}
-
-void k_final_ranges_all(hbtx_ctx *c, Batch &B, View &V)
-{
-  k_all_ranges<<<blocks_for(V.nsub, 256, 1 << 20), 256, 0, c->stream>>>(V.S, B.rbegin.p, B.rlen.p);
-}
-
 // Iterate one view to convergence. Returns rounds used.
 // Per-view state at the start of the unbinding: particles, frames, the initial
 // Mbound (:537-541) and the leading do-not-subsample run (:522-524).
@@ -1243,8 +1259,7 @@ void init_view(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, bool warm)
   k_init_particles<<<gb, 256, 0, st>>>(V.S, V.Q, V.n);
   k_init_subs<<<gs, 256, 0, st>>>(V.S, B.ref_in.p + 6 * V.s0, B.mb_in.p + 6 * V.s0, nullptr);
   k_fill_i32<<<1, 64, 0, st>>>(B.misc.p, 8, 0);
-  k_final_ranges_all(c, B, V);
-  const int32_t *nt = red_tiles(c, B.rbegin.p, B.rlen.p, V.nsub, V.n);
+  const int32_t *nt = red_tiles(c, RangeAll{V.S}, V.nsub, V.n);
   k_fill_i32<<<gs, 256, 0, st>>>(B.aux32.p, V.nsub, 0x7fffffff);
   k_fill_i32<<<gs, 256, 0, st>>>(V.S.first_idx, V.nsub, 0x7fffffff);
   if (warm && P.periodic)
@@ -1261,10 +1276,10 @@ void init_view(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, bool warm)
 }
 
 // First part of a round, up to the walk: plan, sources, octrees, work items.
-// graph: no host synchronisation (the part is being captured).  level (a bound
-// the host knows from the previous round): 0 any subhalo; 1 every active
-// subhalo fits the LDS sort (no radix passes); 2 every active subhalo also takes
-// the direct sum (no tree cells, no moment passes).
+// graph: no host synchronisation (the part is being captured).  level (from the
+// largest source count of the round, which the host has from the round before): 0
+// any; 1 every subhalo's sources fit the LDS sort (no radix passes); 2 every subhalo
+// takes the direct sum (no keys, sorts, cells or moments).
 void round_head(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, bool graph, bool warm_round, int level = 0)
 {
   hipStream_t st = c->stream;
@@ -1272,12 +1287,11 @@ void round_head(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, bool graph, 
   k_round_begin<<<1, 64, 0, st>>>(V.S.active_count, round_ptr(B), V.S.max_active_n);
   k_plan<<<gs, 256, 0, st>>>(V.S, P, round_ptr(B));
   round_sources_and_tree(c, B, V, P, graph, level);
-  if (warm_round)
+  if (warm_round && level < 2)
   {
     // warm round: every target, in Hilbert order of its cell in the proposal's tree cube
-    k_warm_keys<<<blocks_for(V.n), 256, 0, st>>>(V.S, V.Q, V.n, B.keys.p, B.seg_begin.p, B.seg_len.p);
-    k_warm_segments<<<gs, 256, 0, st>>>(V.S, B.seg_begin.p, B.seg_len.p);
-    seg_sort(c, B.keys.p, V.Q.cur, V.nsub, B.seg_begin.p, B.seg_len.p, V.n, 30);
+    k_warm_keys<<<blocks_for(V.n), 256, 0, st>>>(V.S, V.Q, V.n, B.keys.p);
+    seg_sort(c, B.keys.p, V.Q.cur, V.nsub, RangeWarm{V.S}, B.seg_begin.p, B.seg_len.p, V.n, 30, V.max_count);
   }
   round_items(c, B, V);
 }
@@ -1390,8 +1404,12 @@ int run_view(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, bool want_pot, 
   }
   init_view(c, B, V, P, warm);
   c->walk_items_hint = INT64_MAX;
-  int round = 0, level = 0;
+  // (the first round's sources: at most every particle)
+  auto level_of = [&](int64_t max_src) { return (max_src <= P.direct_cutoff) ? 2 : (max_src <= SORT_SMALL_MAX ? 1 : 0); };
+  int round = 0, level = level_of(V.max_count);
   const int max_rounds = 2000;
+  if (!c->round_words)
+    HIPCHK(hipHostMalloc((void **)&c->round_words, 8 * sizeof(int32_t), hipHostMallocDefault));
   while (true)
   {
     REQUIRE(round < max_rounds, HBTX_E_INVALID, "unbinding did not converge within the round limit");
@@ -1406,13 +1424,16 @@ int run_view(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, bool want_pot, 
     }
     else
     {
-      round_head(c, B, V, P, false, warm && round == 1, round == 1 ? 0 : level);
+      round_head(c, B, V, P, false, warm && round == 1, level);
       round_walk_launch(c, B, V, P);
       round_partition(c, B, V, P, warm && round == 1);
     }
-    int32_t h_misc[8];
-    HIPCHK(hipMemcpyAsync(h_misc, B.misc.p, sizeof(h_misc), hipMemcpyDeviceToHost, st));
+    // the round's words straight into pinned host memory (a copy of 32 bytes costs more
+    // than the wait itself)
+    k_publish<<<1, 64, 0, st>>>(B.misc.p, c->round_words, 8);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(st));
+    const int32_t *h_misc = c->round_words;
     float wms = 0.f;
     HIPCHK(hipEventElapsedTime(&wms, c->wev0, c->wev1));
     c->walk_ms += wms;
@@ -1420,9 +1441,7 @@ int run_view(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, bool want_pot, 
     c->tree_entries += h_misc[3];
     if (round == 1)
       c->tree_entries_first += h_misc[3];
-    // the next round's level: subhaloes only leave the active set
-    const int64_t maxn = h_misc[6];
-    level = (maxn <= P.direct_cutoff) ? 2 : (maxn <= SORT_SMALL_MAX ? 1 : 0);
+    level = level_of(h_misc[6]);
     check_overflow(h_misc[2]);
     if (h_misc[0] == 0)
       break;
@@ -1717,7 +1736,7 @@ void tree_points(hbtx_ctx *c, hbtx_tree *T, int64_t nt, const float *tpos, const
   W.phi.alloc(nt);
   W.keys.alloc(nt);
   W.vals.alloc(nt);
-  W.seg.alloc(2);
+  W.seg.alloc(4); // the range, and the sort's copy of it
   W.counter.alloc(2); // [0] work counter, [1] overflow word
   std::vector<XferPart> parts{xfer_from(0, tpos, 3 * nt * sizeof(float))};
   if (tmass)
@@ -1728,7 +1747,7 @@ void tree_points(hbtx_ctx *c, hbtx_tree *T, int64_t nt, const float *tpos, const
   // walk order: targets sorted by their key in the tree cube
   k_point_keys<<<blocks_for(nt), 256, 0, st>>>(W.tgt.p, (int32_t)nt, T->cube.p, W.keys.p, W.vals.p);
   if (T->treemode)
-    seg_sort(c, W.keys.p, W.vals.p, 1, W.seg.p, W.seg.p + 1, nt, 63);
+    seg_sort(c, W.keys.p, W.vals.p, 1, RangeArray{W.seg.p, W.seg.p + 1}, W.seg.p + 2, W.seg.p + 3, nt, 63, nt);
   PointArgs A;
   A.tgt = W.tgt.p;
   A.tgt_order = W.vals.p;
@@ -1906,6 +1925,8 @@ void hbtx_destroy(hbtx_ctx *c)
   if (c->wev1)
     (void)hipEventDestroy(c->wev1);
   drop_graphs(c);
+  if (c->round_words)
+    (void)hipHostFree(c->round_words);
   hipStream_t st = c->stream;
   delete c;
   if (st)
@@ -2259,7 +2280,8 @@ int hbtx_batch_profiles(hbtx_ctx *c, const hbtx_params *prm, hbtx_sub_profile *o
     A.seg_len = B.seg_len.p;
     A.rc = B.prof_r.p;
     A.mc = B.prof_m.p;
-    run_profiles(c, *prm, A, B.n, B.nsub, B.sub_of.p, B.seg_begin.p, B.seg_len.p, B.keys.p, B.src.p, B.dprof.p);
+    run_profiles(c, *prm, A, B.n, B.nsub, B.sub_of.p, B.seg_begin.p, B.seg_len.p, B.keys.p, B.src.p, B.dprof.p,
+                 B.max_count);
     HIPCHK(c->staging.down(c->device, c->stream, {xfer_to(out, B.dprof.p, B.nsub * sizeof(hbtx_sub_profile))}));
   });
 }
@@ -2276,6 +2298,7 @@ int hbtx_profiles(hbtx_ctx *c, const hbtx_params *prm, int64_t n, const float *p
     hipStream_t st = c->stream;
     std::vector<int32_t> hoff(nsub + 1);
     std::vector<hbtx_sub_result> hres(nsub);
+    int64_t max_len = 0;
     for (int64_t s = 0; s < nsub; s++)
     {
       const int64_t a = offsets[s], e = offsets[s + 1];
@@ -2286,6 +2309,7 @@ int hbtx_profiles(hbtx_ctx *c, const hbtx_params *prm, int64_t n, const float *p
       std::memset(&R, 0, sizeof(R));
       R.nbound = nbound[s];
       R.mbound = mbound[s];
+      max_len = std::max(max_len, nbound[s]);
       if (nbound[s] > 0)
         for (int k = 0; k < 3; k++)
           R.mostbound_pos[k] = pos[3 * a + k];
@@ -2320,7 +2344,8 @@ int hbtx_profiles(hbtx_ctx *c, const hbtx_params *prm, int64_t n, const float *p
     A.seg_len = W.seg.p + nsub + 1;
     A.rc = W.rc.p;
     A.mc = W.mc.p;
-    run_profiles(c, *prm, A, n, (int32_t)nsub, W.sub_of.p, W.seg.p, W.seg.p + nsub + 1, W.keys.p, W.vals.p, W.prof.p);
+    run_profiles(c, *prm, A, n, (int32_t)nsub, W.sub_of.p, W.seg.p, W.seg.p + nsub + 1, W.keys.p, W.vals.p, W.prof.p,
+                 max_len);
     HIPCHK(c->staging.down(c->device, st, {xfer_to(out, W.prof.p, nsub * sizeof(hbtx_sub_profile))}));
   });
 }
@@ -2340,8 +2365,12 @@ int hbtx_reassign_targets(hbtx_ctx *c, const hbtx_params *prm, int64_t n, const 
     REQUIRE(k >= 1 && k <= 32, HBTX_E_INVALID, "k (NumNeighboursForReassignment) must lie in 1..32");
     REQUIRE(group_offsets[0] == 0 && group_offsets[ngroups] == n, HBTX_E_INVALID,
             "group offsets must start at 0 and end at n");
+    int64_t max_group = 0;
     for (int64_t g = 0; g < ngroups; g++)
+    {
       REQUIRE(group_offsets[g] <= group_offsets[g + 1], HBTX_E_INVALID, "group offsets must ascend");
+      max_group = std::max(max_group, group_offsets[g + 1] - group_offsets[g]);
+    }
     // GeoTree_t::NearestNeighbours(centre, k, SofteningHalo * 0.1) (src/subhalo_reassign_gas.cpp:144)
     const float r0 = (rguess > 0.f) ? rguess : (float)(prm->softening * 0.1);
     REQUIRE(r0 > 0.f && std::isfinite(r0), HBTX_E_INVALID, "the first search radius must be positive");
@@ -2373,7 +2402,7 @@ int hbtx_reassign_targets(hbtx_ctx *c, const hbtx_params *prm, int64_t n, const 
     R.qval.alloc(n);
     R.tkey.alloc(n);
     R.qkey.alloc(n);
-    R.seg.alloc(4 * (int64_t)G);
+    R.seg.alloc(6 * (int64_t)G);
     R.out.alloc(n);
     R.tot.alloc(RS_LEVELS + 2);
     R.grp.alloc(G);
@@ -2438,9 +2467,11 @@ int hbtx_reassign_targets(hbtx_ctx *c, const hbtx_params *prm, int64_t n, const 
     HIPCHK(hipMemcpyAsync(R.lbase.p, lb, sizeof(lb), hipMemcpyHostToDevice, st));
     k_rs_keys<<<blocks_for(n), 256, 0, st>>>(A, NT);
     k_rs_group_finish<<<blocks_for(G, 256, 1 << 20), 256, 0, st>>>(A);
-    seg_sort(c, R.tkey.p, R.tval.p, G, R.seg.p, R.seg.p + G, std::max<int32_t>(NT, 1), 3 * RS_KEY_BITS);
-    seg_sort(c, R.qkey.p, R.qval.p, G, R.seg.p + 2 * (int64_t)G, R.seg.p + 3 * (int64_t)G,
-             std::max<int64_t>(n - NT, 1), 3 * RS_KEY_BITS);
+    int32_t *sort_b = R.seg.p + 4 * (int64_t)G, *sort_l = R.seg.p + 5 * (int64_t)G;
+    seg_sort(c, R.tkey.p, R.tval.p, G, RangeArray{R.seg.p, R.seg.p + G}, sort_b, sort_l, std::max<int32_t>(NT, 1),
+             3 * RS_KEY_BITS, max_group);
+    seg_sort(c, R.qkey.p, R.qval.p, G, RangeArray{R.seg.p + 2 * (int64_t)G, R.seg.p + 3 * (int64_t)G}, sort_b, sort_l,
+             std::max<int64_t>(n - NT, 1), 3 * RS_KEY_BITS, max_group);
     if (NT > 0)
       k_rs_records<<<blocks_for(NT), 256, 0, st>>>(A, NT);
     for (int l = 0; l < RS_LEVELS; l++)
@@ -2482,7 +2513,10 @@ int hbtx_segmented_sort(hbtx_ctx *c, int64_t n, uint64_t *keys, int32_t *vals, i
     REQUIRE(n < (int64_t)0x40000000 && nseg < (int64_t)0x7fffffff, HBTX_E_INVALID, "too large");
     hipStream_t st = c->stream;
     DArr<uint64_t> dk;
-    DArr<int32_t> dv, sb, sl;
+    DArr<int32_t> dv, sb, sl, sb2, sl2;
+    int64_t max_len = 0;
+    sb2.alloc(nseg);
+    sl2.alloc(nseg);
     dk.alloc(n);
     dv.alloc(n);
     sb.alloc(nseg);
@@ -2493,6 +2527,7 @@ int hbtx_segmented_sort(hbtx_ctx *c, int64_t n, uint64_t *keys, int32_t *vals, i
       REQUIRE(seg_offsets[s + 1] >= seg_offsets[s], HBTX_E_INVALID, "bad segments");
       hb[s] = (int32_t)seg_offsets[s];
       hl[s] = (int32_t)(seg_offsets[s + 1] - seg_offsets[s]);
+      max_len = std::max<int64_t>(max_len, hl[s]);
     }
     HIPCHK(c->staging.up(c->device, st, dk.p, {xfer_from(0, keys, n * 8)}));
     HIPCHK(c->staging.up(c->device, st, dv.p, {xfer_from(0, vals, n * 4)}));
@@ -2505,7 +2540,7 @@ int hbtx_segmented_sort(hbtx_ctx *c, int64_t n, uint64_t *keys, int32_t *vals, i
     int bits = 1;
     while (bits < 64 && (any >> bits) != 0)
       bits++;
-    seg_sort(c, dk.p, dv.p, (int32_t)nseg, sb.p, sl.p, n, bits);
+    seg_sort(c, dk.p, dv.p, (int32_t)nseg, RangeArray{sb.p, sl.p}, sb2.p, sl2.p, n, bits, max_len);
     HIPCHK(c->staging.down(c->device, st, {xfer_to(keys, dk.p, n * 8), xfer_to(vals, dv.p, n * 4)}));
   });
 }

@@ -2,6 +2,7 @@
 // block scan + offset).  out[i] = sum(in[0..i)), out[n] = total.  In-place safe.
 #pragma once
 #include "common.h"
+#include <type_traits>
 
 namespace hbtx
 {
@@ -9,18 +10,52 @@ namespace hbtx
 #define SCAN_ITEMS 16
 #define SCAN_TILE (SCAN_THREADS * SCAN_ITEMS)
 
+// the value that lane - shift of the same row of 16 (or the last lane of the row or
+// half before, for the broadcasts) holds, 0 where there is none
+template <int CTRL, int ROWS, typename T>
+HBTX_DEV T dpp_shifted(T v)
+{
+  static_assert(std::is_integral<T>::value && (sizeof(T) == 4 || sizeof(T) == 8), "integers of one or two words");
+  if constexpr (sizeof(T) == 4)
+    return (T)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+  else
+  {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(uint64_t)v, CTRL, ROWS, 0xf, false);
+    const uint32_t hi =
+      (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)((uint64_t)v >> 32), CTRL, ROWS, 0xf, false);
+    return (T)(((uint64_t)hi << 32) | lo);
+  }
+}
+
+// Inclusive prefix sum over the wave.  Integers: lane moves inside the vector
+// instructions (within rows of 16, then across rows and halves); six LDS shuffles a
+// scan made a 16-wave block's scan LDS-bound (5 us for 8192 values).  Floating
+// point keeps the shuffles, whose order of additions its results have.
 template <typename T>
 HBTX_DEV T wave_incl_scan(T v)
 {
-  const int l = lane_id();
-#pragma unroll
-  for (int d = 1; d < HBTX_WAVE; d <<= 1)
+  if constexpr (std::is_integral<T>::value)
   {
-    T o = __shfl_up(v, d, HBTX_WAVE);
-    if (l >= d)
-      v += o;
+    v += dpp_shifted<0x111, 0xf>(v); // row_shr:1
+    v += dpp_shifted<0x112, 0xf>(v); // row_shr:2
+    v += dpp_shifted<0x114, 0xf>(v); // row_shr:4
+    v += dpp_shifted<0x118, 0xf>(v); // row_shr:8
+    v += dpp_shifted<0x142, 0xa>(v); // row_bcast:15 into rows 1 and 3
+    v += dpp_shifted<0x143, 0xc>(v); // row_bcast:31 into rows 2 and 3
+    return v;
   }
-  return v;
+  else
+  {
+    const int l = lane_id();
+#pragma unroll
+    for (int d = 1; d < HBTX_WAVE; d <<= 1)
+    {
+      T o = __shfl_up(v, d, HBTX_WAVE);
+      if (l >= d)
+        v += o;
+    }
+    return v;
+  }
 }
 
 // Exclusive scan of one value per thread across a 256-thread block; returns the

@@ -206,33 +206,6 @@ __global__ __launch_bounds__(SORT_THREADS) void k_sort_wave4(uint64_t *__restric
   }
 }
 
-// Number of radix tiles of every segment (0 for segments sorted in LDS).
-__global__ void k_sort_ntiles(const int32_t *__restrict__ seg_len, int32_t nseg, int32_t *__restrict__ ntile)
-{
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s < nseg)
-  {
-    const int len = seg_len[s];
-    ntile[s] = (len > SORT_SMALL_MAX) ? (len + SORT_TILE - 1) / SORT_TILE : 0;
-  }
-}
-
-// tiles[t] = (segment, begin, end, 0)
-__global__ void k_sort_tiles(const int32_t *__restrict__ seg_begin, const int32_t *__restrict__ seg_len,
-                             const int32_t *__restrict__ tile_off, int32_t nseg, int4 *__restrict__ tiles)
-{
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= nseg)
-    return;
-  const int len = seg_len[s];
-  if (len <= SORT_SMALL_MAX)
-    return;
-  const int b = seg_begin[s], e = b + len;
-  int t = tile_off[s];
-  for (int x = b; x < e; x += SORT_TILE, t++)
-    tiles[t] = make_int4(s, x, min(e, x + SORT_TILE), 0);
-}
-
 template <int RB>
 __global__ __launch_bounds__(SORT_THREADS) void k_radix_hist(const uint64_t *__restrict__ kin,
                                                             const int4 *__restrict__ tiles,

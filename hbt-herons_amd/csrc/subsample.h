@@ -197,16 +197,6 @@ __global__ __launch_bounds__(256) void k_upscale_tiles(SubArrays S, PartArrays Q
   }
 }
 
-// Ranges for the upscale sums: full-mode subhaloes that subsample this round.
-__global__ void k_upscale_ranges(SubArrays S, int32_t *begin, int32_t *len)
-{
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= S.nsub)
-    return;
-  begin[s] = S.off[s];
-  len[s] = (S.mode[s] == MODE_FULL && S.nsrc[s] < S.ntgt[s]) ? (S.off[s + 1] - S.off[s]) : 0;
-}
-
 // GetMassUpscaleFactor (:290-317) or ...PerParticleType (:323-361), in float.
 __global__ void k_upscale_finish(SubArrays S, DevParams P, const double *red)
 {
@@ -318,8 +308,7 @@ __global__ void k_mark_refine(SubArrays S, PartArrays Q, int64_t n, const int32_
   }
 }
 
-__global__ void k_refine_keys(SubArrays S, int64_t n, const int32_t *vals, const float *eref, uint64_t *keys,
-                              int32_t *seg_begin, int32_t *seg_len)
+__global__ void k_refine_keys(SubArrays S, int64_t n, const int32_t *vals, const float *eref, uint64_t *keys)
 {
   GRID_STRIDE(q, n)
   {
@@ -327,15 +316,6 @@ __global__ void k_refine_keys(SubArrays S, int64_t n, const int32_t *vals, const
     if (S.mode[s] == MODE_REFINE && (int)(q - S.off[s]) < S.nsrc[s])
       keys[q] = (uint64_t)float_to_ordered(eref[vals[q]]);
   }
-}
-
-__global__ void k_refine_segments(SubArrays S, int32_t *seg_begin, int32_t *seg_len)
-{
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= S.nsub)
-    return;
-  seg_begin[s] = S.off[s];
-  seg_len[s] = (S.mode[s] == MODE_REFINE) ? S.nsrc[s] : 0;
 }
 
 } // namespace hbtx

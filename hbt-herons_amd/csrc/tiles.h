@@ -14,27 +14,7 @@ namespace hbtx
 #define SLOT_THREADS 256
 #define SLOT_ITEMS (SLOT_TILE / SLOT_THREADS)
 
-__global__ void k_slot_ntiles(SubArrays S, int32_t *ntile)
-{
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= S.nsub)
-    return;
-  const int n = S.off[s + 1] - S.off[s];
-  ntile[s] = (S.mode[s] != MODE_IDLE) ? (n + SLOT_TILE - 1) / SLOT_TILE : 0;
-}
-
-// tile = (subhalo, first slot, end slot, index of the subhalo's first tile)
-__global__ void k_slot_tiles(SubArrays S, const int32_t *toff, int4 *tiles)
-{
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= S.nsub || S.mode[s] == MODE_IDLE)
-    return;
-  const int b = S.off[s], e = S.off[s + 1];
-  const int t0 = toff[s];
-  for (int k = 0; b + k * SLOT_TILE < e; k++)
-    tiles[t0 + k] = make_int4(s, b + k * SLOT_TILE, min(e, b + (k + 1) * SLOT_TILE), t0);
-}
-
+// (tile = (subhalo, first slot, end slot, index of the subhalo's first tile))
 // Pass 1: per tile sum of the flags (tsum[t] = 0 for t in [ntiles, maxt)).
 template <typename T>
 __global__ __launch_bounds__(SLOT_THREADS) void k_tile_sum(const int4 *__restrict__ tiles, const int32_t *ntiles_p,

@@ -195,6 +195,20 @@ __global__ void k_tree_emit(TreeArgs A)
     tree_emit_one(A, j);
 }
 
+// The records of a round of direct sums only: source j's at unit 2 j (no cells).
+__global__ void k_emit_direct(TreeArgs A)
+{
+  const int S = *A.s_total;
+  for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < S; j += gridDim.x * blockDim.x)
+  {
+    const int p = A.src[j];
+    const float4 x = A.posm[p];
+    const float m = source_mass(A, p, A.src_sub[j]);
+    A.wt[2 * j] = make_uint2(__float_as_uint(x.x), __float_as_uint(x.y));
+    A.wt[2 * j + 1] = make_uint2(__float_as_uint(x.z), __float_as_uint(m));
+  }
+}
+
 // Cell moments (mass and centre of mass) bottom-up, in child (sub-index) order
 // with double accumulation of the float child values, as UpdateInternalNodes /
 // ProcessNode do (src/gravity_tree.cpp:25-80), without one launch per depth.

@@ -32,7 +32,7 @@ struct SubArrays
   int32_t *bnd_cnt, *bnd_tr;
   int32_t *first_idx;       // smallest candidate index (periodic reference particle)
   int32_t *active_count;    // [1]
-  int32_t *max_active_n;    // [1] particles of the largest subhalo still active after the round
+  int32_t *max_active_n;    // [1] sources of the next round's largest source set
   // learned warm start: warm = WARM_* state; npro = proposed particles; nadd = bound
   // particles outside the proposal (re-admitted by the warm round); reset = proposal
   // rejected, restart from all particles
@@ -62,10 +62,10 @@ __global__ void k_fill_i32(int32_t *p, int64_t n, int32_t v)
 {
   GRID_STRIDE(i, n) p[i] = v;
 }
-__global__ void k_copy_i32(const int32_t *src, int32_t *dst)
+__global__ void k_publish(const int32_t *src, int32_t *dst, int n)
 {
-  if (blockIdx.x == 0 && threadIdx.x == 0)
-    *dst = *src;
+  if ((int)threadIdx.x < n)
+    dst[threadIdx.x] = src[threadIdx.x];
 }
 __global__ void k_fill_u64(unsigned long long *p, int64_t n, unsigned long long v)
 {
@@ -280,61 +280,23 @@ __global__ void k_sub_src(SubArrays S, const int32_t *sub_first)
   }
 }
 
-// Bounding box of each tree-mode subhalo's sources (src/oct_tree.tpp:344-355).
-// Waves whose lanes share one subhalo reduce first, then one atomic per wave.
-__global__ void k_bbox(SubArrays S, const float4 *posm, const int32_t *src, const int32_t *s_total)
+// A round of direct sums only: source ranges and their record units (k_emit_direct),
+// and the round's entries, which are its sources.
+__global__ void k_sub_src_direct(SubArrays S, const int32_t *sub_first, const int32_t *s_total, int32_t *e_total)
 {
-  const int ST = *s_total;
-  for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < ST; base += (int64_t)gridDim.x * blockDim.x)
-  {
-    const int64_t j = base + threadIdx.x;
-    const bool valid = j < ST;
-    int s = -1;
-    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (valid)
-    {
-      const int p = src[j];
-      s = S.sub_of[p];
-      if (!S.treemode[s])
-        s = -1;
-      else
-        x = posm[p];
-    }
-    const int s0 = __shfl(s, 0, HBTX_WAVE);
-    const bool same = ballot(s != s0) == 0ull;
-    if (same)
-    {
-      if (s0 < 0)
-        continue;
-      float mn[3] = {x.x, x.y, x.z}, mx[3] = {x.x, x.y, x.z};
-#pragma unroll
-      for (int d = 1; d < HBTX_WAVE; d <<= 1)
-#pragma unroll
-        for (int k = 0; k < 3; k++)
-        {
-          mn[k] = fminf(mn[k], __shfl_xor(mn[k], d, HBTX_WAVE));
-          mx[k] = fmaxf(mx[k], __shfl_xor(mx[k], d, HBTX_WAVE));
-        }
-      if (lane_id() == 0)
-        for (int k = 0; k < 3; k++)
-        {
-          atomicMin(S.bbox + 6 * s0 + k, float_to_ordered(mn[k]));
-          atomicMax(S.bbox + 6 * s0 + 3 + k, float_to_ordered(mx[k]));
-        }
-    }
-    else if (s >= 0)
-    {
-      const float xs[3] = {x.x, x.y, x.z};
-      for (int k = 0; k < 3; k++)
-      {
-        atomicMin(S.bbox + 6 * s + k, float_to_ordered(xs[k]));
-        atomicMax(S.bbox + 6 * s + 3 + k, float_to_ordered(xs[k]));
-      }
-    }
-  }
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s == 0)
+    *e_total = *s_total;
+  if (s >= S.nsub)
+    return;
+  const int b = (S.mode[s] != MODE_IDLE) ? sub_first[s] : 0;
+  S.src_off[s] = b;
+  S.ent_begin[s] = wrec_unit(b, 0);
+  S.ent_end[s] = wrec_unit(b + S.nsrc[s], 0);
 }
 
-// Bounding box per tile of a dense source range (tiles never span subhaloes):
+// Bounding box of each tree-mode subhalo's sources (src/oct_tree.tpp:344-355), per
+// tile of a dense source range (tiles never span subhaloes):
 // block min/max reduction, then six atomics per tile (min/max are order-free).
 __global__ __launch_bounds__(256) void k_bbox_tiles(SubArrays S, const float4 *posm, const int32_t *src,
                                                     const int4 *tiles, const int32_t *ntiles_p)
@@ -390,16 +352,6 @@ __global__ __launch_bounds__(256) void k_bbox_tiles(SubArrays S, const float4 *p
   }
 }
 
-// Dense source ranges of tree-mode subhaloes (for the bounding-box tiles).
-__global__ void k_tree_src_ranges(SubArrays S, int32_t *begin, int32_t *len)
-{
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= S.nsub)
-    return;
-  begin[s] = S.src_off[s];
-  len[s] = (S.mode[s] != MODE_IDLE && S.treemode[s]) ? S.nsrc[s] : 0;
-}
-
 // Root cube: Len = max extent, Center = bbox midpoint (src/oct_tree.tpp:357-365).
 __global__ void k_cube(SubArrays S)
 {
@@ -440,16 +392,6 @@ __global__ void k_keys(SubArrays S, DevParams P, const float4 *posm, const int32
     const uint64_t k = octree_key(x.x, x.y, x.z, c[0], c[1], c[2], c[3]);
     keys[j] = hash_digits(k, resolution_depth(c[3], 0.5 * P.res), (uint32_t)(p - S.off[s]));
   }
-}
-
-// Sort segments: tree-mode sources only.
-__global__ void k_sort_segments(SubArrays S, int32_t *seg_begin, int32_t *seg_len)
-{
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= S.nsub)
-    return;
-  seg_begin[s] = S.src_off[s];
-  seg_len[s] = (S.mode[s] != MODE_IDLE && S.treemode[s]) ? S.nsrc[s] : 0;
 }
 
 // Walk order of a full round: when every target is a source, the targets take
@@ -706,7 +648,7 @@ __global__ void k_warm_reset_subs(SubArrays S, const float *ref_in)
 
 // Warm-round walk order: every target sorted by its key in the proposal's tree cube
 // (top 10 levels).
-__global__ void k_warm_keys(SubArrays S, PartArrays Q, int64_t n, uint64_t *keys, int32_t *seg_begin, int32_t *seg_len)
+__global__ void k_warm_keys(SubArrays S, PartArrays Q, int64_t n, uint64_t *keys)
 {
   GRID_STRIDE(q, n)
   {
@@ -722,17 +664,6 @@ __global__ void k_warm_keys(SubArrays S, PartArrays Q, int64_t n, uint64_t *keys
       keys[q] = hilbert3_10(octree_key(x.x, x.y, x.z, c[0], c[1], c[2], c[3]) >> (3 * (HBTX_KEY_LEVELS - 10)));
     }
   }
-}
-
-__global__ void k_warm_segments(SubArrays S, int32_t *seg_begin, int32_t *seg_len)
-{
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= S.nsub)
-    return;
-  seg_begin[s] = S.off[s];
-  seg_len[s] = (S.warm[s] == WARM_PENDING && S.mode[s] == MODE_FULL && S.treemode[s] && S.nsrc[s] < S.ntgt[s])
-                 ? (S.off[s + 1] - S.off[s])
-                 : 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -815,24 +746,6 @@ HBTX_DEV void wave_reduce_tile(int b, int e, double tot[RED_NV], Acc acc)
       tot[k] += x;
     }
   }
-}
-
-__global__ void k_red_ntiles(const int32_t *len, int32_t nsub, int32_t *ntile)
-{
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s < nsub)
-    ntile[s] = (len[s] + RED_TILE - 1) / RED_TILE;
-}
-
-__global__ void k_red_tiles(const int32_t *begin, const int32_t *len, const int32_t *toff, int32_t nsub, int4 *tiles)
-{
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= nsub)
-    return;
-  const int b = begin[s], e = b + len[s];
-  int t = toff[s];
-  for (int x = b; x < e; x += RED_TILE, t++)
-    tiles[t] = make_int4(s, x, min(e, x + RED_TILE), 0);
 }
 
 // Centre-of-mass frame of the bound candidates (CentreOfMassReferenceFrame, :151-198),
@@ -928,16 +841,6 @@ inline int red_finalize_blocks(int32_t nsub)
   return (int)(((int64_t)nsub * RED_NV + 255) / 256);
 }
 
-// Reduction range of the CoM: bound candidates of subhaloes still active after the decision.
-__global__ void k_com_ranges(SubArrays S, int32_t *begin, int32_t *len)
-{
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= S.nsub)
-    return;
-  begin[s] = S.off[s];
-  len[s] = (S.mode[s] != MODE_IDLE && S.status[s] == ST_ACTIVE) ? (S.off[s + 1] - S.off[s]) : 0;
-}
-
 // smallest input index among bound candidates (the E list's first particle)
 __global__ void k_first_index(SubArrays S, PartArrays Q, int64_t n)
 {
@@ -978,7 +881,17 @@ __global__ void k_round_finish(SubArrays S, DevParams P, const double *red)
   else
   {
     atomicAdd(S.active_count, 1);
-    atomicMax(S.max_active_n, S.off[s + 1] - S.off[s]);
+    // the sources k_plan will give it
+    int ns = (int)nb;
+    if (S.reset[s])
+      ns = S.off[s + 1] - S.off[s];
+    else if (S.warm[s] == WARM_ADD)
+      ns = S.nadd[s];
+    else if (S.corr[s])
+      ns = S.nrem[s];
+    else if (P.mss > 0)
+      ns = (int)min(nb, P.mss + S.nuns[s]);
+    atomicMax(S.max_active_n, ns);
   }
 }
 
@@ -1020,15 +933,6 @@ __global__ void k_final_keys(SubArrays S, PartArrays Q, int64_t n, int32_t round
     keys[p] = key;
     vals[p] = (int32_t)p;
   }
-}
-
-__global__ void k_final_segments(SubArrays S, int32_t *seg_begin, int32_t *seg_len)
-{
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= S.nsub)
-    return;
-  seg_begin[s] = S.off[s];
-  seg_len[s] = (S.status[s] == ST_CONVERGED) ? (S.off[s + 1] - S.off[s]) : 0;
 }
 
 // AverageKinematics (:200-249) and CountParticleTypes sums over the bound particles
@@ -1218,15 +1122,6 @@ __global__ void k_core_wave(SubArrays S, PartArrays Q, DevParams P, const int32_
     if (lane_id() == 0)
       out[(int64_t)RED_NV * s + k] = x;
   }
-}
-
-__global__ void k_final_ranges(SubArrays S, int32_t *begin, int32_t *len)
-{
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= S.nsub)
-    return;
-  begin[s] = S.off[s];
-  len[s] = (S.status[s] == ST_CONVERGED) ? (S.off[s + 1] - S.off[s]) : 0;
 }
 
 // ParticlePotentialEnergies (GetPotentialEnergy, :114-135) of the bound part.
