@@ -1053,7 +1053,7 @@ void round_partition(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, bool wa
   scan_excl<int64_t>(c, B.tsum64.p, B.tpre64.p, maxt, c->part64);
   k_partition_scatter<<<tg, SLOT_THREADS, 0, st>>>(V.S, V.Q, B.stiles.p, nt, round_ptr(B), B.flag64.p, B.tpre64.p,
                                                    B.sub_total64.p);
-  k_copy_cur<<<tg, 256, 0, st>>>(V.S, V.Q, B.stiles.p, nt, B.sub_total64.p);
+  k_copy_cur<<<tg, 256, 0, st>>>(V.S, V.Q, B.stiles.p, nt, B.sub_total64.p, P.periodic);
   if (P.mss > 0)
   {
     k_fill_i32<<<gs, 256, 0, st>>>(B.aux32.p, V.nsub, 0);
@@ -1061,11 +1061,6 @@ void round_partition(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, bool wa
     k_set_unsampled<<<gs, 256, 0, st>>>(V.S, B.aux32.p);
   }
   k_round_decide<<<gs, 256, 0, st>>>(V.S, P, B.sub_total64.p, warm_round ? B.aux32.p : nullptr);
-  if (P.periodic)
-  {
-    k_fill_i32<<<gs, 256, 0, st>>>(V.S.first_idx, V.nsub, 0x7fffffff);
-    k_first_index<<<gb, 256, 0, st>>>(V.S, V.Q, n);
-  }
   const int32_t *ntiles = red_tiles(c, RangeCom{V.S}, V.nsub, n);
   k_red_tile<ComOp><<<red_grid(c, n, V.nsub), RED_THREADS, 0, st>>>(V.S, V.Q, P, c->red_tiles.p, ntiles,
                                                                      c->red_partial.p);

@@ -115,8 +115,16 @@ __global__ void k_first_proposed(SubArrays S, PartArrays Q, int64_t n)
 {
   GRID_STRIDE(p, n)
   {
-    if (Q.proposal[p])
-      atomicMin(S.first_idx + S.sub_of[p], (int32_t)p);
+    const int s = S.sub_of[p];
+    const uint64_t m = ballot(Q.proposal[p] != 0);
+    if (ballot(s != uniform(s)) == 0ull)
+    {
+      // one subhalo's wave: its first proposed lane has the smallest slot
+      if (m != 0ull && lane_id() == __ffsll((long long)m) - 1)
+        atomicMin(S.first_idx + s, (int32_t)p);
+    }
+    else if (Q.proposal[p])
+      atomicMin(S.first_idx + s, (int32_t)p);
   }
 }
 

@@ -129,6 +129,7 @@ __global__ void k_plan(SubArrays S, DevParams P, const int32_t *round_p)
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= S.nsub)
     return;
+  S.first_idx[s] = 0x7fffffff;
   if (S.status[s] != ST_ACTIVE)
   {
     S.mode[s] = MODE_IDLE;
@@ -513,8 +514,11 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_partition_flags(SubArrays S, P
     tsum[t] = 0;
 }
 
+// The compacted candidates back to cur; per subhalo also the smallest index among
+// them, the E list's first particle, which a periodic frame wraps about (one atomic
+// a wave: a pass of its own with one a particle took 830 us for 10^6 particles).
 __global__ void k_copy_cur(SubArrays S, PartArrays Q, const int4 *tiles, const int32_t *ntiles_p,
-                           const int64_t *sub_total)
+                           const int64_t *sub_total, int periodic)
 {
   TILE_LOOP(tiles, ntiles_p)
   {
@@ -522,8 +526,21 @@ __global__ void k_copy_cur(SubArrays S, PartArrays Q, const int4 *tiles, const i
     const int s = tl.x;
     const int nb = (int)(sub_total[s] & 0xffffffffll);
     const int end = min(tl.z, S.off[s] + nb);
+    int32_t first = 0x7fffffff;
     for (int q = tl.y + threadIdx.x; q < end; q += blockDim.x)
-      Q.cur[q] = Q.cur2[q];
+    {
+      const int32_t p = Q.cur2[q];
+      Q.cur[q] = p;
+      first = min(first, p);
+    }
+    if (periodic)
+    {
+#pragma unroll
+      for (int d = 1; d < HBTX_WAVE; d <<= 1)
+        first = min(first, __shfl_xor(first, d, HBTX_WAVE));
+      if (lane_id() == 0 && first != 0x7fffffff)
+        atomicMin(S.first_idx + s, first);
+    }
   }
 }
 
@@ -821,7 +838,9 @@ __global__ __launch_bounds__(RED_THREADS) void k_red_tile(SubArrays S, PartArray
 }
 
 // One thread per (subhalo, value): the tiles' partial sums in tile order, with
-// reads and writes contiguous across the RED_NV values of a subhalo.
+// reads and writes contiguous across the RED_NV values of a subhalo.  Eight tiles'
+// values are loaded together: the serial chain is the additions, not the loads (one
+// load an addition: 31 us for a subhalo of 750,000 particles, 184 tiles).
 __global__ void k_red_finalize(const int32_t *toff, const int32_t *ntile, int32_t nsub, const double *partial,
                                double *out)
 {
@@ -830,27 +849,27 @@ __global__ void k_red_finalize(const int32_t *toff, const int32_t *ntile, int32_
     return;
   const int s = (int)(i / RED_NV), k = (int)(i - (int64_t)s * RED_NV);
   const int t0 = toff[s], n = ntile[s];
+  const double *p = partial + (int64_t)t0 * RED_NV + k;
   double v = 0.;
-  for (int t = t0; t < t0 + n; t++)
-    v += partial[(int64_t)t * RED_NV + k];
+  int t = 0;
+  for (; t + 8 <= n; t += 8)
+  {
+    double x[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      x[j] = p[(int64_t)(t + j) * RED_NV];
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      v += x[j];
+  }
+  for (; t < n; t++)
+    v += p[(int64_t)t * RED_NV];
   out[i] = v;
 }
 
 inline int red_finalize_blocks(int32_t nsub)
 {
   return (int)(((int64_t)nsub * RED_NV + 255) / 256);
-}
-
-// smallest input index among bound candidates (the E list's first particle)
-__global__ void k_first_index(SubArrays S, PartArrays Q, int64_t n)
-{
-  GRID_STRIDE(q, n)
-  {
-    const int s = S.sub_of[q];
-    const int k = (int)(q - S.off[s]);
-    if (S.mode[s] != MODE_IDLE && S.status[s] == ST_ACTIVE && k < S.nbound[s])
-      atomicMin(S.first_idx + s, Q.cur[q]);
-  }
 }
 
 // Frame update and convergence test (:687-690).
