@@ -137,6 +137,16 @@ HBTX_DEV int uniform(int v)
   return __builtin_amdgcn_readfirstlane(v);
 }
 
+// Orders one wave's LDS writes before its later LDS reads by other lanes: the
+// LDS serves a wave's instructions in order, so only the compiler's reordering
+// has to be held back (no workgroup barrier).
+HBTX_DEV void wave_lds_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 HBTX_DEV uint64_t lanemask_lt()
 {
   const int l = lane_id();

@@ -109,7 +109,7 @@ struct DArr
     release();
     g_alloc_gen++;
     size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
-    hipError_t e = hipMalloc((void **)&p, bytes);
+    hipError_t e = hipMalloc((void **)&p, (bytes + 15) & ~(size_t)15); // (small transfers move whole words)
     if (e != hipSuccess)
     {
       p = nullptr;
@@ -1569,8 +1569,7 @@ void upload_batch(hbtx_ctx *c, Batch &B, int64_t n, const float *pos, const floa
   k_load_sub_of<<<blocks_for((n + 3) / 4), 256, 0, st>>>(B.off.p, (int32_t)nsub, n, B.sub_of.p, nullptr);
   HIPCHK(hipGetLastError());
   int32_t bad = 0;
-  HIPCHK(hipMemcpyAsync(&bad, B.load_bad.p, sizeof(bad), hipMemcpyDeviceToHost, st));
-  HIPCHK(hipStreamSynchronize(st));
+  HIPCHK(c->staging.down(c->device, st, {xfer_to(&bad, B.load_bad.p, sizeof(bad))}));
   B.raw.release();
   if (bad)
     B.n = B.nsub = 0; // nothing is loaded
@@ -2579,6 +2578,19 @@ void mlp_upload(hbtx_ctx *c, hbtx_mlp *M, const float *master)
   M->step = 0;
 }
 
+// proposed particles of the loaded batch
+int64_t count_proposed(hbtx_ctx *c, Batch &B)
+{
+  hipStream_t st = c->stream;
+  c->ws.counter.alloc(2);
+  k_fill_i32<<<1, 64, 0, st>>>(c->ws.counter.p, 1, 0);
+  k_count_flags<<<blocks_for((B.n + 15) / 16, 256, 1024), 256, 0, st>>>(B.proposal.p, B.n, c->ws.counter.p);
+  HIPCHK(hipGetLastError());
+  int32_t cnt = 0;
+  HIPCHK(c->staging.down(c->device, st, {xfer_to(&cnt, c->ws.counter.p, sizeof(cnt))}));
+  return cnt;
+}
+
 // samples of a call (labels may be null) into the context's workspace
 void mlp_samples(hbtx_ctx *c, int64_t n, const float *X, const uint8_t *y)
 {
@@ -2595,11 +2607,11 @@ void mlp_samples(hbtx_ctx *c, int64_t n, const float *X, const uint8_t *y)
 void mlp_grad_device(hbtx_ctx *c, hbtx_mlp *M, const float *dX, const uint8_t *dy, const int32_t *idx, int64_t nb)
 {
   hipStream_t st = c->stream;
-  const int nblk = (int)((nb + MLP_BLOCK - 1) / MLP_BLOCK);
+  const int nblk = mlp_grad_blocks(nb, c->num_cu);
   M->partial.alloc((int64_t)nblk * MLP_NPAR);
   M->lossp.alloc(nblk);
   k_mlp_grad<<<nblk, MLP_BLOCK, 0, st>>>(M->wf.p, dX, dy, idx, nb, 1.f / (float)nb, M->partial.p, M->lossp.p);
-  k_mlp_reduce<<<(MLP_NPAR + 255) / 256, 256, 0, st>>>(M->partial.p, nblk, M->grad.p, M->lossp.p, M->loss.p);
+  k_mlp_reduce<<<(MLP_NPAR + HBTX_WAVE - 1) / HBTX_WAVE, 256, 0, st>>>(M->partial.p, nblk, M->grad.p, M->lossp.p, M->loss.p);
   HIPCHK(hipGetLastError());
 }
 } // namespace
@@ -2680,10 +2692,10 @@ int hbtx_mlp_gradient(hbtx_ctx *c, hbtx_mlp *M, int64_t n, const float *X, const
     auto &dy = c->ws.y;
     mlp_grad_device(c, M, dX.p, dy.p, nullptr, n);
     double l = 0.0;
+    std::vector<XferPart> parts{xfer_to(&l, M->loss.p, sizeof(double))};
     if (grad)
-      HIPCHK(hipMemcpyAsync(grad, M->grad.p, MLP_NPAR * sizeof(float), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(&l, M->loss.p, sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+      parts.push_back(xfer_to(grad, M->grad.p, MLP_NPAR * sizeof(float)));
+    HIPCHK(c->staging.down(c->device, st, parts));
     if (loss)
       *loss = l / (double)n;
   });
@@ -2866,12 +2878,7 @@ int hbtx_batch_propose(hbtx_ctx *c, hbtx_mlp *M, float threshold, int64_t min_pa
     B.has_proposal = true;
     if (nproposed)
     {
-      std::vector<uint8_t> h(n);
-      HIPCHK(hipMemcpy(h.data(), B.proposal.p, n, hipMemcpyDeviceToHost));
-      int64_t cnt = 0;
-      for (int64_t i = 0; i < n; i++)
-        cnt += h[i];
-      *nproposed = cnt;
+      *nproposed = count_proposed(c, B);
     }
   });
 }
@@ -2939,12 +2946,7 @@ int hbtx_batch_warm_proposal(hbtx_ctx *c, const hbtx_params *prm, hbtx_mlp *M, f
     }
     if (nproposed)
     {
-      std::vector<uint8_t> h(n);
-      HIPCHK(hipMemcpy(h.data(), B.proposal.p, n, hipMemcpyDeviceToHost));
-      int64_t cnt = 0;
-      for (int64_t i = 0; i < n; i++)
-        cnt += h[i];
-      *nproposed = cnt;
+      *nproposed = count_proposed(c, B);
     }
   });
 }

@@ -82,4 +82,17 @@ __global__ void k_proposal_from_logit(const float *logit, int64_t n, float cut, 
   }
 }
 
+// Number of set flags (at most 2^29).
+__global__ __launch_bounds__(256) void k_count_flags(const uint8_t *__restrict__ flag, int64_t n, int32_t *count)
+{
+  int32_t c = 0;
+  GRID_STRIDE(i, n)
+    c += flag[i] != 0;
+#pragma unroll
+  for (int d = 1; d < HBTX_WAVE; d <<= 1)
+    c += __shfl_xor(c, d, HBTX_WAVE);
+  if (lane_id() == 0 && c)
+    atomicAdd(count, c);
+}
+
 } // namespace hbtx

@@ -1,8 +1,7 @@
 // Per-particle bound-set classifier for the learned warm start: an
 // 8 -> 64 -> 64 -> 1 MLP with ReLU hidden layers and a logistic output.
 // Parameters are kept as FP32 master weights for the optimiser and rounded to
-// BF16 for every forward/backward pass (accumulation in FP32).  Weight reads are
-// wave-uniform, so they go through the scalar cache.
+// BF16 for every forward/backward pass (accumulation in FP32).
 //
 // Flat parameter layout: W1[64][8] | b1[64] | W2[64][64] | b2[64] | w3[64] | b3.
 #pragma once
@@ -19,13 +18,6 @@ namespace hbtx
 #define MLP_OFF_W3 (MLP_OFF_B2 + MLP_H)
 #define MLP_OFF_B3 (MLP_OFF_W3 + MLP_H)
 #define MLP_NPAR (MLP_OFF_B3 + 1)
-#define MLP_BLOCK 128
-
-HBTX_DEV float wload(const float *w, int i)
-{
-  typedef const __attribute__((address_space(4))) float cf;
-  return ((cf *)(uintptr_t)w)[i];
-}
 
 // round-to-nearest-even FP32 -> BF16 bits
 HBTX_HD uint16_t f32_to_bf16(float f)
@@ -164,155 +156,305 @@ inline int mlp_forward_blocks(int64_t n)
   return (int)std::max<int64_t>(1, std::min<int64_t>((groups + 3) / 4, 4096));
 }
 
-// Forward + backward of one block of MLP_BLOCK samples; writes this block's
-// gradient sum (already divided by the batch size) and loss sum.
-// sample k of the batch is row idx[k] of X (idx may be null: row k).
-__global__ __launch_bounds__(MLP_BLOCK) void k_mlp_grad(const float *__restrict__ w, const float *__restrict__ X,
-                                                        const uint8_t *__restrict__ y, const int32_t *__restrict__ idx,
-                                                        int64_t nbatch, float inv_batch, float *__restrict__ partial,
-                                                        double *__restrict__ loss_partial)
+// Forward and backward of the network on the FP32 matrix instructions
+// (v_mfma_f32_32x32x2_f32): a wave takes 32 samples at a time, neurons as matrix
+// rows and samples as columns, as k_mlp_forward does, with every product and sum
+// in FP32.
+//   H1^T[64 x 32] = W1 X^T + b1,  H2^T = W2 relu(H1^T) + b2,  dH1^T = W2^T dH2^T:
+//     a lane's accumulator rows are the K entries it supplies to the next product;
+//   dW2[64 x 64] = dH2^T[64 x 32] H1[32 x 64],  dW1 = dH1^T X:  K is the sample, so
+//     dH2, H1 and dH1 pass through the wave's own LDS to become operands.
+// The weight gradients stay in the accumulators over all of a wave's samples, and a
+// block's four waves add theirs in order at the end, so that a block leaves one
+// partial gradient.  (One sample a lane on the vector units, a partial gradient per
+// 128 samples: 1009 us for 400,000 samples, and 888 us to add 3126 partials.)
+#define MLP_TILE 32
+#define MLP_WAVES 4
+#define MLP_BLOCK (MLP_WAVES * HBTX_WAVE)
+#define MLP_LD (MLP_H + 1)
+struct MlpLds
 {
-  __shared__ float sx[MLP_BLOCK][MLP_IN];
-  __shared__ float sh1[MLP_BLOCK][MLP_H + 1];
-  __shared__ float sh2[MLP_BLOCK][MLP_H + 1]; // h2, later dh1
-  __shared__ float sdh2[MLP_BLOCK][MLP_H + 1];
-  __shared__ float sdz[MLP_BLOCK];
-  __shared__ double sloss[MLP_BLOCK];
-  const int t = threadIdx.x;
-  const int64_t k = (int64_t)blockIdx.x * MLP_BLOCK + t;
-  const bool valid = k < nbatch;
-  const int64_t row = valid ? (idx ? (int64_t)idx[k] : k) : 0;
-  float x[MLP_IN];
-#pragma unroll
-  for (int i = 0; i < MLP_IN; i++)
+  float w2[MLP_H * MLP_LD];
+  float w1[MLP_H * (MLP_IN + 1)];
+  float b1[MLP_H], b2[MLP_H], w3[MLP_H];
+  union
   {
-    x[i] = valid ? X[row * MLP_IN + i] : 0.f;
-    sx[t][i] = x[i];
+    struct
+    {
+      float d[MLP_TILE * MLP_LD]; // dH2, then dH1: [sample][neuron]
+      float h[MLP_TILE * MLP_LD]; // H1
+      float x[MLP_TILE * (MLP_IN + 1)];
+    } wave[MLP_WAVES];
+    float grad[MLP_NPAR + 3]; // the block's sum, once every sample is done
+  };
+  double loss[MLP_WAVES];
+};
+
+__global__ __launch_bounds__(MLP_BLOCK, 1) void k_mlp_grad(const float *__restrict__ w, const float *__restrict__ X,
+                                                           const uint8_t *__restrict__ y,
+                                                           const int32_t *__restrict__ idx, int64_t nbatch,
+                                                           float inv_batch, float *__restrict__ partial,
+                                                           double *__restrict__ loss_partial)
+{
+  __shared__ MlpLds L;
+  const int tid = threadIdx.x, wv = uniform(tid / HBTX_WAVE), lane = lane_id(), h = lane >> 5, c = lane & 31;
+  for (int i = tid; i < MLP_H * MLP_H; i += MLP_BLOCK)
+    L.w2[(i / MLP_H) * MLP_LD + i % MLP_H] = w[MLP_OFF_W2 + i];
+  for (int i = tid; i < MLP_H * MLP_IN; i += MLP_BLOCK)
+    L.w1[(i / MLP_IN) * (MLP_IN + 1) + i % MLP_IN] = w[MLP_OFF_W1 + i];
+  for (int i = tid; i < MLP_H; i += MLP_BLOCK)
+  {
+    L.b1[i] = w[MLP_OFF_B1 + i];
+    L.b2[i] = w[MLP_OFF_B2 + i];
+    L.w3[i] = w[MLP_OFF_W3 + i];
   }
-  float h1[MLP_H];
+  const float b3 = w[MLP_OFF_B3];
+  __syncthreads();
+  auto &T = L.wave[wv];
+  // accumulator register r of row block mb: neuron (row) 32 mb + 8 (r / 4) + 4 h + r % 4
+  auto row = [&](int mb, int r) { return 32 * mb + 8 * (r / 4) + 4 * h + (r & 3); };
+  f32x16 gw2[2][2], gw1[2];
+  float gw3[2][16], gb2[2] = {0.f, 0.f}, gb1[2] = {0.f, 0.f}, gb3 = 0.f;
+  double loss = 0.0;
 #pragma unroll
-  for (int j = 0; j < MLP_H; j++)
+  for (int mb = 0; mb < 2; mb++)
+#pragma unroll
+    for (int r = 0; r < 16; r++)
+    {
+      gw2[mb][0][r] = gw2[mb][1][r] = gw1[mb][r] = 0.f;
+      gw3[mb][r] = 0.f;
+    }
+  const int64_t ntile = (nbatch + MLP_TILE - 1) / MLP_TILE;
+  for (int64_t t = (int64_t)blockIdx.x * MLP_WAVES + wv; t < ntile; t += (int64_t)gridDim.x * MLP_WAVES)
   {
-    float a = wload(w, MLP_OFF_B1 + j);
+    const int64_t k = t * MLP_TILE + c;
+    const bool valid = k < nbatch;
+    const int64_t at = valid ? (idx ? (int64_t)idx[k] : k) : 0;
+    float x[MLP_IN];
+    {
+      const float4 u0 = reinterpret_cast<const float4 *>(X + at * MLP_IN)[0];
+      const float4 u1 = reinterpret_cast<const float4 *>(X + at * MLP_IN)[1];
+      const float xs[MLP_IN] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
 #pragma unroll
-    for (int i = 0; i < MLP_IN; i++)
-      a += wload(w, MLP_OFF_W1 + j * MLP_IN + i) * x[i];
-    h1[j] = fmaxf(a, 0.f);
-    sh1[t][j] = h1[j];
+      for (int f = 0; f < MLP_IN; f++)
+        x[f] = valid ? xs[f] : 0.f;
+    }
+    const float yy = valid ? (float)y[at] : 0.f;
+    f32x16 h1[2], h2[2];
+#pragma unroll
+    for (int mb = 0; mb < 2; mb++)
+    {
+#pragma unroll
+      for (int r = 0; r < 16; r++)
+        h1[mb][r] = L.b1[row(mb, r)];
+#pragma unroll
+      for (int s = 0; s < MLP_IN / 2; s++)
+        h1[mb] = __builtin_amdgcn_mfma_f32_32x32x2f32(L.w1[(32 * mb + c) * (MLP_IN + 1) + 2 * s + h],
+                                                      h ? x[2 * s + 1] : x[2 * s], h1[mb], 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 16; r++)
+      {
+        h1[mb][r] = fmaxf(h1[mb][r], 0.f);
+        h2[mb][r] = L.b2[row(mb, r)];
+      }
+    }
+#pragma unroll
+    for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+      for (int r = 0; r < 16; r++)
+#pragma unroll
+        for (int mb = 0; mb < 2; mb++)
+          h2[mb] = __builtin_amdgcn_mfma_f32_32x32x2f32(L.w2[(32 * mb + c) * MLP_LD + row(kb, r)], h1[kb][r], h2[mb],
+                                                        0, 0, 0);
+    float z = 0.f;
+#pragma unroll
+    for (int mb = 0; mb < 2; mb++)
+#pragma unroll
+      for (int r = 0; r < 16; r++)
+      {
+        h2[mb][r] = fmaxf(h2[mb][r], 0.f);
+        z += L.w3[row(mb, r)] * h2[mb][r];
+      }
+    z += __shfl_xor(z, 32, HBTX_WAVE);
+    z += b3;
+    const float sig = 1.f / (1.f + __expf(-z));
+    const float dz = valid ? (sig - yy) * inv_batch : 0.f;
+    // binary cross-entropy with logits: softplus(z) - y z (a sample's two lanes hold the same)
+    if (valid && h == 0)
+    {
+      loss += (double)(fmaxf(z, 0.f) + log1pf(__expf(-fabsf(z))) - yy * z);
+      gb3 += dz;
+    }
+    f32x16 d1[2];
+#pragma unroll
+    for (int mb = 0; mb < 2; mb++)
+#pragma unroll
+      for (int r = 0; r < 16; r++)
+      {
+        const int j = row(mb, r);
+        gw3[mb][r] += dz * h2[mb][r];
+        h2[mb][r] = (h2[mb][r] > 0.f) ? dz * L.w3[j] : 0.f; // dH2 from here on
+        d1[mb][r] = 0.f;
+        T.d[c * MLP_LD + j] = h2[mb][r];
+        T.h[c * MLP_LD + j] = h1[mb][r];
+      }
+    if (h == 0)
+#pragma unroll
+      for (int f = 0; f < MLP_IN; f++)
+        T.x[c * (MLP_IN + 1) + f] = x[f];
+#pragma unroll
+    for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+      for (int r = 0; r < 16; r++)
+#pragma unroll
+        for (int mb = 0; mb < 2; mb++)
+          d1[mb] = __builtin_amdgcn_mfma_f32_32x32x2f32(L.w2[row(kb, r) * MLP_LD + 32 * mb + c], h2[kb][r], d1[mb],
+                                                        0, 0, 0);
+    wave_lds_sync();
+#pragma unroll
+    for (int s2 = 0; s2 < MLP_TILE / 2; s2++)
+    {
+      const int s = 2 * s2 + h;
+      const float a0 = T.d[s * MLP_LD + c], a1 = T.d[s * MLP_LD + 32 + c];
+      const float e0 = T.h[s * MLP_LD + c], e1 = T.h[s * MLP_LD + 32 + c];
+      gb2[0] += a0;
+      gb2[1] += a1;
+      gw2[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, e0, gw2[0][0], 0, 0, 0);
+      gw2[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, e1, gw2[0][1], 0, 0, 0);
+      gw2[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, e0, gw2[1][0], 0, 0, 0);
+      gw2[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, e1, gw2[1][1], 0, 0, 0);
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int mb = 0; mb < 2; mb++)
+#pragma unroll
+      for (int r = 0; r < 16; r++)
+        T.d[c * MLP_LD + row(mb, r)] = (h1[mb][r] > 0.f) ? d1[mb][r] : 0.f;
+    wave_lds_sync();
+#pragma unroll
+    for (int s2 = 0; s2 < MLP_TILE / 2; s2++)
+    {
+      const int s = 2 * s2 + h;
+      const float a0 = T.d[s * MLP_LD + c], a1 = T.d[s * MLP_LD + 32 + c];
+      const float e = (c < MLP_IN) ? T.x[s * (MLP_IN + 1) + min(c, MLP_IN)] : 0.f;
+      gb1[0] += a0;
+      gb1[1] += a1;
+      gw1[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, e, gw1[0], 0, 0, 0);
+      gw1[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, e, gw1[1], 0, 0, 0);
+    }
+    wave_lds_sync(); // the next samples' rows go where these were read
   }
-  float z = wload(w, MLP_OFF_B3);
-  for (int j = 0; j < MLP_H; j++)
-  {
-    float a = wload(w, MLP_OFF_B2 + j);
+  // sums over the lanes that share a value
 #pragma unroll
-    for (int i = 0; i < MLP_H; i++)
-      a += wload(w, MLP_OFF_W2 + j * MLP_H + i) * h1[i];
-    const float h2 = fmaxf(a, 0.f);
-    sh2[t][j] = h2;
-    z += wload(w, MLP_OFF_W3 + j) * h2;
+  for (int mb = 0; mb < 2; mb++)
+  {
+    gb2[mb] += __shfl_xor(gb2[mb], 32, HBTX_WAVE);
+    gb1[mb] += __shfl_xor(gb1[mb], 32, HBTX_WAVE);
+#pragma unroll
+    for (int r = 0; r < 16; r++)
+#pragma unroll
+      for (int d = 1; d < 32; d <<= 1)
+        gw3[mb][r] += __shfl_xor(gw3[mb][r], d, HBTX_WAVE);
   }
-  const float yy = valid ? (float)y[row] : 0.f;
-  const float sig = 1.f / (1.f + __expf(-z));
-  const float dz = valid ? (sig - yy) * inv_batch : 0.f;
-  sdz[t] = dz;
-  // binary cross-entropy with logits: softplus(z) - y z
-  sloss[t] = valid ? (double)(fmaxf(z, 0.f) + log1pf(__expf(-fabsf(z))) - yy * z) : 0.0;
-  float dh1[MLP_H];
 #pragma unroll
-  for (int i = 0; i < MLP_H; i++)
-    dh1[i] = 0.f;
-  for (int j = 0; j < MLP_H; j++)
+  for (int d = 1; d < HBTX_WAVE; d <<= 1)
   {
-    const float d2 = (sh2[t][j] > 0.f) ? dz * wload(w, MLP_OFF_W3 + j) : 0.f;
-    sdh2[t][j] = d2;
+    gb3 += __shfl_xor(gb3, d, HBTX_WAVE);
+    loss += __shfl_xor(loss, d, HBTX_WAVE);
+  }
+  if (lane == 0)
+    L.loss[wv] = loss;
+  __syncthreads(); // (the waves' tiles are done: their LDS becomes the block's sum)
+  for (int q = tid; q < MLP_NPAR; q += MLP_BLOCK)
+    L.grad[q] = 0.f;
+  for (int k = 0; k < MLP_WAVES; k++)
+  {
+    __syncthreads();
+    if (wv != k)
+      continue;
 #pragma unroll
-    for (int i = 0; i < MLP_H; i++)
-      dh1[i] += wload(w, MLP_OFF_W2 + j * MLP_H + i) * d2;
+    for (int mb = 0; mb < 2; mb++)
+    {
+#pragma unroll
+      for (int r = 0; r < 16; r++)
+      {
+        const int j = row(mb, r);
+        L.grad[MLP_OFF_W2 + j * MLP_H + c] += gw2[mb][0][r];
+        L.grad[MLP_OFF_W2 + j * MLP_H + 32 + c] += gw2[mb][1][r];
+        if (c < MLP_IN)
+          L.grad[MLP_OFF_W1 + j * MLP_IN + c] += gw1[mb][r];
+        if (c == 0)
+          L.grad[MLP_OFF_W3 + j] += gw3[mb][r];
+      }
+      if (h == 0)
+      {
+        L.grad[MLP_OFF_B2 + 32 * mb + c] += gb2[mb];
+        L.grad[MLP_OFF_B1 + 32 * mb + c] += gb1[mb];
+      }
+    }
+    if (lane == 0)
+      L.grad[MLP_OFF_B3] += gb3;
   }
   __syncthreads();
-  float *out = partial + (int64_t)blockIdx.x * MLP_NPAR;
-  // output layer and second hidden layer: sums over the block's samples
-  for (int q = t; q < MLP_H * MLP_H + 2 * MLP_H + 1; q += MLP_BLOCK)
-  {
-    float acc = 0.f;
-    if (q < MLP_H * MLP_H)
-    {
-      const int j = q / MLP_H, i = q % MLP_H;
-      for (int s = 0; s < MLP_BLOCK; s++)
-        acc += sdh2[s][j] * sh1[s][i];
-      out[MLP_OFF_W2 + q] = acc;
-    }
-    else if (q < MLP_H * MLP_H + MLP_H)
-    {
-      const int j = q - MLP_H * MLP_H;
-      for (int s = 0; s < MLP_BLOCK; s++)
-        acc += sdh2[s][j];
-      out[MLP_OFF_B2 + j] = acc;
-    }
-    else if (q < MLP_H * MLP_H + 2 * MLP_H)
-    {
-      const int j = q - MLP_H * MLP_H - MLP_H;
-      for (int s = 0; s < MLP_BLOCK; s++)
-        acc += sdz[s] * sh2[s][j];
-      out[MLP_OFF_W3 + j] = acc;
-    }
-    else
-    {
-      for (int s = 0; s < MLP_BLOCK; s++)
-        acc += sdz[s];
-      out[MLP_OFF_B3] = acc;
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < MLP_H; i++)
-    sh2[t][i] = (h1[i] > 0.f) ? dh1[i] : 0.f;
-  __syncthreads();
-  for (int q = t; q < MLP_H * MLP_IN + MLP_H; q += MLP_BLOCK)
-  {
-    float acc = 0.f;
-    if (q < MLP_H * MLP_IN)
-    {
-      const int j = q / MLP_IN, i = q % MLP_IN;
-      for (int s = 0; s < MLP_BLOCK; s++)
-        acc += sh2[s][j] * sx[s][i];
-      out[MLP_OFF_W1 + q] = acc;
-    }
-    else
-    {
-      const int j = q - MLP_H * MLP_IN;
-      for (int s = 0; s < MLP_BLOCK; s++)
-        acc += sh2[s][j];
-      out[MLP_OFF_B1 + j] = acc;
-    }
-  }
-  if (t == 0)
+  for (int q = tid; q < MLP_NPAR; q += MLP_BLOCK)
+    partial[(int64_t)blockIdx.x * MLP_NPAR + q] = L.grad[q];
+  if (tid == 0)
   {
     double l = 0.0;
-    for (int s = 0; s < MLP_BLOCK; s++)
-      l += sloss[s];
+    for (int k = 0; k < MLP_WAVES; k++)
+      l += L.loss[k];
     loss_partial[blockIdx.x] = l;
   }
 }
 
-// Sum of the block partials (fixed order, deterministic).
-__global__ void k_mlp_reduce(const float *__restrict__ partial, int nblocks, float *__restrict__ grad,
-                             const double *__restrict__ loss_partial, double *__restrict__ loss)
+// Blocks of the gradient: one a CU, no more than there are samples for.
+inline int mlp_grad_blocks(int64_t nbatch, int num_cu)
 {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t tiles = (nbatch + MLP_TILE - 1) / MLP_TILE;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(num_cu, (tiles + MLP_WAVES - 1) / MLP_WAVES));
+}
+
+// Sum of the block partials in a fixed order: a block takes 64 parameters, each of
+// its four waves a quarter of the partials, eight loads at a time.
+__global__ __launch_bounds__(256) void k_mlp_reduce(const float *__restrict__ partial, int nblocks,
+                                                    float *__restrict__ grad, const double *__restrict__ loss_partial,
+                                                    double *__restrict__ loss)
+{
+  __shared__ float part[4][HBTX_WAVE];
+  const int g = threadIdx.x / HBTX_WAVE, lane = lane_id();
+  const int q = blockIdx.x * HBTX_WAVE + lane;
+  const int b0 = nblocks * g / 4, b1 = nblocks * (g + 1) / 4;
+  float acc = 0.f;
   if (q < MLP_NPAR)
   {
-    float acc = 0.f;
-    for (int b = 0; b < nblocks; b++)
+    int b = b0;
+    for (; b + 8 <= b1; b += 8)
+    {
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++)
+        v[k] = partial[(int64_t)(b + k) * MLP_NPAR + q];
+#pragma unroll
+      for (int k = 0; k < 8; k++)
+        acc += v[k];
+    }
+    for (; b < b1; b++)
       acc += partial[(int64_t)b * MLP_NPAR + q];
-    grad[q] = acc;
   }
-  if (q == 0)
+  part[g][lane] = acc;
+  __syncthreads();
+  if (g == 0 && q < MLP_NPAR)
+    grad[q] = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+  if (blockIdx.x == 0 && g == 1)
   {
     double l = 0.0;
-    for (int b = 0; b < nblocks; b++)
+    for (int b = lane; b < nblocks; b += HBTX_WAVE)
       l += loss_partial[b];
-    *loss = l;
+#pragma unroll
+    for (int d = 1; d < HBTX_WAVE; d <<= 1)
+      l += __shfl_xor(l, d, HBTX_WAVE);
+    if (lane == 0)
+      *loss = l;
   }
 }
 

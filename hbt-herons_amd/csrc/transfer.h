@@ -51,12 +51,31 @@ inline XferPart xfer_to(void *dst, const void *dev, size_t bytes)
           [dst](char *slot, size_t off, size_t len) { std::memcpy((char *)dst + off, slot, len); }};
 }
 
+// Small transfers as one kernel that reads or writes the pinned slot itself over the
+// link (a copy of its own costs about 11 us, and waiting for it as much again).
+struct XferSmall
+{
+  static constexpr int MAX_PARTS = 6;
+  static constexpr size_t MAX_BYTES = 128 << 10;
+  int nparts;
+  uint32_t *dst[MAX_PARTS];
+  const uint32_t *src[MAX_PARTS];
+  uint32_t words[MAX_PARTS];
+};
+__global__ void k_xfer_small(XferSmall X)
+{
+  for (int k = 0; k < X.nparts; k++)
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < X.words[k]; i += gridDim.x * blockDim.x)
+      X.dst[k][i] = X.src[k][i];
+}
+
 // The pinned slots of one context, made at the first transfer and released with the
 // context.  One transfer at a time (a context serves one host thread).
 struct Staging
 {
   char *pinned = nullptr;
   hipEvent_t ev[XFER_SLOTS] = {};
+  unsigned small_slot = 0;
 
   hipError_t init()
   {
@@ -124,6 +143,23 @@ struct Staging
     if (e0 != hipSuccess || parts.empty())
       return e0;
     const size_t total = parts.back().at + parts.back().bytes;
+    if (total <= XferSmall::MAX_BYTES)
+    {
+      const int s = small_slot++ % XFER_SLOTS;
+      hipError_t e = hipEventSynchronize(ev[s]);
+      if (e != hipSuccess)
+        return e;
+      for (const XferPart &p : parts)
+        p.host(slot(s) + p.at, 0, p.bytes);
+      XferSmall X;
+      X.nparts = 1;
+      X.dst[0] = (uint32_t *)dev;
+      X.src[0] = (const uint32_t *)slot(s);
+      X.words[0] = (uint32_t)((total + 3) / 4); // (device blocks are whole words long)
+      k_xfer_small<<<std::max(1u, (X.words[0] + 1023) / 1024), 256, 0, stream>>>(X);
+      e = hipGetLastError();
+      return (e == hipSuccess) ? hipEventRecord(ev[s], stream) : e;
+    }
     const size_t nc = (total + XFER_CHUNK - 1) / XFER_CHUNK;
     const int nt = threads_for(total, nc);
     std::atomic<size_t> next{0};
@@ -180,6 +216,34 @@ struct Staging
         chunks.push_back({&p, o, std::min(XFER_CHUNK, p.bytes - o)});
         total += chunks.back().len;
       }
+    bool words = parts.size() <= XferSmall::MAX_PARTS;
+    for (const XferPart &p : parts)
+      words = words && (p.bytes & 3) == 0;
+    if (total <= XferSmall::MAX_BYTES && words)
+    {
+      const int s = small_slot++ % XFER_SLOTS;
+      hipError_t e = hipEventSynchronize(ev[s]);
+      if (e != hipSuccess)
+        return e;
+      XferSmall X;
+      X.nparts = (int)parts.size();
+      size_t at = 0;
+      for (int k = 0; k < X.nparts; k++)
+      {
+        X.dst[k] = (uint32_t *)(slot(s) + at);
+        X.src[k] = (const uint32_t *)parts[k].dev;
+        X.words[k] = (uint32_t)(parts[k].bytes / 4);
+        at += parts[k].bytes;
+      }
+      k_xfer_small<<<std::max<size_t>(1, (total + 4095) / 4096), 256, 0, stream>>>(X);
+      e = hipGetLastError();
+      if (e == hipSuccess)
+        e = hipStreamSynchronize(stream);
+      if (e == hipSuccess)
+        for (int k = 0; k < X.nparts; k++)
+          parts[k].host((char *)X.dst[k], 0, parts[k].bytes);
+      return e;
+    }
     const size_t nc = chunks.size();
     const int nt = threads_for(total, nc);
     std::atomic<size_t> next{0};

@@ -153,17 +153,6 @@ HBTX_DEV void fma_neg_on(uint64_t m, float &acc, float a, float b)
                : "scc");
 }
 
-// Orders one wave's LDS writes before its later LDS reads by other lanes: the
-// LDS serves a wave's instructions in order, so only the compiler's reordering
-// has to be held back (no workgroup barrier: the waves of a walk workgroup are
-// independent).
-HBTX_DEV void wave_lds_sync()
-{
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 struct WalkLds
 {
   int4 stk[WSTACK_CAP];  // (record offset, chain end, reached mask low, high word)
