@@ -354,12 +354,21 @@ __global__ __launch_bounds__(MOM_GROUP) void k_moments_groups(TreeArgs A, const 
       ws[threadIdx.x] = -1;
     __syncthreads();
     const int64_t u = g * MOM_GROUP + threadIdx.x;
+    // this unit's cells and their ends, all depths' loads in flight together
+    int cell[MOM_SLOTS], cend[MOM_SLOTS];
+#pragma unroll
+    for (int d = 0; d < MOM_SLOTS; d++)
+      cell[d] = (u < nunits) ? slots_in[u * MOM_SLOTS + d] : -1;
+#pragma unroll
+    for (int d = 0; d < MOM_SLOTS; d++)
+      cend[d] = A.eskip[max(cell[d], 0)];
+#pragma unroll
     for (int d = MOM_SLOTS - 1; d >= 0; d--)
     {
-      const int q = (u < nunits) ? slots_in[u * MOM_SLOTS + d] : -1;
+      const int q = cell[d];
       if (q >= 0)
       {
-        const int end = min(A.eskip[q], E);
+        const int end = min(cend[d], E);
         if (end > gend)
           ws[d] = q;
         else

@@ -691,6 +691,39 @@ __global__ void k_warm_keys(SubArrays S, PartArrays Q, int64_t n, uint64_t *keys
 #define RED_TILE 4096
 #define RED_NV 20
 
+// lane i's partner of a downward shuffle by D (correct in the lanes that hold a
+// partial sum at that step: the lower D)
+template <int D>
+HBTX_DEV uint32_t lane_down(uint32_t v)
+{
+  if constexpr (D == 32)
+    return __builtin_amdgcn_permlane32_swap(v, v, false, false)[1];
+  else if constexpr (D == 16)
+    return __builtin_amdgcn_permlane16_swap(v, v, false, false)[1];
+  else
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x100 + D, 0xf, 0xf, true); // row_shl:D
+}
+template <int D>
+HBTX_DEV double lane_down(double x)
+{
+  const uint64_t u = __builtin_bit_cast(uint64_t, x);
+  const uint64_t lo = lane_down<D>((uint32_t)u), hi = lane_down<D>((uint32_t)(u >> 32));
+  return __builtin_bit_cast(double, lo | (hi << 32));
+}
+// The wave's sum in lane 0: the halves, then halves of the halves, as six downward
+// shuffles add them, by moves of the vector unit (an LDS shuffle a word and step
+// made the frames' reductions LDS-bound).
+HBTX_DEV double wave_sum_down(double x)
+{
+  x += lane_down<32>(x);
+  x += lane_down<16>(x);
+  x += lane_down<8>(x);
+  x += lane_down<4>(x);
+  x += lane_down<2>(x);
+  x += lane_down<1>(x);
+  return x;
+}
+
 // Sum the first NV of the RED_NV values over a 256-thread block (thread 0 gets
 // the totals, in wave order).  A wave whose lanes saw no element of the tile
 // holds zeros: it skips the shuffles, since its sum is zero.
@@ -702,11 +735,7 @@ HBTX_DEV void block_reduce_vec(double v[RED_NV], double *lds /* [RED_THREADS/64]
 #pragma unroll
     for (int k = 0; k < NV; k++)
     {
-      double x = v[k];
-#pragma unroll
-      for (int d = 32; d >= 1; d >>= 1)
-        x += __shfl_down(x, d, HBTX_WAVE);
-      v[k] = x;
+      v[k] = wave_sum_down(v[k]);
     }
   }
   const int w = threadIdx.x / HBTX_WAVE;
@@ -756,11 +785,7 @@ HBTX_DEV void wave_reduce_tile(int b, int e, double tot[RED_NV], Acc acc)
 #pragma unroll
     for (int k = 0; k < NV; k++)
     {
-      double x = v[k];
-#pragma unroll
-      for (int d = 32; d >= 1; d >>= 1)
-        x += __shfl_down(x, d, HBTX_WAVE);
-      tot[k] += x;
+      tot[k] += wave_sum_down(v[k]);
     }
   }
 }
@@ -1135,9 +1160,7 @@ __global__ void k_core_wave(SubArrays S, PartArrays Q, DevParams P, const int32_
   }
   for (int k = 0; k < 13; k++)
   {
-    double x = v[k];
-    for (int d = 32; d >= 1; d >>= 1)
-      x += __shfl_down(x, d, HBTX_WAVE);
+    const double x = wave_sum_down(v[k]);
     if (lane_id() == 0)
       out[(int64_t)RED_NV * s + k] = x;
   }
