@@ -147,6 +147,12 @@ HBTX_DEV void wave_lds_sync()
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Set bits of the wave-uniform mask m below this lane, plus add.
+HBTX_DEV int mask_rank(uint64_t m, int add)
+{
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, add));
+}
+
 HBTX_DEV uint64_t lanemask_lt()
 {
   const int l = lane_id();

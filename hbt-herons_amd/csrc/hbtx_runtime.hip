@@ -396,7 +396,8 @@ const int32_t *list_tiles(hbtx_ctx *c, const R &r, int32_t ns, int tile, int ove
 
 // Radix tiles of a segmented sort over n elements in nseg segments: a segment
 // longer than SORT_SMALL_MAX takes ceil(len / SORT_TILE) <= len / SORT_TILE + 1
-// tiles, and at most n / (SORT_SMALL_MAX + 1) segments are that long.
+// tiles, and at most n / (SORT_SMALL_MAX + 1) segments are that long.  (The block sort
+// takes one tile a segment, so the same bound holds.)
 int64_t sort_tile_bound(int64_t n, int64_t nseg)
 {
   return n / SORT_TILE + std::min<int64_t>(nseg, n / (SORT_SMALL_MAX + 1)) + 2;
@@ -422,10 +423,15 @@ void seg_sort(hbtx_ctx *c, uint64_t *keys, int32_t *vals, int32_t nseg, const R 
               int32_t *seg_len, int64_t n_cap, int key_bits, int64_t max_len = INT64_MAX)
 {
   reserve_sort(c, n_cap, nseg);
-  const bool radix = max_len > SORT_SMALL_MAX;
-  if (radix)
-    list_tiles(c, r, nseg, SORT_TILE, SORT_SMALL_MAX, false, c->sort_ntile.p, c->sort_toff.p, c->sort_tiles.p, seg_begin,
-               seg_len);
+  // Above SORT_SMALL_MAX: a workgroup a segment where no segment is beyond one (a single
+  // 12,000: 67 us, against 115 us in 32 launches through the tiled passes), else tiled
+  // passes for all of them (with a larger segment's passes to be launched in any case,
+  // those of 2,049 to 16,384 ride along: three sorts of 8e6 slots 960 us, and 1,160 with the
+  // shorter segments in a workgroup each).
+  const bool radix = max_len > SORT_BLOCK_MAX, block = !radix && max_len > SORT_SMALL_MAX;
+  if (radix || block)
+    list_tiles(c, r, nseg, radix ? SORT_TILE : SORT_BLOCK_MAX, SORT_SMALL_MAX, false, c->sort_ntile.p, c->sort_toff.p,
+               c->sort_tiles.p, seg_begin, seg_len);
   else
     k_list_counts<<<blocks_for(nseg, 256, 1 << 24), 256, 0, c->stream>>>(r, nseg, SORT_TILE, SORT_SMALL_MAX,
                                                                          (int32_t *)nullptr, seg_begin, seg_len);
@@ -438,10 +444,14 @@ void seg_sort(hbtx_ctx *c, uint64_t *keys, int32_t *vals, int32_t nseg, const R 
     k_sort_small<<<std::max(1, std::min(nseg, 16384)), SORT_THREADS, 0, c->stream>>>(keys, vals, seg_begin, seg_len,
                                                                                       nseg);
   HIPCHK(hipGetLastError());
-  if (!radix)
-    return;
   const int32_t *ntiles_p = c->sort_toff.p + nseg;
   const int64_t maxt = sort_tile_bound(n_cap, nseg);
+  if (block)
+    k_sort_block<<<(int)std::min<int64_t>(maxt, c->num_cu), SORT_BLOCK_THREADS, sizeof(SortBlockLds), c->stream>>>(
+        keys, vals, c->sort_tiles.p, ntiles_p, key_bits);
+  HIPCHK(hipGetLastError());
+  if (!radix)
+    return;
   const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(maxt, 4 * c->num_cu));
   // an even number of passes leaves the result in place; 9-bit digits where they save passes
   auto even_passes = [&](int rb) {
@@ -927,7 +937,7 @@ void build_sources_tree(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, cons
   }
   // (buffers that hold the largest trees the view can make need no count; a captured
   // round, which cannot wait for one, always has them)
-  k_tree_emit<<<blocks_for(n, 256, 8 * 1024), 256, 0, st>>>(T);
+  k_tree_emit<<<blocks_for(n, EMIT_TILE, 8 * 1024), EMIT_TILE, 0, st>>>(T);
   k_sub_entries<<<gs, 256, 0, st>>>(V.S, B.cscan.p, B.ent_cap, B.misc.p + 2);
   k_entry_total<<<1, 1, 0, st>>>(s_total, B.cscan.p, B.misc.p + 3, B.ent_cap, B.misc.p + 2);
   // moments bottom-up: LDS-staged windows, then one pass per level of window
@@ -1885,6 +1895,9 @@ int hbtx_create(hbtx_ctx **out, int device)
     HIPCHK(hipGetDeviceProperties(&prop, device));
     c->num_cu = std::max(1, prop.multiProcessorCount);
     c->scratch = scratch_address(device);
+    // (more than the 64 KiB a kernel gets unasked)
+    HIPCHK(hipFuncSetAttribute((const void *)k_sort_block, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)sizeof(SortBlockLds)));
     load_tuning(c);
     HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     HIPCHK(hipEventCreate(&c->ev0));

@@ -2,7 +2,9 @@
 //  * segments of <= SORT_WAVE_MAX elements: one wave each, bitonic sort in lanes;
 //  * segments of <= SORT_SMALL_MAX elements: one workgroup each, the same bitonic
 //    network in LDS;
-//  * larger segments: tiled LSD radix sort (8- or 9-bit digits, whichever needs
+//  * where no segment is longer than SORT_BLOCK_MAX, those above: one workgroup each, a
+//    stable LSD radix sort whose passes stay in registers and LDS (the order of the next);
+//  * else the segments above SORT_SMALL_MAX: tiled LSD radix sort (8- or 9-bit digits, whichever needs
 //    fewer passes) where every tile of SORT_TILE elements ranks its keys stably
 //    with wave ballots (match of the digit bits) and LDS per-digit counters, so
 //    all large segments advance together in one launch per pass.
@@ -22,6 +24,9 @@ namespace hbtx
 #define SORT_TILE 2048
 #endif
 #define RADIX_MAX_BINS 512 // (9-bit digits)
+#define SORT_BLOCK_THREADS 1024
+#define SORT_BLOCK_ITEMS 16
+#define SORT_BLOCK_MAX (SORT_BLOCK_THREADS * SORT_BLOCK_ITEMS)
 
 __global__ __launch_bounds__(SORT_THREADS) void k_sort_small(uint64_t *__restrict__ keys, int32_t *__restrict__ vals,
                                                             const int32_t *__restrict__ seg_begin,
@@ -203,6 +208,241 @@ __global__ __launch_bounds__(SORT_THREADS) void k_sort_wave4(uint64_t *__restric
         vals[b + e] = val[r];
       }
     }
+  }
+}
+
+// Segments of SORT_SMALL_MAX + 1 .. SORT_BLOCK_MAX elements (tiles: one a segment), one
+// workgroup each, by stable 8-bit LSD passes over (32 key bits, place in the segment)
+// in registers: wave w owns elements [64 R w, 64 R (w + 1)), R = ceil(n / 1024), ranks
+// them by ballot match against its own digit counters, and they change places through
+// LDS.  A pass in which every key has the same digit moves nothing.  The keys' top 32
+// bits come first; an element among equals of those (a few in 12,000 with spatial
+// keys) then counts the members of its run that go before it by the bits below.  A run
+// of more than SORT_RUN_MAX sends the segment through the passes of the lower bits
+// first, then the upper ones.
+// Bound: the match (8 ballots an element) and the LDS on the one CU of the segment,
+// some 12 us a pass.  A segment of 12,000, 63 bits: 67 us; through the tiled passes (four
+// launches of 2 to 12 us a pass) 115 us; eight passes with key and value in registers
+// and LDS 93 us.
+#define SORT_RUN_MAX 32
+struct SortBlockLds
+{
+  uint64_t x[SORT_BLOCK_MAX];                        // the elements in passage
+  uint16_t cnt[SORT_BLOCK_THREADS / HBTX_WAVE][256]; // per wave and digit (at most 1024), then its base
+  int32_t base[256];
+  int32_t scan[4];
+  int32_t same, long_run;
+};
+
+// The lanes whose digit (bits [shift, shift + 8) of v) is this lane's.
+HBTX_DEV uint64_t match_digit(uint32_t v, int shift)
+{
+  uint32_t lo = ~0u, hi = ~0u;
+#pragma unroll
+  for (int bit = 0; bit < 8; bit++)
+  {
+    const int32_t on = __builtin_amdgcn_sbfe((int32_t)v, shift + bit, 1); // 0 or -1
+    const uint64_t bb = __builtin_amdgcn_sicmp(on, 0, 33 /* ne */);
+    lo &= ~((uint32_t)bb ^ (uint32_t)on);
+    hi &= ~((uint32_t)(bb >> 32) ^ (uint32_t)on);
+  }
+  return ((uint64_t)hi << 32) | lo;
+}
+
+__global__ __launch_bounds__(SORT_BLOCK_THREADS) void k_sort_block(uint64_t *__restrict__ keys,
+                                                                  int32_t *__restrict__ vals,
+                                                                  const int4 *__restrict__ tiles,
+                                                                  const int32_t *__restrict__ ntiles_p, int key_bits)
+{
+  extern __shared__ __align__(16) unsigned char sort_lds[];
+  SortBlockLds &L = *reinterpret_cast<SortBlockLds *>(sort_lds);
+  constexpr int NW = SORT_BLOCK_THREADS / HBTX_WAVE;
+  const int tid = threadIdx.x, w = uniform(tid / HBTX_WAVE), lane = lane_id();
+  const int low_bits = max(0, key_bits - 32), top_bits = key_bits - low_bits;
+  const uint64_t low_mask = (1ull << low_bits) - 1ull;
+  const int nt = *ntiles_p;
+  for (int t = blockIdx.x; t < nt; t += gridDim.x)
+  {
+    const int4 tl = tiles[t];
+    const int b = tl.y, n = tl.z - tl.y;
+    // R rows of a wave's lanes; the places past n hold the largest key, which no pass
+    // moves off the end
+    const int R = (n + SORT_BLOCK_THREADS - 1) / SORT_BLOCK_THREADS;
+    const int i0 = w * R * HBTX_WAVE + lane; // this thread's places: i0 + 64 r, r < R
+    uint64_t el[SORT_BLOCK_ITEMS];           // key bits above, the element's place at the start below
+    int32_t pos[SORT_BLOCK_ITEMS];
+    auto passes = [&](int bits) {
+      for (int shift = 0; shift < bits; shift += 8)
+      {
+        for (int i = tid; i < NW * 256 / 2; i += SORT_BLOCK_THREADS)
+          reinterpret_cast<uint32_t *>(&L.cnt[0][0])[i] = 0u;
+        if (tid == 0)
+          L.same = 0;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < SORT_BLOCK_ITEMS; r++)
+        {
+          if (r >= R)
+            break;
+          const uint32_t v = (uint32_t)(el[r] >> 32);
+          const int d = (int)((v >> shift) & 255u);
+          const uint64_t m = match_digit(v, shift);
+          const int before = (int)L.cnt[w][d];
+          pos[r] = before + mask_rank(m, 0);
+          // (the wave's LDS accesses are in order: the read above comes before this write)
+          if ((m >> lane) == 1ull)
+            L.cnt[w][d] = (uint16_t)(pos[r] + 1);
+        }
+        __syncthreads();
+        if (tid < 256)
+        {
+          // digit tid: the waves' bases among its elements, then the digits' own
+          int run = 0;
+#pragma unroll
+          for (int k = 0; k < NW; k++)
+          {
+            const int c = L.cnt[k][tid];
+            L.cnt[k][tid] = (uint16_t)run;
+            run += c;
+          }
+          if (run - (tid == 255 ? R * SORT_BLOCK_THREADS - n : 0) == n)
+            L.same = 1;
+          const int incl = wave_incl_scan(run);
+          if (lane == HBTX_WAVE - 1)
+            L.scan[w] = incl;
+          L.base[tid] = incl - run;
+        }
+        __syncthreads();
+        if (L.same)
+        {
+          __syncthreads(); // every thread has read it before the next pass clears it
+          continue;
+        }
+        if (tid < 256)
+        {
+          int off = L.base[tid];
+#pragma unroll
+          for (int k = 0; k < 3; k++)
+            off += (tid >= 64 * (k + 1)) ? L.scan[k] : 0;
+          L.base[tid] = off;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < SORT_BLOCK_ITEMS; r++)
+        {
+          if (r >= R)
+            break;
+          const int d = (int)((uint32_t)(el[r] >> 32) >> shift & 255u);
+          L.x[L.base[d] + (int)L.cnt[w][d] + pos[r]] = el[r];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < SORT_BLOCK_ITEMS; r++)
+        {
+          if (r >= R)
+            break;
+          el[r] = L.x[i0 + HBTX_WAVE * r];
+        }
+        // (the next pass writes x only after its own barriers)
+      }
+    };
+    bool low_first = false;
+    for (;;)
+    {
+#pragma unroll
+      for (int r = 0; r < SORT_BLOCK_ITEMS; r++)
+      {
+        if (r >= R)
+          break;
+        const int i = i0 + HBTX_WAVE * r;
+        const uint64_t k = keys[b + min(i, n - 1)];
+        const uint32_t part = (uint32_t)(low_first ? k & low_mask : k >> low_bits);
+        el[r] = ((uint64_t)(i < n ? part : 0xffffffffu) << 32) | (uint32_t)i;
+      }
+      if (low_first)
+      {
+        passes(low_bits);
+#pragma unroll
+        for (int r = 0; r < SORT_BLOCK_ITEMS; r++)
+        {
+          if (r >= R)
+            break;
+          const int i = (int)(uint32_t)el[r];
+          const uint32_t part = (uint32_t)(keys[b + min(i, n - 1)] >> low_bits);
+          el[r] = ((uint64_t)(i < n ? part : 0xffffffffu) << 32) | (uint32_t)i;
+        }
+      }
+      passes(top_bits);
+      // the elements' places among equals of the top bits
+#pragma unroll
+      for (int r = 0; r < SORT_BLOCK_ITEMS; r++)
+        pos[r] = i0 + HBTX_WAVE * r;
+      if (low_bits == 0 || low_first)
+        break;
+      if (tid == 0)
+        L.long_run = 0;
+#pragma unroll
+      for (int r = 0; r < SORT_BLOCK_ITEMS; r++)
+      {
+        if (r >= R)
+          break;
+        L.x[pos[r]] = el[r]; // (again: passes that moved nothing left it as it was)
+      }
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < SORT_BLOCK_ITEMS; r++)
+      {
+        if (r >= R)
+          break;
+        const int i = i0 + HBTX_WAVE * r;
+        const uint32_t top = (uint32_t)(el[r] >> 32);
+        int a = i, e = i + 1; // the run
+        while (a > 0 && i - a < SORT_RUN_MAX && (uint32_t)(L.x[a - 1] >> 32) == top)
+          a--;
+        while (e < n && e - i < SORT_RUN_MAX && (uint32_t)(L.x[e] >> 32) == top)
+          e++;
+        if (e - a == 1 || i >= n)
+          continue;
+        if (e - a > SORT_RUN_MAX)
+        {
+          L.long_run = 1;
+          continue;
+        }
+        const uint64_t low = keys[b + (int)(uint32_t)el[r]] & low_mask;
+        int to = a;
+        for (int j = a; j < e; j++)
+        {
+          const uint64_t lj = keys[b + (int)(uint32_t)L.x[j]] & low_mask;
+          to += (lj < low || (lj == low && j < i)) ? 1 : 0;
+        }
+        pos[r] = to;
+      }
+      __syncthreads();
+      if (!L.long_run)
+        break;
+      low_first = true;
+      __syncthreads(); // every thread has read it before anything below is written
+    }
+    int32_t val[SORT_BLOCK_ITEMS];
+#pragma unroll
+    for (int r = 0; r < SORT_BLOCK_ITEMS; r++)
+    {
+      if (r >= R)
+        break;
+      const int i = b + min((int)(uint32_t)el[r], n - 1);
+      el[r] = keys[i];
+      val[r] = vals[i];
+    }
+    __syncthreads(); // every key and value has been read
+#pragma unroll
+    for (int r = 0; r < SORT_BLOCK_ITEMS; r++)
+    {
+      if (r >= R || i0 + HBTX_WAVE * r >= n)
+        break;
+      keys[b + pos[r]] = el[r];
+      vals[b + pos[r]] = val[r];
+    }
+    __syncthreads();
   }
 }
 
