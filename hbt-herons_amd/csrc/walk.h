@@ -153,12 +153,32 @@ HBTX_DEV void fma_neg_on(uint64_t m, float &acc, float a, float b)
                : "scc");
 }
 
+// acc -= m[k] * q[k] for k = 0..3 in order, each on the lanes of its wave-uniform
+// mask only (a subset of exec): the sums of four records without a vector select, the
+// exec mask saved and restored once.
+HBTX_DEV void fma_neg_on4(const uint64_t on[4], float &acc, const float m[4], const float q[4])
+{
+  uint64_t save;
+  asm volatile("s_mov_b64 %1, exec\n\t"
+               "s_mov_b64 exec, %10\n\t"
+               "v_fma_f32 %0, -%2, %6, %0\n\t"
+               "s_mov_b64 exec, %11\n\t"
+               "v_fma_f32 %0, -%3, %7, %0\n\t"
+               "s_mov_b64 exec, %12\n\t"
+               "v_fma_f32 %0, -%4, %8, %0\n\t"
+               "s_mov_b64 exec, %13\n\t"
+               "v_fma_f32 %0, -%5, %9, %0\n\t"
+               "s_mov_b64 exec, %1"
+               : "+v"(acc), "=&s"(save)
+               : "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "v"(q[0]), "v"(q[1]), "v"(q[2]), "v"(q[3]), "s"(on[0]),
+                 "s"(on[1]), "s"(on[2]), "s"(on[3]));
+}
+
 struct WalkLds
 {
   int4 stk[WSTACK_CAP];  // (record offset, chain end, reached mask low, high word)
-  float4 rec[HBTX_WAVE + 1]; // a batch's records: x, y, z, m (then the lanes that opened each)
-  float4 aux[HBTX_WAVE + 1]; // crit2 (0 for a particle), mask low, crit2, mask high
-  // (one spare slot each: the record after a batch's last is read ahead and not used)
+  float4 rec[HBTX_WAVE]; // a batch's records: x, y, z, m (then the lanes that opened each)
+  float4 aux[HBTX_WAVE]; // crit2 (a cell only), mask low, crit2, mask high
 };
 
 #define WALK_STACK_OVERFLOW 4 // overflow-word bit: the walk stack was full (never expected)
@@ -192,41 +212,39 @@ HBTX_DEV void tree_walk_stack(const uint2 *wt, int ub, int ue, bool valid, float
   while (top > 0)
   {
     const int room = WSTACK_CAP - WSTACK_HEADROOM - top;
-    const int nb = uniform(min(min(HBTX_WAVE, top), max(1, room)));
+    const int nb = min(min(HBTX_WAVE, top), max(1, room));
     top -= nb;
-    const bool mine = lane < nb;
-    int4 it = make_int4(0, 0, 0, 0);
-    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-    float c2 = 0.f;
-    int32_t nx = 0;
-    bool cell = false;
-    if (mine)
+    const uint64_t mine = ~0ull >> (HBTX_WAVE - nb); // the lanes with an entry of the batch
+    // (a lane past them reads the last entry and stages it in the slot of its own number,
+    // which is past the batch: no branch)
+    const int src = top + min(lane, nb - 1);
+    int32_t nx;
+    int slot, ncell;
+    uint64_t cmask;
+    bool small_cells; // some cell's opening radius is below the softening length
     {
-      it = L.stk[top + lane];
+      const int4 it = L.stk[src];
       // 24 bytes whatever the record: a particle's last 8 are the next record's
       // (or the spare units past the records' end) and are not used, so that
       // both loads go out together
       const uint2 *rp = tree + (it.x >> 3);
       const uint2 u0 = rp[0], u1 = rp[1], u2 = rp[2];
-      a = make_float4(__uint_as_float(u0.x), __uint_as_float(u0.y), __uint_as_float(u1.x),
-                      __uint_as_float(u1.y));
-      cell = (int32_t)u1.y < 0;
-      c2 = cell ? __uint_as_float(u2.x) : 0.f;
+      const float c2 = __uint_as_float(u2.x);
+      // staged cells first, then particles (the order within a batch is free): a
+      // particle is never opened, so its visit skips the opening test and mask
+      cmask = __builtin_amdgcn_sicmp((int32_t)u1.y, 0, 40 /* < */) & mine;
+      small_cells = (cmask & ~__builtin_amdgcn_fcmpf(c2, P.h2, 3 /* ordered >= */)) != 0ull;
+      ncell = __popcll(cmask);
+      const bool cell = (int32_t)u1.y < 0 && lane < nb;
       nx = cell ? (int32_t)u2.y : it.x + 16;
-    }
-    // staged cells first, then particles (the order within a batch is free): a
-    // particle is never opened, so its visit skips the opening test and mask
-    const uint64_t lt = lanemask_lt();
-    const uint64_t cmask = wave_mask(mine && cell), pmask = wave_mask(mine && !cell);
-    const int ncell = __popcll(cmask);
-    const int slot = cell ? __popcll(cmask & lt) : ncell + __popcll(pmask & lt);
-    if (mine)
-    {
-      L.rec[slot] = make_float4(a.x, a.y, a.z, fabsf(a.w));
+      const int before = mask_rank(cmask, 0);
+      slot = cell ? before : ncell + lane - before;
+      L.rec[slot] = make_float4(__uint_as_float(u0.x), __uint_as_float(u0.y), __uint_as_float(u1.x),
+                                fabsf(__uint_as_float(u1.y)));
       L.aux[slot] = make_float4(c2, __int_as_float(it.z), c2, __int_as_float(it.w));
     }
     wave_lds_sync();
-    // Record j of the batch against every lane's target.  The lane predicates are
+    // Records of the batch against every lane's target.  The lane predicates are
     // single compares whose masks the scalar unit combines: reached R, opened Lt
     // (r2 < crit2), near N (r2 < h2).  An accepted lane (R, not Lt) adds -m/r,
     // or the spline where N; the sum runs under the accepting lanes' exec mask,
@@ -234,40 +252,90 @@ HBTX_DEV void tree_walk_stack(const uint2 *wt, int ub, int ue, bool valid, float
     // record is the target itself).  A cell's visit returns the lanes that opened it.
     using XF = std::true_type;
     using YF = std::false_type;
-    float4 rn = rec[0];
-    float2 wn = aw[0];
+    using CELL = std::true_type;
+    using PART = std::false_type;
     // (xf: the first of a group of four and the records past the last group square x
     // first, the others y)
-    auto visit = [&](int j, bool is_cell, auto xf) -> uint64_t {
-      // record j was read ahead; read record j + 1 while it is evaluated
-      const float4 r = rn;
-      const float2 w = wn;
-      rn = rec[j + 1];
-      wn = aw[2 * (j + 1)];
-      const float r2 = sep2<PERIODIC, decltype(xf)::value>(r.x, r.y, r.z, px, py, pz, P);
-      const uint64_t rm = __builtin_amdgcn_uicmp(__float_as_uint(w.y) & bit, 0u, 33 /* ne */);
-      const uint64_t lm = is_cell ? __builtin_amdgcn_fcmpf(r2, w.x, 4 /* ordered < */) : 0ull;
-      const uint64_t nm = __builtin_amdgcn_fcmpf(r2, P.h2, 4 /* ordered < */);
-      const float rinv = __builtin_amdgcn_rsqf(r2);
-      fma_neg_on(rm & ~(lm | nm), blk, r.w, rinv);
-      const uint64_t na = rm & nm & ~lm;
-      if (na != 0ull)
-      {
-        if (STATS)
-          wc.nnear++;
-        // at zero distance (the target's own record, or a coincident source) the
-        // spline is its value at u = 0, m hinv (-2.8), as spline_near forms it
-        const uint64_t zm = __builtin_amdgcn_fcmpf(r2, 0.f, 1 /* ordered == */);
-        const float tn = ((na & ~zm) == 0ull) ? (r.w * P.hinv) * -2.8f : spline_near(r2, rinv, r.w, P.hinv);
-        blk += lane_select(na, tn, 0.f);
-      }
+    auto reached = [&](float mask_word) {
+      return __builtin_amdgcn_uicmp(__float_as_uint(mask_word) & bit, 0u, 33 /* ne */);
+    };
+    auto near_terms = [&](uint64_t na, float r2, float rinv, float m) {
+      if (STATS)
+        wc.nnear++;
+      // at zero distance (the target's own record, or a coincident source) the
+      // spline is its value at u = 0, m hinv (-2.8), as spline_near forms it
+      const uint64_t zm = __builtin_amdgcn_fcmpf(r2, 0.f, 1 /* ordered == */);
+      const float tn = ((na & ~zm) == 0ull) ? (m * P.hinv) * -2.8f : spline_near(r2, rinv, m, P.hinv);
+      blk += lane_select(na, tn, 0.f);
+    };
+    auto count = [&](uint64_t rm, uint64_t lm) {
       if (STATS)
       {
         wc.steps++;
         wc.visits += __popcll(rm);
         wc.accepts += __popcll(rm & ~lm);
       }
+    };
+    auto visit = [&](int j, auto is_cell, auto xf) -> uint64_t {
+      const float4 r = rec[j];
+      const float2 w = aw[2 * j];
+      const float r2 = sep2<PERIODIC, decltype(xf)::value>(r.x, r.y, r.z, px, py, pz, P);
+      const uint64_t rm = reached(w.y);
+      const uint64_t lm = is_cell ? __builtin_amdgcn_fcmpf(r2, w.x, 4 /* ordered < */) : 0ull;
+      const uint64_t nm = __builtin_amdgcn_fcmpf(r2, P.h2, 4 /* ordered < */);
+      const float rinv = __builtin_amdgcn_rsqf(r2);
+      fma_neg_on(rm & ~(lm | nm), blk, r.w, rinv);
+      const uint64_t na = rm & nm & ~lm;
+      if (na != 0ull)
+        near_terms(na, r2, rinv, r.w);
+      count(rm, lm);
       return rm & lm;
+    };
+    // Four records at once.  A cell no smaller than the softening (crit2 >= h2: all but
+    // some 0.3% of the cells met) is opened by every lane it is near to, so it has no
+    // near test; four particles share one branch on it.  Bound: the vector unit (some 16
+    // instructions a record, 69% of its cycles) and, of a few waves, the latency of a
+    // record's chain.  With a near test and branch a record: 8e6 particles, five rounds'
+    // walks 5.33 ms, 5.16 so; a halo of 12,000 (two rounds of 188 waves) 0.394 and 0.366 ms.
+    auto visit4 = [&](int j, auto is_cell, uint64_t opened[4]) {
+      float m[4], r2[4], rinv[4];
+      uint64_t rm[4], lm[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+      {
+        const float4 r = rec[j + k];
+        const float2 w = aw[2 * (j + k)];
+        r2[k] = (k == 0) ? sep2<PERIODIC, true>(r.x, r.y, r.z, px, py, pz, P)
+                         : sep2<PERIODIC, false>(r.x, r.y, r.z, px, py, pz, P);
+        m[k] = r.w;
+        rm[k] = reached(w.y);
+        // (opened by: a cell; near to: a particle)
+        lm[k] = __builtin_amdgcn_fcmpf(r2[k], is_cell ? w.x : P.h2, 4 /* ordered < */);
+        rinv[k] = __builtin_amdgcn_rsqf(r2[k]);
+        count(rm[k], is_cell ? lm[k] : 0ull);
+      }
+      if (is_cell)
+      {
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+        {
+          opened[k] = rm[k] & lm[k];
+          rm[k] &= ~lm[k];
+        }
+        fma_neg_on4(rm, blk, m, rinv);
+      }
+      else if (((rm[0] & lm[0]) | (rm[1] & lm[1]) | (rm[2] & lm[2]) | (rm[3] & lm[3])) == 0ull)
+        fma_neg_on4(rm, blk, m, rinv);
+      else
+      {
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+        {
+          fma_neg_on(rm[k] & ~lm[k], blk, m[k], rinv[k]);
+          if ((rm[k] & lm[k]) != 0ull)
+            near_terms(rm[k] & lm[k], r2[k], rinv[k], m[k]);
+        }
+      }
     };
     // plain FP32 sums over blocks of at least 16 records, Kahan-compensated
     // across blocks
@@ -285,20 +353,27 @@ HBTX_DEV void tree_walk_stack(const uint2 *wt, int ub, int ue, bool valid, float
     int j = 0;
     for (; j + 4 <= ncell; j += 4)
     {
-      const uint64_t o0 = visit(j, true, XF()), o1 = visit(j + 1, true, YF()),
-                     o2 = visit(j + 2, true, YF()), o3 = visit(j + 3, true, YF());
+      uint64_t o[4];
+      if (small_cells)
+      {
+        o[0] = visit(j, CELL(), XF());
+        o[1] = visit(j + 1, CELL(), YF());
+        o[2] = visit(j + 2, CELL(), YF());
+        o[3] = visit(j + 3, CELL(), YF());
+      }
+      else
+        visit4(j, CELL(), o);
       if (lane == 0)
       {
-        omw[2 * j] = make_uint2((uint32_t)o0, (uint32_t)(o0 >> 32));
-        omw[2 * j + 2] = make_uint2((uint32_t)o1, (uint32_t)(o1 >> 32));
-        omw[2 * j + 4] = make_uint2((uint32_t)o2, (uint32_t)(o2 >> 32));
-        omw[2 * j + 6] = make_uint2((uint32_t)o3, (uint32_t)(o3 >> 32));
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+          omw[2 * (j + k)] = make_uint2((uint32_t)o[k], (uint32_t)(o[k] >> 32));
       }
       block_end(4);
     }
     for (; j < ncell; j++)
     {
-      const uint64_t o = visit(j, true, XF());
+      const uint64_t o = visit(j, CELL(), XF());
       if (lane == 0)
         omw[2 * j] = make_uint2((uint32_t)o, (uint32_t)(o >> 32));
       block_end(1);
@@ -306,28 +381,22 @@ HBTX_DEV void tree_walk_stack(const uint2 *wt, int ub, int ue, bool valid, float
     // particles
     for (; j + 4 <= nb; j += 4)
     {
-      visit(j, false, XF());
-      visit(j + 1, false, YF());
-      visit(j + 2, false, YF());
-      visit(j + 3, false, YF());
+      visit4(j, PART(), nullptr);
       block_end(4);
     }
     for (; j < nb; j++)
     {
-      visit(j, false, XF());
+      visit(j, PART(), XF());
       block_end(1);
     }
     // push the chains' rests and the opened cells' children
     wave_lds_sync();
     // (the popped entries are still in place: nothing is pushed before this point)
-    if (mine)
-      it = L.stk[top + lane];
-    const bool is_cell = slot < ncell;
+    const int4 it = L.stk[src];
     const uint2 om = reinterpret_cast<const uint2 *>(L.rec)[2 * slot];
-    const bool sib = mine && nx < it.y;
-    const bool kid = mine && is_cell && (om.x | om.y) != 0u;
-    const uint64_t msib = wave_mask(sib), mkid = wave_mask(kid);
-    int pos = top + __popcll(msib & lt) + __popcll(mkid & lt);
+    const uint64_t msib = __builtin_amdgcn_sicmp(nx, it.y, 40 /* < */) & mine;
+    const uint64_t mkid = __builtin_amdgcn_uicmp(om.x | om.y, 0u, 33 /* ne */) & cmask;
+    int pos = mask_rank(mkid, mask_rank(msib, top));
     const int pushed = __popcll(msib) + __popcll(mkid);
     if (top + pushed > WSTACK_CAP)
     {
@@ -335,9 +404,9 @@ HBTX_DEV void tree_walk_stack(const uint2 *wt, int ub, int ue, bool valid, float
         atomicOr(overflow, WALK_STACK_OVERFLOW);
       break;
     }
-    if (sib)
+    if (nx < it.y && lane < nb)
       L.stk[pos++] = make_int4(nx, it.y, it.z, it.w);
-    if (kid)
+    if ((om.x | om.y) != 0u && slot < ncell)
       L.stk[pos] = make_int4(it.x + 24, nx, (int)om.x, (int)om.y);
     top = uniform(top + pushed);
     wave_lds_sync();
