@@ -974,6 +974,7 @@ WalkArgs walk_args(hbtx_ctx *c, Batch &B, View &V, const DevParams &P)
   W.ntgt = V.S.ntgt;
   W.mode = V.S.mode;
   W.treemode = V.S.treemode;
+  W.cube = V.S.cube;
   W.ent_begin = V.S.ent_begin;
   W.ent_end = V.S.ent_end;
   W.wt = B.wt.p;
@@ -1759,6 +1760,7 @@ void tree_points(hbtx_ctx *c, hbtx_tree *T, int64_t nt, const float *tpos, const
   A.eb = 0;
   A.ee = T->nw;
   A.treemode = T->treemode;
+  A.cube = T->cube.p;
   A.wt = T->wt.p;
   A.phi = nullptr;
   A.phi_d = W.phi.p;
@@ -2255,6 +2257,7 @@ int hbtx_direct_potential_noalloc(hbtx_ctx *c, const hbtx_params *prm, int64_t n
       A.eb = 0;
       A.ee = (int32_t)(2 * n_src);
       A.treemode = 0;
+      A.cube = nullptr;
       A.wt = wt;
       A.phi = nullptr;
       A.phi_d = d_out_pot;

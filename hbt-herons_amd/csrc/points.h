@@ -13,6 +13,7 @@ struct PointArgs
   int32_t ntgt;
   int32_t eb, ee;          // walk-record unit range
   int32_t treemode;
+  const double *cube;      // the tree's root cube (centre, half side)
   const uint2 *wt;         // walk records
   float *phi;              // specific potential, scattered to the target's input index, or null
   double *phi_d;           // optional double output
@@ -63,11 +64,18 @@ __global__ __launch_bounds__(WALK_WG_THREADS, 8) void k_points_potential(PointAr
     {
       if (A.treemode)
       {
-        tree_walk_stack<PERIODIC, STATS>(A.wt, A.eb, A.ee, valid, x.x, x.y, x.z, A.P, acc, wc, wl, A.overflow);
+        if (PERIODIC && cube_may_wrap(A.cube, valid, x.x, x.y, x.z, A.P))
+          tree_walk_stack<PERIODIC, STATS>(A.wt, A.eb, A.ee, valid, x.x, x.y, x.z, A.P, acc, wc, wl, A.overflow);
+        else
+          tree_walk_stack<false, STATS>(A.wt, A.eb, A.ee, valid, x.x, x.y, x.z, A.P, acc, wc, wl, A.overflow);
       }
       else
       {
-        direct_sum<PERIODIC>(A.wt, A.eb, A.ee, x.x, x.y, x.z, A.P, acc, wc);
+        if (PERIODIC &&
+            records_may_wrap(A.wt + A.eb, lane, HBTX_WAVE, (A.ee - A.eb) / 2, valid, x.x, x.y, x.z, A.P))
+          direct_sum<PERIODIC>(A.wt, A.eb, A.ee, x.x, x.y, x.z, A.P, acc, wc);
+        else
+          direct_sum<false>(A.wt, A.eb, A.ee, x.x, x.y, x.z, A.P, acc, wc);
         if (STATS)
           st_pairs += (unsigned long long)__popcll(wave_mask(valid)) * (unsigned long long)((A.ee - A.eb) / 2);
       }
@@ -128,15 +136,19 @@ __global__ __launch_bounds__(DS_THREADS) void k_points_direct(PointArgs A)
       x = A.tgt[ti];
     Kahan acc;
     acc.init();
+    const bool wraps = PERIODIC && __syncthreads_or(records_may_wrap(ent, threadIdx.x, DS_THREADS, ee, valid, x.x, x.y,
+                                                                     x.z, A.P));
     // stage st is formed in buffer st & 1 while stage st - 1 is added from the other
     for (int st = 0; st <= nstage; st++)
     {
       if (w < DS_WAVES)
       {
         const int g0 = (st * DS_WAVES + w) * DS_GROUPS;
-        if (st < nstage)
-          direct_groups<PERIODIC, 2>(ent, g0, min(ng, g0 + DS_GROUPS), x.x, x.y, x.z, A.P, wc,
-                                  [&](int g, float part) { parts[st & 1][w * DS_GROUPS + (g - g0)][lane] = part; });
+        auto emit = [&](int g, float part) { parts[st & 1][w * DS_GROUPS + (g - g0)][lane] = part; };
+        if (st < nstage && PERIODIC && wraps)
+          direct_groups<PERIODIC, 2>(ent, g0, min(ng, g0 + DS_GROUPS), x.x, x.y, x.z, A.P, wc, emit);
+        else if (st < nstage)
+          direct_groups<false, 2>(ent, g0, min(ng, g0 + DS_GROUPS), x.x, x.y, x.z, A.P, wc, emit);
       }
       else if (st > 0)
       {

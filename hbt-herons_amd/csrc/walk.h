@@ -43,6 +43,7 @@ struct WalkArgs
   const int32_t *ntgt;
   const int32_t *mode;
   const int32_t *treemode;
+  const double *cube;       // per subhalo: its tree's root cube (centre, half side), see cube_may_wrap
   const int32_t *ent_begin; // per subhalo: first walk-record unit of its tree
   const int32_t *ent_end;   // per subhalo: end unit
   const uint2 *wt;          // walk records (8-byte units, two spare units past the end)
@@ -85,6 +86,55 @@ HBTX_DEV float sep2(float ex, float ey, float ez, float px, float py, float pz, 
     dz = ez - pz;
   }
   return __builtin_fmaf(dz, dz, XFIRST ? __builtin_fmaf(dy, dy, dx * dx) : __builtin_fmaf(dx, dx, dy * dy));
+}
+
+// In a periodic box a pair's separation is wrapped only where one of its components
+// is beyond half the box; elsewhere the wrapped separation and its rounding are those
+// of a plain difference.  So a wave first asks whether any of its pairs can be: where
+// none can (every subhalo that does not straddle the box edge), its targets take the
+// non-periodic form, 3 vector instructions a pair for the separation instead of 33, and
+// the same bits.  1e6 particles of periodic subhaloes: walks of five rounds 1.74 ms with
+// every pair wrapped, 1.05 ms so.
+//
+// Of the targets against a tree: the particles lie in the root cube, the cells' centres
+// of mass within rounding of it (the margin).
+HBTX_DEV bool cube_may_wrap(const double *cube, bool valid, float px, float py, float pz, const DevParams &P)
+{
+  const double reach = 0.999 * (double)P.box_half - cube[3];
+  const bool ok = fabs((double)px - cube[0]) <= reach && fabs((double)py - cube[1]) <= reach &&
+                  fabs((double)pz - cube[2]) <= reach;
+  return wave_mask(valid && !ok) != 0ull; // (NaN: wrapped)
+}
+
+// Of the targets against the particle records first, first + step, ... < n of this lane;
+// the wave's answer covers all its lanes' records.
+HBTX_DEV bool records_may_wrap(const uint2 *ent, int first, int step, int n, bool valid, float px, float py, float pz,
+                               const DevParams &P)
+{
+  float lo[3] = {px, py, pz}, hi[3] = {px, py, pz};
+#pragma unroll
+  for (int k = 0; k < 3; k++)
+  {
+    lo[k] = valid ? lo[k] : INFINITY;
+    hi[k] = valid ? hi[k] : -INFINITY;
+#pragma unroll
+    for (int d = 1; d < HBTX_WAVE; d <<= 1)
+    {
+      lo[k] = fminf(lo[k], __shfl_xor(lo[k], d, HBTX_WAVE));
+      hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], d, HBTX_WAVE));
+    }
+  }
+  bool ok = true;
+#pragma unroll 4
+  for (int i = first; i < n; i += step)
+  {
+    const uint2 a = ent[2 * (int64_t)i], b = ent[2 * (int64_t)i + 1];
+    const float r[3] = {__uint_as_float(a.x), __uint_as_float(a.y), __uint_as_float(b.x)};
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+      ok = ok && r[k] - lo[k] <= P.box_half && r[k] - hi[k] >= -P.box_half;
+  }
+  return wave_mask(!ok) != 0ull; // (NaN: wrapped)
 }
 
 // Per-wave work counters of one walk (uniform values, kept only in the stats
@@ -354,7 +404,7 @@ HBTX_DEV void tree_walk_stack(const uint2 *wt, int ub, int ue, bool valid, float
     for (; j + 4 <= ncell; j += 4)
     {
       uint64_t o[4];
-      if (small_cells)
+      if (PERIODIC || small_cells) // (wrapped separations of four at once do not fit the registers)
       {
         o[0] = visit(j, CELL(), XF());
         o[1] = visit(j + 1, CELL(), YF());
@@ -381,7 +431,15 @@ HBTX_DEV void tree_walk_stack(const uint2 *wt, int ub, int ue, bool valid, float
     // particles
     for (; j + 4 <= nb; j += 4)
     {
-      visit4(j, PART(), nullptr);
+      if (PERIODIC)
+      {
+        visit(j, PART(), XF());
+        visit(j + 1, PART(), YF());
+        visit(j + 2, PART(), YF());
+        visit(j + 3, PART(), YF());
+      }
+      else
+        visit4(j, PART(), nullptr);
       block_end(4);
     }
     for (; j < nb; j++)
@@ -594,11 +652,17 @@ __global__ __launch_bounds__(WALK_WG_THREADS, 8) void k_walk_energy(WalkArgs A)
     {
       if (A.treemode[s])
       {
-        tree_walk_stack<PERIODIC, STATS>(A.wt, eb, ee, valid, x.x, x.y, x.z, P, acc, wc, wl, A.overflow);
+        if (PERIODIC && cube_may_wrap(A.cube + 4 * (int64_t)s, valid, x.x, x.y, x.z, P))
+          tree_walk_stack<PERIODIC, STATS>(A.wt, eb, ee, valid, x.x, x.y, x.z, P, acc, wc, wl, A.overflow);
+        else
+          tree_walk_stack<false, STATS>(A.wt, eb, ee, valid, x.x, x.y, x.z, P, acc, wc, wl, A.overflow);
       }
       else
       {
-        direct_sum<PERIODIC>(A.wt, eb, ee, x.x, x.y, x.z, P, acc, wc);
+        if (PERIODIC && records_may_wrap(A.wt + eb, lane, HBTX_WAVE, (ee - eb) / 2, valid, x.x, x.y, x.z, P))
+          direct_sum<PERIODIC>(A.wt, eb, ee, x.x, x.y, x.z, P, acc, wc);
+        else
+          direct_sum<false>(A.wt, eb, ee, x.x, x.y, x.z, P, acc, wc);
         if (STATS)
           st_pairs += (unsigned long long)__popcll(wave_mask(valid)) * (unsigned long long)((ee - eb) / 2);
       }
