@@ -20,6 +20,9 @@
 #include "transfer.h"
 
 #define WALK_MAX_CHUNKS 16
+#define WALK_COUNTERS ((WALK_MAX_CHUNKS + 1) * QUEUE_STRIDE) // ints
+#define POINT_CHUNKS 8 // chunks of a point walk's items (one per XCD)
+#define POINT_COUNTERS ((POINT_CHUNKS + 1) * QUEUE_STRIDE)
 // entries whose walk records (at most 3 units each) keep unit offsets in int32
 #define WREC_MAX_ENTRIES ((int64_t)0x7ffffff0 / 3 - 8)
 
@@ -205,7 +208,7 @@ struct Batch
   DArr<double> cube, len0, red, red2;
   DArr<uint32_t> bbox;
   DArr<int32_t> misc; // [0] active, [1] (unused), [2] overflow, [3] entry total, [4] max depth
-  DArr<int32_t> wctr; // walk work counters, 16 ints apart
+  DArr<int32_t> wctr; // walk work counters
   DArr<char2> lev;                // per dense source: the level pair of its tree
   DArr<int32_t> mom_slots;        // moment passes: per window / group, the cells that end beyond it
   DArr<hbtx_sub_result> dres;
@@ -700,7 +703,7 @@ void batch_reserve(hbtx_ctx *c, Batch &B)
   B.red2.alloc((int64_t)RED_NV * ns + RED_NV);
   B.bbox.alloc(6 * (int64_t)ns + 6);
   B.misc.alloc(8);
-  B.wctr.alloc(16 * WALK_MAX_CHUNKS);
+  B.wctr.alloc(WALK_COUNTERS);
   B.dres.alloc(ns + 1);
   c->stats.alloc(NSTATS);
   {
@@ -1000,12 +1003,12 @@ void round_items(hbtx_ctx *c, Batch &B, View &V)
   const int gs = blocks_for(V.nsub, 256, 1 << 20);
   int32_t *total = B.misc.p + 7; // read after the round
   if (V.nsub <= LIST_ONE_MAX)
-    k_items_one<<<1, LIST_THREADS, 0, st>>>(V.S, V.order, B.iscan.p, B.wctr.p, 16 * WALK_MAX_CHUNKS, total);
+    k_items_one<<<1, LIST_THREADS, 0, st>>>(V.S, V.order, B.iscan.p, B.wctr.p, WALK_COUNTERS, total);
   else
   {
     k_items_count<<<gs, 256, 0, st>>>(V.S, V.order, B.icnt.p);
     scan32(c, B.icnt.p, B.iscan.p, V.nsub);
-    k_items_finish<<<1, 256, 0, st>>>(B.iscan.p + V.nsub, B.wctr.p, 16 * WALK_MAX_CHUNKS, total);
+    k_items_finish<<<1, 256, 0, st>>>(B.iscan.p + V.nsub, B.wctr.p, WALK_COUNTERS, total);
   }
   k_items_emit<<<blocks_for((int64_t)V.nsub * HBTX_WAVE, 256, 1 << 24), 256, 0, st>>>(V.S, V.order, B.iscan.p,
                                                                                        B.items.p);
@@ -1742,13 +1745,13 @@ void tree_points(hbtx_ctx *c, hbtx_tree *T, int64_t nt, const float *tpos, const
   W.keys.alloc(nt);
   W.vals.alloc(nt);
   W.seg.alloc(4); // the range, and the sort's copy of it
-  W.counter.alloc(2); // [0] work counter, [1] overflow word
+  W.counter.alloc(POINT_COUNTERS + 1); // work counters, then the overflow word
   std::vector<XferPart> parts{xfer_from(0, tpos, 3 * nt * sizeof(float))};
   if (tmass)
     parts.push_back(xfer_from(3 * nt * sizeof(float), tmass, nt * sizeof(float)));
   HIPCHK(c->staging.up(c->device, st, W.raw.p, parts));
   k_pack_points<<<blocks_for(nt), 256, 0, st>>>(W.raw.p, tmass ? W.raw.p + 3 * nt : nullptr, (int32_t)nt, W.tgt.p);
-  k_points_begin<<<1, 64, 0, st>>>(W.counter.p, W.seg.p, (int32_t)nt);
+  k_points_begin<<<1, 256, 0, st>>>(W.counter.p, POINT_COUNTERS + 1, W.seg.p, (int32_t)nt);
   // walk order: targets sorted by their key in the tree cube
   k_point_keys<<<blocks_for(nt), 256, 0, st>>>(W.tgt.p, (int32_t)nt, T->cube.p, W.keys.p, W.vals.p);
   if (T->treemode)
@@ -1765,8 +1768,9 @@ void tree_points(hbtx_ctx *c, hbtx_tree *T, int64_t nt, const float *tpos, const
   A.phi = nullptr;
   A.phi_d = W.phi.p;
   A.counter = W.counter.p;
+  A.chunks = POINT_CHUNKS;
   A.stats = c->stats.p;
-  A.overflow = W.counter.p + 1;
+  A.overflow = W.counter.p + POINT_COUNTERS;
   A.P = T->P;
   HIPCHK(hipMemsetAsync(c->stats.p, 0, NSTATS * sizeof(unsigned long long), st));
   HIPCHK(hipEventRecord(c->wev0, st));
@@ -1777,7 +1781,7 @@ void tree_points(hbtx_ctx *c, hbtx_tree *T, int64_t nt, const float *tpos, const
   HIPCHK(hipEventRecord(c->wev1, st));
   HIPCHK(hipGetLastError());
   int32_t ov = 0;
-  HIPCHK(c->staging.down(c->device, st, {xfer_to(out, W.phi.p, nt * sizeof(double)), xfer_to(&ov, W.counter.p + 1, 4)}));
+  HIPCHK(c->staging.down(c->device, st, {xfer_to(out, W.phi.p, nt * sizeof(double)), xfer_to(&ov, W.counter.p + POINT_COUNTERS, 4)}));
   REQUIRE(ov == 0, HBTX_E_CAPACITY, "tree walk stack capacity exceeded");
   float wms = 0.f;
   HIPCHK(hipEventElapsedTime(&wms, c->wev0, c->wev1));
@@ -2261,7 +2265,8 @@ int hbtx_direct_potential_noalloc(hbtx_ctx *c, const hbtx_params *prm, int64_t n
       A.wt = wt;
       A.phi = nullptr;
       A.phi_d = d_out_pot;
-      A.counter = counter;
+      A.counter = counter; // (the scratch array holds one)
+      A.chunks = 1;
       A.stats = nullptr;
       A.overflow = nullptr; // direct sums only
       A.P = P;

@@ -17,7 +17,8 @@ struct PointArgs
   const uint2 *wt;         // walk records
   float *phi;              // specific potential, scattered to the target's input index, or null
   double *phi_d;           // optional double output
-  int32_t *counter;
+  int32_t *counter;        // work counters (ItemQueue), zeroed before launch
+  int32_t chunks;          // item list split into this many contiguous chunks
   unsigned long long *stats;
   int32_t *overflow;       // set to WALK_STACK_OVERFLOW if the walk stack was full, or null
   DevParams P;
@@ -43,13 +44,12 @@ __global__ __launch_bounds__(WALK_WG_THREADS, 8) void k_points_potential(PointAr
   WalkLds &wl = wls[threadIdx.x / HBTX_WAVE];
   unsigned long long st_steps = 0, st_visits = 0, st_accepts = 0, st_pairs = 0, st_near = 0;
   const int nitems = (A.ntgt + HBTX_WAVE - 1) / HBTX_WAVE;
+  ItemQueue queue;
+  queue.init(A.counter, A.chunks, nitems);
   for (;;)
   {
-    int it = 0;
-    if (lane == 0)
-      it = atomicAdd(A.counter, 1);
-    it = uniform(__shfl(it, 0, HBTX_WAVE));
-    if (it >= nitems)
+    const int it = queue.next();
+    if (it < 0)
       break;
     const int t = it * HBTX_WAVE + lane;
     const bool valid = t < A.ntgt;
@@ -188,14 +188,14 @@ __global__ __launch_bounds__(DS_THREADS) void k_points_direct(PointArgs A)
   }
 }
 
-// the walk's counters cleared, and one sort segment over the n targets
-__global__ void k_points_begin(int32_t *counter, int32_t *seg, int32_t n)
+// the walk's n_words counters (and overflow word) cleared, and one sort segment over the
+// n targets
+__global__ void k_points_begin(int32_t *counter, int n_words, int32_t *seg, int32_t n)
 {
-  if (blockIdx.x == 0 && threadIdx.x < 2)
-  {
-    counter[threadIdx.x] = 0;
+  for (int i = threadIdx.x; i < n_words; i += blockDim.x)
+    counter[i] = 0;
+  if (threadIdx.x < 2)
     seg[threadIdx.x] = (threadIdx.x == 0) ? 0 : n;
-  }
 }
 
 // keys of external target points in a tree's cube (walk order for coherence)

@@ -36,8 +36,8 @@ struct WalkArgs
 {
   const int2 *items;        // (subhalo, first target) per work item
   const int32_t *nitems;    // number of items (device)
-  int32_t *counter;         // work-stealing counters, one per item chunk, 16 ints apart (zeroed before launch)
-  int32_t nchunks;          // item list split into this many contiguous chunks (1 = one shared counter)
+  int32_t *counter;         // work counters (ItemQueue), zeroed before launch
+  int32_t nchunks;          // item list split into this many contiguous chunks
   const int32_t *cur;       // slot-layout target order
   const int32_t *off;       // per subhalo slot offset
   const int32_t *ntgt;
@@ -65,6 +65,83 @@ HBTX_DEV uint64_t wave_mask(bool p)
 {
   return __builtin_amdgcn_ballot_w64(p);
 }
+
+// Waves per walk workgroup.  Every wave walks on its own (its own items and its
+// own LDS stack, no workgroup barrier); one, two and four waves a workgroup
+// time the same, as a CU holds 32 one-wave workgroups with this LDS size.
+#ifndef HBTX_WALK_WG_WAVES
+#define HBTX_WALK_WG_WAVES 2
+#endif
+constexpr int WALK_WG_THREADS = HBTX_WAVE * HBTX_WALK_WG_WAVES;
+
+// Work items 0 .. nit - 1 handed to the waves of a persistent kernel.  The list is cut
+// into nch contiguous chunks with a counter each: workgroups go round the XCDs, so
+// workgroup b drains chunk b % nch first (neighbouring items, which read the same part of
+// a tree, stay on one XCD's L2), then helps with the others.  The wave that finds a chunk
+// empty first sets its bit in the word after the counters, and a wave looking for
+// another chunk reads that word before it touches a counter.  With a failed addition on
+// each of eight counters a wave, which are served one after the other, 8,192 waves spent
+// longer on ending than a round of small items takes: walks of 1.2e6 particles in
+// subhaloes of at most 2,000, 0.89 ms, 0.47 so; in subhaloes up to a million, 2.1e6
+// particles 2.12 and 1.72 ms, 8e6 5.08 and 4.74.  (More counters than one an XCD made it worse, 5.9 ms of 8e6: a wave that
+// looks for work then reads them all, and they are what the others are adding to.)
+#define QUEUE_STRIDE 32 // ints between counters: a cache line each
+struct ItemQueue
+{
+  int32_t *ctr;
+  int nch, q, r; // chunks, items a chunk (one more in the first r)
+  int wq, wr;    // the same of the workgroups
+  int cur;
+  int first;     // this wave's number among its chunk's (-1 once it has taken that item)
+  uint32_t done; // the chunks known to be empty
+
+  HBTX_DEV void init(int32_t *counters, int chunks, int nit)
+  {
+    ctr = counters;
+    nch = chunks;
+    nit = uniform(nit);
+    q = nit / nch;
+    r = nit - q * nch;
+    wq = gridDim.x / nch;
+    wr = gridDim.x - wq * nch;
+    const int g = blockIdx.x / nch;
+    cur = blockIdx.x - g * nch;
+    first = g * HBTX_WALK_WG_WAVES + uniform(threadIdx.x / HBTX_WAVE);
+    done = 0u;
+  }
+  // the next item, or -1 (every wave ends: a turn that gives no item marks a chunk)
+  HBTX_DEV int next()
+  {
+    for (;;)
+    {
+      // the chunk's first items go to its own waves by number, the rest by the counter
+      const int size = q + (cur < r ? 1 : 0), waves = (wq + (cur < wr ? 1 : 0)) * HBTX_WALK_WG_WAVES;
+      int got = first;
+      if (first < 0)
+      {
+        got = 0;
+        if (lane_id() == 0)
+          got = atomicAdd(ctr + QUEUE_STRIDE * cur, 1);
+        got = waves + uniform(got);
+      }
+      first = -1;
+      if (got < size)
+        return cur * q + min(cur, r) + got;
+      done |= 1u << cur;
+      if (nch == 1)
+        return -1;
+      uint32_t *word = reinterpret_cast<uint32_t *>(ctr + QUEUE_STRIDE * nch);
+      if (got == max(size, waves) && lane_id() == 0)
+        atomicOr(word, 1u << cur);
+      done |= (uint32_t)uniform((int)__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+      const uint32_t left = ~done & ((1u << nch) - 1u);
+      if (left == 0u)
+        return -1;
+      const uint32_t after = left & ~((2u << cur) - 1u); // the next chunk, or the first
+      cur = __ffs((int)(after ? after : left)) - 1;
+    }
+  }
+};
 
 // Squared distance with the fused multiply-adds written out, so that every kernel
 // rounds alike: the x square first where XFIRST, else the y square.
@@ -169,14 +246,6 @@ struct WalkCounts
 // taken) raises the overflow word instead of writing.
 constexpr int WSTACK_CAP = 160;
 constexpr int WSTACK_HEADROOM = 32;
-
-// Waves per walk workgroup.  Every wave walks on its own (its own items and its
-// own LDS stack, no workgroup barrier); one, two and four waves a workgroup
-// time the same, as a CU holds 32 one-wave workgroups with this LDS size.
-#ifndef HBTX_WALK_WG_WAVES
-#define HBTX_WALK_WG_WAVES 2
-#endif
-constexpr int WALK_WG_THREADS = HBTX_WAVE * HBTX_WALK_WG_WAVES;
 
 // m's bit for this lane ? a : b, with m a wave-uniform lane mask: one
 // v_cndmask on the mask's SGPR pair, where a select on a per-lane bool would first
@@ -605,33 +674,11 @@ __global__ __launch_bounds__(WALK_WG_THREADS, 8) void k_walk_energy(WalkArgs A)
   WalkLds &wl = wls[threadIdx.x / HBTX_WAVE];
   unsigned long long st_steps = 0, st_visits = 0, st_accepts = 0, st_pairs = 0, st_targets = 0, st_items = 0,
                      st_near = 0;
-  // XCD-aware work distribution: workgroups are dispatched round-robin over the
-  // XCDs, so workgroup b runs on XCD b % 8.  The item list (targets in key order,
-  // largest subhalo first) is cut into nchunks contiguous chunks; a wave drains the
-  // chunk of its XCD first, so neighbouring targets - which walk the same part of
-  // the tree - share that XCD's L2, then helps with the other chunks.
-  const int nit = *A.nitems;
-  const int nch = A.nchunks;
-  int chunk = blockIdx.x % nch;
-  int tried = 0;
+  ItemQueue queue;
+  queue.init(A.counter, A.nchunks, *A.nitems);
   for (;;)
   {
-    int it = -1;
-    while (tried < nch)
-    {
-      const int cb = (int)((int64_t)nit * chunk / nch), ce = (int)((int64_t)nit * (chunk + 1) / nch);
-      int got = 0;
-      if (lane == 0)
-        got = atomicAdd(A.counter + 16 * chunk, 1);
-      got = uniform(__shfl(got, 0, HBTX_WAVE));
-      if (cb + got < ce)
-      {
-        it = cb + got;
-        break;
-      }
-      tried++;
-      chunk = (chunk + 1 == nch) ? 0 : chunk + 1;
-    }
+    const int it = queue.next();
     if (it < 0)
       break;
     const int2 item = A.items[it];
