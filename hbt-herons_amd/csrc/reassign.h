@@ -455,15 +455,16 @@ __global__ void k_rs_tiles(RsArgs A, int4 *tiles, int32_t ntiles)
 
 // Squared pair distance as the reference computes it: double differences of
 // the float coordinates, NEAREST per axis, rounded to float for the heap
-// (src/geometric_tree.cpp:158-181; LocatedParticle_t::d2 is HBTReal).
-HBTX_DEV double rs_r2(float tx, float ty, float tz, float qx, float qy, float qz, const RsArgs &A, double &dx,
-                      double &dy, double &dz)
+// (src/geometric_tree.cpp:158-181; LocatedParticle_t::d2 is HBTReal).  wraps: NEAREST may
+// change a difference.
+HBTX_DEV double rs_r2(float tx, float ty, float tz, float qx, float qy, float qz, const RsArgs &A, bool wraps,
+                      double &dx, double &dy, double &dz)
 {
 #pragma clang fp contract(off) // no fused multiply-add: the sum rounds as the host's does
   dx = (double)tx - (double)qx;
   dy = (double)ty - (double)qy;
   dz = (double)tz - (double)qz;
-  if (A.periodic)
+  if (wraps)
   {
     dx = nearest_d(dx, (double)A.box, (double)A.half);
     dy = nearest_d(dy, (double)A.box, (double)A.half);
@@ -529,14 +530,36 @@ HBTX_DEV float rs_box_gap2(float ux, float uy, float uz, float lx, float ly, flo
 // Neighbours are ordered by (squared distance, particle index), one 64-bit key
 // (the float bits of a non-negative distance order as integers): the reference
 // orders exactly equal float distances by its tree's traversal order and its
-// heap's internals, which no other search reproduces.
-HBTX_DEV uint64_t rs_nkey(float d2, int pid)
+// heap's internals, which no other search reproduces.  The key is held as the double of
+// the same bits (never a NaN: a distance's bits stay below 0x7ff00000), which order the
+// same way, so that an insertion into the sorted list is one v_min_f64 and one
+// v_max_f64 a place (written out: the builtins first quiet NaNs of unknown operands).
+// The kernel is bound by the vector unit (93% of its cycles), an insertion through
+// 64-bit compares and selects was half of it: k = 10 of 3.8e6 particles 2.30 ms, 2.13 so;
+// k = 20 of 2.1e6, 6.9 and 2.5; k = 32 of 6.0e6, 23.7 and 7.2.
+HBTX_DEV double rs_nkey(float d2, int pid)
 {
-  return ((uint64_t)__float_as_uint(d2) << 32) | (uint32_t)pid;
+  return __longlong_as_double((long long)(((uint64_t)__float_as_uint(d2) << 32) | (uint32_t)pid));
 }
-HBTX_DEV float rs_nkey_d2(uint64_t key)
+HBTX_DEV float rs_nkey_d2(double key)
 {
-  return __uint_as_float((uint32_t)(key >> 32));
+  return __uint_as_float((uint32_t)((uint64_t)__double_as_longlong(key) >> 32));
+}
+HBTX_DEV int rs_nkey_pid(double key)
+{
+  return (int32_t)(uint32_t)(uint64_t)__double_as_longlong(key);
+}
+HBTX_DEV double rs_kmin(double a, double b)
+{
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+HBTX_DEV double rs_kmax(double a, double b)
+{
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
 }
 
 // Union walk of one wave over its host halo's boxes.  Every lane keeps the k
@@ -592,26 +615,35 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_knn(RsArgs A, const int4 *__r
     auto level_base = [&](int l) -> int64_t {
       return ((int64_t)rd_lane(lb_hi, l) << 32) | (uint32_t)rd_lane(lb_lo, l);
     };
-    uint64_t key[K];
+    double key[K];
 #pragma unroll
     for (int j = 0; j < K; j++)
-      key[j] = (j < K - k) ? 0ull : ~0ull;
+      key[j] = (j < K - k) ? 0. : (double)INFINITY;
     // a lane's screen: no tracer whose float lower bound of the squared distance
     // exceeds it can be nearer than its k-th (+inf until k are held; inactive lanes
     // pass nothing)
     float kth = active ? INFINITY : -1.f;
-    auto insert = [&](uint64_t x) {
+    auto insert = [&](double x) { // (a key beyond the k-th changes nothing)
 #pragma unroll
       for (int j = K - 1; j > 0; j--)
-      {
-        const bool sh = x < key[j - 1];
-        const bool pl = !sh && x < key[j];
-        key[j] = sh ? key[j - 1] : (pl ? x : key[j]);
-      }
-      if (x < key[0])
-        key[0] = x;
-      kth = (key[K - 1] == ~0ull) ? INFINITY : rs_nkey_d2(key[K - 1]);
+        key[j] = rs_kmax(key[j - 1], rs_kmin(key[j], x));
+      key[0] = rs_kmin(key[0], x);
+      kth = (key[K - 1] == (double)INFINITY) ? INFINITY : rs_nkey_d2(key[K - 1]);
     };
+    float qlo[3] = {qx, qy, qz}, qhi[3] = {qx, qy, qz}; // the wave's queries' bounds (used if periodic)
+    if (A.periodic)
+#pragma unroll
+      for (int j = 0; j < 3; j++)
+      {
+#pragma unroll
+        for (int d = 1; d < HBTX_WAVE; d <<= 1)
+        {
+          qlo[j] = fminf(qlo[j], __shfl_xor(qlo[j], d, HBTX_WAVE));
+          qhi[j] = fmaxf(qhi[j], __shfl_xor(qhi[j], d, HBTX_WAVE));
+        }
+        qlo[j] = rd_lane(qlo[j], 0);
+        qhi[j] = rd_lane(qhi[j], 0);
+      }
     const float slack = A.periodic ? A.box * 2.5e-7f : 0.f;
     // A leaf's 32 tracers go through the wave's LDS.  First every lane screens all of
     // them with a float lower bound (each difference is rounded once, and wrapped with
@@ -632,7 +664,13 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_knn(RsArgs A, const int4 *__r
       wave_lds_sync();
       const float screen = kth * (1.0f + 4.4e-6f);
       uint32_t pass = 0u;
-      if (A.periodic)
+      // one of the leaf's tracers may be beyond half the box of one of the queries: else
+      // NEAREST changes no difference (periodic, k = 10, 3.8e6 particles: 3.6 ms with every
+      // pair wrapped, 2.2 so)
+      const bool wraps =
+        A.periodic && ballot(lane < n && !(r.x - qlo[0] <= A.half && r.x - qhi[0] >= -A.half && r.y - qlo[1] <= A.half &&
+                                           r.y - qhi[1] >= -A.half && r.z - qlo[2] <= A.half && r.z - qhi[2] >= -A.half));
+      if (wraps)
       {
 #pragma unroll 8
         for (int j = RS_LEAF - 1; j >= 0; j--)
@@ -662,10 +700,9 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_knn(RsArgs A, const int4 *__r
         pass &= pass - 1u;
         const float4 t = T.leaf[j];
         double dx, dy, dz;
-        const uint64_t x =
-          rs_nkey((float)rs_r2(t.x, t.y, t.z, qx, qy, qz, A, dx, dy, dz), __float_as_int(t.w));
-        if (x < key[K - 1])
-          insert(x);
+        const double d2 = wraps ? rs_r2(t.x, t.y, t.z, qx, qy, qz, A, true, dx, dy, dz)
+                                : rs_r2(t.x, t.y, t.z, qx, qy, qz, A, false, dx, dy, dz);
+        insert(rs_nkey((float)d2, __float_as_int(t.w)));
       }
     };
     // the leaves the queries' keys fall in
@@ -769,11 +806,12 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_knn(RsArgs A, const int4 *__r
     {
       je[j] = RS_RADII;
       se[j] = -1;
-      if (j >= K - k && key[j] != ~0ull)
+      if (j >= K - k && key[j] != (double)INFINITY)
       {
-        const int64_t p = (int32_t)(uint32_t)key[j];
+        const int64_t p = rs_nkey_pid(key[j]);
         double dx, dy, dz;
-        const double r2 = rs_r2(A.pos[3 * p], A.pos[3 * p + 1], A.pos[3 * p + 2], qx, qy, qz, A, dx, dy, dz);
+        const double r2 = rs_r2(A.pos[3 * p], A.pos[3 * p + 1], A.pos[3 * p + 2], qx, qy, qz, A, A.periodic, dx,
+                                dy, dz);
         int a = 0, b = RS_RADII - 1; // smallest index that collects it (the last entry always does)
         while (a < b)
         {
