@@ -34,6 +34,7 @@
 #include <sstream>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <numeric>
 #include <stdexcept>
@@ -138,6 +139,11 @@ struct DArr
     release();
   }
   DArr() = default;
+  void swap(DArr &o)
+  {
+    std::swap(p, o.p);
+    std::swap(n, o.n);
+  }
   DArr(const DArr &) = delete;
   DArr &operator=(const DArr &) = delete;
 };
@@ -237,21 +243,79 @@ struct View
   int32_t *type_cnt, *first_tracer;
 };
 
-struct hbtx_tree
+struct TreeBufs
 {
-  hbtx_ctx *ctx = nullptr;
+  DArr<float4> ent;
+  DArr<int32_t> eskip;
+  DArr<int8_t> ent_depth;
+  DArr<uint2> wt; // walk records of the tree
+  DArr<int32_t> src_of_entry;
+  DArr<double> cube;
+  size_t bytes() const
+  {
+    return ent.n * sizeof(float4) + (eskip.n + src_of_entry.n) * sizeof(int32_t) + ent_depth.n + wt.n * sizeof(uint2) +
+           cube.n * sizeof(double);
+  }
+  void swap(TreeBufs &o)
+  {
+    ent.swap(o.ent);
+    eskip.swap(o.eskip);
+    ent_depth.swap(o.ent_depth);
+    wt.swap(o.wt);
+    src_of_entry.swap(o.src_of_entry);
+    cube.swap(o.cube);
+  }
+};
+
+// The buffers of the last tree freed, for a context's next one: a program that builds a
+// tree, uses it and frees it spent 0.7 ms of a tree of 2e6 giving the buffers back and 0.3
+// getting them again (a free above some 100 MB unmaps).  One tree's, TREE_SPARE_MAX bytes
+// at most, given back with the context; a tree may be freed by any thread and after its
+// context.  Nothing is in flight on a freed tree: the calls that read one wait for
+// their results.
+#define TREE_SPARE_MAX ((size_t)512 << 20)
+struct TreeSpare
+{
+  std::mutex mu;
+  bool open = true;
+  TreeBufs bufs;
+
+  void take(TreeBufs &to)
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    to.swap(bufs);
+  }
+  void give(TreeBufs &from)
+  {
+    if (from.bytes() > TREE_SPARE_MAX)
+      return;
+    std::lock_guard<std::mutex> lock(mu);
+    if (open && from.bytes() > bufs.bytes())
+      bufs.swap(from);
+  }
+  void close()
+  {
+    TreeBufs drop; // (freed after the lock)
+    std::lock_guard<std::mutex> lock(mu);
+    open = false;
+    drop.swap(bufs);
+  }
+};
+
+struct hbtx_tree : TreeBufs
+{
+  std::shared_ptr<TreeSpare> spare;
   int64_t n = 0;
   int32_t ne = 0;
   int64_t ncells = 0;
   DevParams P;
-  DArr<float4> ent;
-  DArr<int32_t> eskip;
-  DArr<int8_t> ent_depth;
-  DArr<uint2> wt;   // walk records of the tree
-  int32_t nw = 0;   // their units
-  DArr<int32_t> src_of_entry;
-  DArr<double> cube;
+  int32_t nw = 0; // units of the walk records
   int32_t treemode = 1;
+  ~hbtx_tree()
+  {
+    if (spare)
+      spare->give(*this);
+  }
 };
 
 struct hbtx_mlp
@@ -284,6 +348,7 @@ struct hbtx_ctx
   hipStream_t stream = nullptr;
   std::string err;
   int num_cu = 256;
+  std::shared_ptr<TreeSpare> tree_spare;
   int walk_chunks = 8;          // item chunks of the walk (one per XCD)
   int64_t direct_cutoff = 1024; // sources at or below use the exact sum when params ask for the tuned value
   int walk_waves = 32;          // resident walk waves per CU (grid of the persistent walk)
@@ -1687,7 +1752,8 @@ void build_tree(hbtx_ctx *c, const hbtx_params &prm, int64_t n, const float *pos
   HIPCHK(hipStreamSynchronize(st));
   check_overflow(h_misc[2]);
   const int32_t ne = h_misc[3];
-  T->ctx = c;
+  T->spare = c->tree_spare;
+  T->spare->take(*T);
   T->n = n;
   T->ne = ne;
   T->ncells = ne - n;
@@ -1911,12 +1977,18 @@ int hbtx_create(hbtx_ctx **out, int device)
     HIPCHK(hipEventCreate(&c->wev0));
     HIPCHK(hipEventCreate(&c->wev1));
     c->stats.alloc(NSTATS);
+    c->tree_spare = std::make_shared<TreeSpare>();
   }
   catch (const Error &e)
   {
     int code = e.code;
     delete c;
     return code;
+  }
+  catch (const std::bad_alloc &)
+  {
+    delete c;
+    return HBTX_E_ALLOC;
   }
   *out = c;
   return HBTX_OK;
@@ -1929,6 +2001,7 @@ void hbtx_destroy(hbtx_ctx *c)
   (void)hipSetDevice(c->device);
   if (c->stream)
     (void)hipStreamSynchronize(c->stream);
+  c->tree_spare->close();
   if (c->ev0)
     (void)hipEventDestroy(c->ev0);
   if (c->ev1)
