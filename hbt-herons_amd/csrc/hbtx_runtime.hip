@@ -604,7 +604,8 @@ void run_profiles(hbtx_ctx *c, const hbtx_params &prm, ProfArgs &A, int64_t n, i
   const int rg = red_grid(c, n, nsub);
   k_prof_tile_sum<<<rg, RED_THREADS, 0, st>>>(A, c->red_tiles.p, nt);
   k_prof_tile_prefix<<<gs, 256, 0, st>>>(nsub, c->red_toff.p, c->red_ntile.p, c->red_partial.p);
-  k_prof_tile_main<<<rg, RED_THREADS, 0, st>>>(A, c->red_tiles.p, nt);
+  k_prof_tile_main<HBTX_WAVE><<<4 * rg, HBTX_WAVE, 0, st>>>(A, c->red_tiles.p, nt);
+  k_prof_tile_main<RED_THREADS><<<rg, RED_THREADS, 0, st>>>(A, c->red_tiles.p, nt);
   k_prof_finish<<<gs, 256, 0, st>>>(A, nsub, c->red_toff.p, c->red_ntile.p, out);
   HIPCHK(hipGetLastError());
 }

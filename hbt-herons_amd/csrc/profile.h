@@ -82,6 +82,7 @@ __global__ void k_prof_keys(ProfArgs A, int64_t n, const int32_t *sub_of, uint64
   }
 }
 
+#define PROF_ITEMS (RED_TILE / RED_THREADS)
 __global__ __launch_bounds__(RED_THREADS) void k_prof_tile_sum(ProfArgs A, const int4 *tiles, const int32_t *ntiles_p)
 {
   __shared__ double lds[RED_THREADS / HBTX_WAVE];
@@ -89,9 +90,20 @@ __global__ __launch_bounds__(RED_THREADS) void k_prof_tile_sum(ProfArgs A, const
   for (int t = blockIdx.x; t < nt; t += gridDim.x)
   {
     const int4 tl = tiles[t];
+    // (every load before the first sum: a thread's gathers are in flight together)
+    float w[PROF_ITEMS];
+    int p[PROF_ITEMS];
+#pragma unroll
+    for (int k = 0; k < PROF_ITEMS; k++)
+      p[k] = A.vals[min(tl.y + (int)threadIdx.x + k * RED_THREADS, tl.z - 1)];
+#pragma unroll
+    for (int k = 0; k < PROF_ITEMS; k++)
+      w[k] = A.posm[p[k]].w;
     double m = 0.;
-    for (int q = tl.y + threadIdx.x; q < tl.z; q += RED_THREADS)
-      m += (double)A.posm[A.vals[q]].w;
+#pragma unroll
+    for (int k = 0; k < PROF_ITEMS; k++)
+      if (tl.y + (int)threadIdx.x + k * RED_THREADS < tl.z)
+        m += (double)w[k];
     double tot;
     block_excl_scan(m, lds, &tot);
     if (threadIdx.x == 0)
@@ -105,61 +117,103 @@ __global__ void k_prof_tile_prefix(int32_t nsub, const int32_t *toff, const int3
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= nsub)
     return;
+  // (eight tiles' sums loaded ahead: the additions are the only chain)
   double run = 0.;
-  for (int t = toff[s]; t < toff[s] + ntile[s]; t++)
+  const int t1 = toff[s] + ntile[s];
+  for (int t = toff[s]; t < t1; t += 8)
   {
-    part[(int64_t)t * RED_NV + PROF_TPRE] = run;
-    run += part[(int64_t)t * RED_NV + PROF_TSUM];
+    double x[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      x[j] = part[(int64_t)min(t + j, t1 - 1) * RED_NV + PROF_TSUM];
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      if (t + j < t1)
+      {
+        part[(int64_t)(t + j) * RED_NV + PROF_TPRE] = run;
+        run += x[j];
+      }
   }
 }
 
-#define PROF_ITEMS (RED_TILE / RED_THREADS)
-__global__ __launch_bounds__(RED_THREADS) void k_prof_tile_main(ProfArgs A, const int4 *tiles, const int32_t *ntiles_p)
+// Bound: the gather of the sorted slots' particles (a 64-byte line each, twice).  The
+// tile's sorted arrays pass through LDS in whole lines (a thread sums 16 consecutive
+// slots, so its own loads and stores touched a line a slot), PROF_AHEAD gathers are in
+// flight together, and a tile of at most PROF_SHORT slots is one wave's, whose slots go to
+// all of its threads.  3.0e6 slots in 5,000 subhaloes: 186 us, so 105 for the long tiles
+// and 16 for the short ones.
+#define PROF_AHEAD 4
+#define PROF_SHORT 512
+template <int THREADS> // 64: tiles of at most PROF_SHORT slots, 256: longer ones
+__global__ __launch_bounds__(THREADS) void k_prof_tile_main(ProfArgs A, const int4 *tiles, const int32_t *ntiles_p)
 {
 #pragma clang fp contract(off) // float expressions rounded as written, as on the host
-  __shared__ double lds[RED_THREADS / HBTX_WAVE];
-  __shared__ double lsum[RED_THREADS / HBTX_WAVE][12];
-  __shared__ float lbv[RED_THREADS / HBTX_WAVE];
-  __shared__ int lbq[RED_THREADS / HBTX_WAVE], lso[RED_THREADS / HBTX_WAVE];
+  constexpr int NW = THREADS / HBTX_WAVE;
+  __shared__ double lds[NW];
+  __shared__ double lsum[NW][12];
+  __shared__ float lbv[NW];
+  __shared__ int lbq[NW], lso[NW];
+  // the tile's particles and radii, then its masses and radii (slot i at i + i / 16: a
+  // thread's consecutive slots without bank conflicts)
+  constexpr int CAP = (THREADS == HBTX_WAVE) ? PROF_SHORT : RED_TILE;
+  __shared__ uint32_t lv[CAP + CAP / 16], lr[CAP + CAP / 16];
+  auto at = [](int i) { return i + (i >> 4); };
   const int nt = *ntiles_p;
   const DevParams &P = A.P;
   const int w = threadIdx.x / HBTX_WAVE;
   for (int t = blockIdx.x; t < nt; t += gridDim.x)
   {
     const int4 tl = tiles[t];
+    if ((tl.z - tl.y <= PROF_SHORT) != (THREADS == HBTX_WAVE))
+      continue;
     const int s = tl.x;
     const int a = A.off[s];
     const int p0 = a + A.ford[a]; // the centre, left out of the shape sums (src/subhalo.cpp:262)
     const float *cen = A.res[s].mostbound_pos;
-    const int q0 = tl.y + PROF_ITEMS * threadIdx.x;
+    const int len = tl.z - tl.y;
+    for (int i = threadIdx.x; i < len; i += THREADS)
+    {
+      lv[at(i)] = (uint32_t)A.vals[tl.y + i];
+      lr[at(i)] = (uint32_t)A.keys[tl.y + i];
+    }
+    __syncthreads();
+    // consecutive slots, few a thread where the tile is short
+    const int items = (len + THREADS - 1) / THREADS;
+    const int i0 = items * threadIdx.x, i1 = min(i0 + items, len);
     double msum = 0.;
+    for (int i = i0; i < i1; i += PROF_AHEAD)
+    {
+      float wk[PROF_AHEAD];
 #pragma unroll
-    for (int k = 0; k < PROF_ITEMS; k++)
-      if (q0 + k < tl.z)
-        msum += (double)A.posm[A.vals[q0 + k]].w;
-    double tot;
-    double run = block_excl_scan(msum, lds, &tot) + A.part[(int64_t)t * RED_NV + PROF_TPRE];
+      for (int k = 0; k < PROF_AHEAD; k++)
+        wk[k] = A.posm[lv[at(min(i + k, i1 - 1))]].w;
+#pragma unroll
+      for (int k = 0; k < PROF_AHEAD; k++)
+        if (i + k < i1)
+          msum += (double)wk[k];
+    }
+    double tot, before;
+    if constexpr (THREADS == HBTX_WAVE)
+      before = wave_incl_scan(msum) - msum;
+    else
+      before = block_excl_scan(msum, lds, &tot);
+    double run = before + A.part[(int64_t)t * RED_NV + PROF_TPRE];
     double sh[12];
 #pragma unroll
     for (int k = 0; k < 12; k++)
       sh[k] = 0.;
     float bv = -1.f;
     int bq = 0x7fffffff, so = -1;
-    for (int k = 0; k < PROF_ITEMS; k++)
-    {
-      const int q = q0 + k;
-      if (q >= tl.z)
-        break;
-      const int p = A.vals[q];
-      const float4 x = A.posm[p];
+    auto slot = [&](int i, int p, float4 x, uint32_t rbits) {
+      const int q = tl.y + i;
       run += (double)x.w;
       const float m = (float)run;
-      float r = __uint_as_float((uint32_t)A.keys[q]);
+      float r = __uint_as_float(rbits);
       if (r < P.eps)
         r = P.eps;
       const float v = __fdiv_rn(m, r);
-      A.rc[q] = r;
-      A.mc[q] = m;
+      lr[at(i)] = __float_as_uint(r);
+      lv[at(i)] = __float_as_uint(m);
       if (v > bv)
       {
         bv = v;
@@ -192,14 +246,39 @@ __global__ __launch_bounds__(RED_THREADS) void k_prof_tile_main(ProfArgs A, cons
         sh[10] += (double)__fdiv_rn(d1 * d2, dr2);
         sh[11] += (double)__fdiv_rn(z2, dr2);
       }
+    };
+    for (int i = i0; i < i1; i += PROF_AHEAD)
+    {
+      int pk[PROF_AHEAD];
+      uint32_t rk[PROF_AHEAD];
+      float4 xk[PROF_AHEAD];
+#pragma unroll
+      for (int k = 0; k < PROF_AHEAD; k++)
+      {
+        pk[k] = (int)lv[at(min(i + k, i1 - 1))];
+        rk[k] = lr[at(min(i + k, i1 - 1))];
+      }
+#pragma unroll
+      for (int k = 0; k < PROF_AHEAD; k++)
+        xk[k] = A.posm[pk[k]];
+#pragma unroll
+      for (int k = 0; k < PROF_AHEAD; k++)
+        if (i + k < i1)
+          slot(i + k, pk[k], xk[k], rk[k]);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < len; i += THREADS)
+    {
+      A.rc[tl.y + i] = __uint_as_float(lr[at(i)]);
+      A.mc[tl.y + i] = __uint_as_float(lv[at(i)]);
     }
     // block: shape sums, the first largest v, the last overdense slot
 #pragma unroll
+    for (int k = 0; k < 12; k++)
+      sh[k] = wave_sum_down(sh[k]);
+#pragma unroll
     for (int d = 32; d >= 1; d >>= 1)
     {
-#pragma unroll
-      for (int k = 0; k < 12; k++)
-        sh[k] += __shfl_down(sh[k], d, HBTX_WAVE);
       const float ov = __shfl_down(bv, d, HBTX_WAVE);
       const int oq = __shfl_down(bq, d, HBTX_WAVE);
       if (ov > bv || (ov == bv && oq < bq))
@@ -225,13 +304,13 @@ __global__ __launch_bounds__(RED_THREADS) void k_prof_tile_main(ProfArgs A, cons
       for (int k = 0; k < 12; k++)
       {
         double x = 0.;
-        for (int ww = 0; ww < RED_THREADS / HBTX_WAVE; ww++)
+        for (int ww = 0; ww < NW; ww++)
           x += lsum[ww][k];
         o[PROF_SHAPE + k] = x;
       }
       float v = lbv[0];
       int q = lbq[0], sq = lso[0];
-      for (int ww = 1; ww < RED_THREADS / HBTX_WAVE; ww++)
+      for (int ww = 1; ww < NW; ww++)
       {
         if (lbv[ww] > v || (lbv[ww] == v && lbq[ww] < q))
         {
@@ -271,18 +350,38 @@ __global__ void k_prof_finish(ProfArgs A, int32_t nsub, const int32_t *toff, con
       sh[k] = 0.;
     float bv = -1.f;
     int bq = a, so = -1;
-    for (int t = toff[s]; t < toff[s] + ntile[s]; t++)
+    // (four tiles' partials loaded ahead)
+    const int t1 = toff[s] + ntile[s];
+    for (int t = toff[s]; t < t1; t += 4)
     {
-      const double *pt = A.part + (int64_t)t * RED_NV;
-      for (int k = 0; k < 12; k++)
-        sh[k] += pt[PROF_SHAPE + k];
-      const float v = (float)pt[PROF_BESTV];
-      if (v > bv)
+      double x[4][15];
+#pragma unroll
+      for (int j = 0; j < 4; j++)
       {
-        bv = v;
-        bq = (int)pt[PROF_BESTQ];
+        const double *pt = A.part + (int64_t)min(t + j, t1 - 1) * RED_NV;
+#pragma unroll
+        for (int k = 0; k < 12; k++)
+          x[j][k] = pt[PROF_SHAPE + k];
+        x[j][12] = pt[PROF_BESTV];
+        x[j][13] = pt[PROF_BESTQ];
+        x[j][14] = pt[PROF_SOQ];
       }
-      so = max(so, (int)pt[PROF_SOQ]);
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+      {
+        if (t + j >= t1)
+          break;
+#pragma unroll
+        for (int k = 0; k < 12; k++)
+          sh[k] += x[j][k];
+        const float v = (float)x[j][12];
+        if (v > bv)
+        {
+          bv = v;
+          bq = (int)x[j][13];
+        }
+        so = max(so, (int)x[j][14]);
+      }
     }
     o.rmax_comoving = A.rc[bq];
     o.vmax_physical = sqrtf(bv * A.vel_unit);
