@@ -28,58 +28,181 @@ namespace hbtx
 #define SORT_BLOCK_ITEMS 16
 #define SORT_BLOCK_MAX (SORT_BLOCK_THREADS * SORT_BLOCK_ITEMS)
 
+// v of the lane whose number differs in the bit X, by moves of the vector unit.
+template <int X>
+HBTX_DEV uint32_t lane_xor(uint32_t v)
+{
+  if constexpr (X == 1)
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, true); // quad_perm [1,0,3,2]
+  else if constexpr (X == 2)
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, true); // quad_perm [2,3,0,1]
+  else if constexpr (X == 4)
+  {
+    const int m = __builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, true); // row_half_mirror: lane ^ 7
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, m, 0x1B, 0xf, 0xf, true);    // quad_perm [3,2,1,0]: lane ^ 3
+  }
+  else if constexpr (X == 8)
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, true); // row_ror:8
+  else if constexpr (X == 16)
+  {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false); // the even rows twice, the odd ones
+    return (lane_id() & 16) ? r[0] : r[1];
+  }
+  else
+  {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false); // the lower half twice, the upper
+    return (lane_id() & 32) ? r[0] : r[1];
+  }
+}
+
+// One step of the network between lanes X apart: up, the pair's direction.
+template <int R, int X>
+HBTX_DEV void net_lanes(uint64_t (&key)[R], int32_t (&val)[R], bool up)
+{
+  const bool low = (lane_id() & X) == 0; // this lane holds the pairs' first elements
+#pragma unroll
+  for (int r = 0; r < R; r++)
+  {
+    const uint64_t ok =
+      ((uint64_t)lane_xor<X>((uint32_t)(key[r] >> 32)) << 32) | lane_xor<X>((uint32_t)key[r]);
+    const int32_t ov = (int32_t)lane_xor<X>((uint32_t)val[r]);
+    if ((low ? key[r] > ok : ok > key[r]) == up)
+    {
+      key[r] = ok;
+      val[r] = ov;
+    }
+  }
+}
+
+// The bitonic network over 256 R elements, element R t + r in register r of thread t:
+// pairs less than R apart meet in a thread's registers, less than 64 R apart through lane
+// moves, and only the three steps beyond that in LDS, between barriers.
+template <int R>
+HBTX_DEV void sort_net(uint64_t *__restrict__ keys, int32_t *__restrict__ vals, int len, uint64_t *sk, int32_t *sv)
+{
+  const int t = threadIdx.x;
+  uint64_t key[R];
+  int32_t val[R];
+#pragma unroll
+  for (int r = 0; r < R; r++)
+  {
+    const int e = R * t + r;
+    key[r] = (e < len) ? keys[e] : ~0ull;
+    val[r] = (e < len) ? vals[e] : 0;
+  }
+  for (int k = 2; k <= SORT_THREADS * R; k <<= 1)
+    for (int j = k >> 1; j > 0; j >>= 1)
+    {
+      const bool up_t = (t & (k / R)) == 0; // (k >= R: the direction of all the thread's elements)
+      if (j >= HBTX_WAVE * R)
+      {
+#pragma unroll
+        for (int r = 0; r < R; r++)
+        {
+          sk[r * SORT_THREADS + t] = key[r];
+          sv[r * SORT_THREADS + t] = val[r];
+        }
+        __syncthreads();
+        const int o = t ^ (j / R);
+#pragma unroll
+        for (int r = 0; r < R; r++)
+        {
+          const uint64_t ok = sk[r * SORT_THREADS + o];
+          const int32_t ov = sv[r * SORT_THREADS + o];
+          if ((t < o ? key[r] > ok : ok > key[r]) == up_t)
+          {
+            key[r] = ok;
+            val[r] = ov;
+          }
+        }
+        __syncthreads();
+      }
+      else if (j >= R)
+      {
+        switch (j / R)
+        {
+        case 1:
+          net_lanes<R, 1>(key, val, up_t);
+          break;
+        case 2:
+          net_lanes<R, 2>(key, val, up_t);
+          break;
+        case 4:
+          net_lanes<R, 4>(key, val, up_t);
+          break;
+        case 8:
+          net_lanes<R, 8>(key, val, up_t);
+          break;
+        case 16:
+          net_lanes<R, 16>(key, val, up_t);
+          break;
+        default:
+          net_lanes<R, 32>(key, val, up_t);
+        }
+      }
+      else
+      {
+#pragma unroll
+        for (int jr = 1; jr < R; jr <<= 1)
+          if (jr == j)
+          {
+#pragma unroll
+            for (int r = 0; r < R; r++)
+            {
+              const int r2 = r ^ jr;
+              if (r2 < r)
+                continue;
+              const bool up = (k < R) ? (r & k) == 0 : up_t;
+              if ((key[r] > key[r2]) == up)
+              {
+                const uint64_t tk = key[r];
+                key[r] = key[r2];
+                key[r2] = tk;
+                const int32_t tv = val[r];
+                val[r] = val[r2];
+                val[r2] = tv;
+              }
+            }
+          }
+      }
+    }
+#pragma unroll
+  for (int r = 0; r < R; r++)
+  {
+    const int e = R * t + r;
+    if (e < len)
+    {
+      keys[e] = key[r];
+      vals[e] = val[r];
+    }
+  }
+}
+
+// Segments of SORT_WAVE4_MAX + 1 .. SORT_SMALL_MAX elements, a workgroup each, padded to
+// 512, 1024 or 2048.  Through LDS and a barrier a step (45 to 66 steps): one segment of
+// 300, 18 us, the segments of a set of 1e6 particles 65 us a launch; by sort_net 13 and
+// 30 us.
 __global__ __launch_bounds__(SORT_THREADS) void k_sort_small(uint64_t *__restrict__ keys, int32_t *__restrict__ vals,
                                                             const int32_t *__restrict__ seg_begin,
                                                             const int32_t *__restrict__ seg_len, int32_t nseg)
 {
   __shared__ uint64_t sk[SORT_SMALL_MAX];
   __shared__ int32_t sv[SORT_SMALL_MAX];
-  const int tid = threadIdx.x;
   for (int s = blockIdx.x; s < nseg; s += gridDim.x)
   {
     const int len = seg_len[s];
     if (len <= SORT_WAVE4_MAX || len > SORT_SMALL_MAX)
       continue; // (segments of up to four per lane: k_sort_wave, k_sort_wave4)
     const int b = seg_begin[s];
-    int P = 1;
-    while (P < len)
-      P <<= 1;
-    for (int i = tid; i < P; i += SORT_THREADS)
-    {
-      sk[i] = (i < len) ? keys[b + i] : ~0ull;
-      sv[i] = (i < len) ? vals[b + i] : 0;
-    }
-    __syncthreads();
-    for (int k = 2; k <= P; k <<= 1)
-      for (int j = k >> 1; j > 0; j >>= 1)
-      {
-        for (int i = tid; i < P; i += SORT_THREADS)
-        {
-          const int ixj = i ^ j;
-          if (ixj > i)
-          {
-            const bool up = (i & k) == 0;
-            const uint64_t a = sk[i], c = sk[ixj];
-            if ((a > c) == up)
-            {
-              sk[i] = c;
-              sk[ixj] = a;
-              const int32_t t = sv[i];
-              sv[i] = sv[ixj];
-              sv[ixj] = t;
-            }
-          }
-        }
-        __syncthreads();
-      }
-    for (int i = tid; i < len; i += SORT_THREADS)
-    {
-      keys[b + i] = sk[i];
-      vals[b + i] = sv[i];
-    }
-    __syncthreads();
+    if (len <= 2 * SORT_THREADS)
+      sort_net<2>(keys + b, vals + b, len, sk, sv);
+    else if (len <= 4 * SORT_THREADS)
+      sort_net<4>(keys + b, vals + b, len, sk, sv);
+    else
+      sort_net<8>(keys + b, vals + b, len, sk, sv);
   }
 }
+static_assert(SORT_SMALL_MAX == 8 * SORT_THREADS, "sort_net's forms cover k_sort_small's segments");
 
 // Segments of at most one wave (the common case for small subhaloes): one wave per
 // segment, element i in lane i, the same bitonic network as k_sort_small (so the
