@@ -326,19 +326,41 @@ struct hbtx_mlp
   int64_t step = 0;
 };
 
-// What a captured round graph depends on besides buffer addresses.
+// What a segmented sort is made of, by its longest segment (seg_sort): each form sorts
+// the segments of the ones before it too, none a longer segment.
+enum SortForm
+{
+  SORT_FORM_WAVE,  // up to SORT_WAVE_MAX
+  SORT_FORM_WAVE4, // up to SORT_WAVE4_MAX
+  SORT_FORM_SMALL, // up to SORT_SMALL_MAX
+  SORT_FORM_BLOCK, // up to SORT_BLOCK_MAX
+  SORT_FORM_TILED
+};
+inline SortForm sort_form(int64_t max_len)
+{
+  return max_len <= SORT_WAVE_MAX    ? SORT_FORM_WAVE
+         : max_len <= SORT_WAVE4_MAX ? SORT_FORM_WAVE4
+         : max_len <= SORT_SMALL_MAX ? SORT_FORM_SMALL
+         : max_len <= SORT_BLOCK_MAX ? SORT_FORM_BLOCK
+                                     : SORT_FORM_TILED;
+}
+
+// What a captured round graph depends on besides buffer addresses: all that the host
+// decides launches and arguments from.  (Buffers stay from load to load, so a batch of
+// other subhaloes may meet the graphs of the one before.)
 struct GraphKey
 {
   uint64_t gen = ~0ull;
   int64_t p0 = -1, n = -1;
   int32_t s0 = -1, nsub = -1;
+  int32_t sort = -1; // form of the source sort (SortForm of the largest subhalo)
   const void *ptype = nullptr, *proposal = nullptr;
   int32_t ent_cap = -1;
   DevParams P;
   bool operator==(const GraphKey &o) const
   {
-    return gen == o.gen && p0 == o.p0 && n == o.n && s0 == o.s0 && nsub == o.nsub && ptype == o.ptype &&
-           proposal == o.proposal && ent_cap == o.ent_cap && std::memcmp(&P, &o.P, sizeof(P)) == 0;
+    return gen == o.gen && p0 == o.p0 && n == o.n && s0 == o.s0 && nsub == o.nsub && sort == o.sort &&
+           ptype == o.ptype && proposal == o.proposal && ent_cap == o.ent_cap && std::memcmp(&P, &o.P, sizeof(P)) == 0;
   }
 };
 
@@ -496,7 +518,8 @@ void seg_sort(hbtx_ctx *c, uint64_t *keys, int32_t *vals, int32_t nseg, const R 
   // passes for all of them (with a larger segment's passes to be launched in any case,
   // those of 2,049 to 16,384 ride along: three sorts of 8e6 slots 960 us, and 1,160 with the
   // shorter segments in a workgroup each).
-  const bool radix = max_len > SORT_BLOCK_MAX, block = !radix && max_len > SORT_SMALL_MAX;
+  const SortForm form = sort_form(max_len);
+  const bool radix = form == SORT_FORM_TILED, block = form == SORT_FORM_BLOCK;
   if (radix || block)
     list_tiles(c, r, nseg, radix ? SORT_TILE : SORT_BLOCK_MAX, SORT_SMALL_MAX, false, c->sort_ntile.p, c->sort_toff.p,
                c->sort_tiles.p, seg_begin, seg_len);
@@ -505,10 +528,10 @@ void seg_sort(hbtx_ctx *c, uint64_t *keys, int32_t *vals, int32_t nseg, const R 
                                                                          (int32_t *)nullptr, seg_begin, seg_len);
   k_sort_wave<<<std::max(1, std::min((nseg + 3) / 4, 16384)), SORT_THREADS, 0, c->stream>>>(keys, vals, seg_begin,
                                                                                             seg_len, nseg);
-  if (max_len > SORT_WAVE_MAX)
+  if (form > SORT_FORM_WAVE)
     k_sort_wave4<<<std::max(1, std::min((nseg + 3) / 4, 16384)), SORT_THREADS, 0, c->stream>>>(keys, vals, seg_begin,
                                                                                               seg_len, nseg);
-  if (max_len > SORT_WAVE4_MAX)
+  if (form > SORT_FORM_WAVE4)
     k_sort_small<<<std::max(1, std::min(nseg, 16384)), SORT_THREADS, 0, c->stream>>>(keys, vals, seg_begin, seg_len,
                                                                                       nseg);
   HIPCHK(hipGetLastError());
@@ -1423,6 +1446,7 @@ bool ensure_round_graphs(hbtx_ctx *c, Batch &B, View &V, const DevParams &P, int
   k.n = V.n;
   k.s0 = V.s0;
   k.nsub = V.nsub;
+  k.sort = sort_form(V.max_count);
   k.ptype = V.Q.ptype;
   k.proposal = V.Q.proposal;
   k.ent_cap = B.ent_cap;
