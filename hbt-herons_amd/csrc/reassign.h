@@ -645,6 +645,9 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_knn(RsArgs A, const int4 *__r
         qhi[j] = rd_lane(qhi[j], 0);
       }
     const float slack = A.periodic ? A.box * 2.5e-7f : 0.f;
+    // NEAREST goes by the exact difference, the leaf's question below by its float rounding:
+    // a difference beyond half the box by less than that would be taken for half the box
+    const float inner = 0.999f * A.half;
     // A leaf's 32 tracers go through the wave's LDS.  First every lane screens all of
     // them with a float lower bound (each difference is rounded once, and wrapped with
     // an error below the float spacing of box, the sum once more: the screen is widened
@@ -668,8 +671,8 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_knn(RsArgs A, const int4 *__r
       // NEAREST changes no difference (periodic, k = 10, 3.8e6 particles: 3.6 ms with every
       // pair wrapped, 2.2 so)
       const bool wraps =
-        A.periodic && ballot(lane < n && !(r.x - qlo[0] <= A.half && r.x - qhi[0] >= -A.half && r.y - qlo[1] <= A.half &&
-                                           r.y - qhi[1] >= -A.half && r.z - qlo[2] <= A.half && r.z - qhi[2] >= -A.half));
+        A.periodic && ballot(lane < n && !(r.x - qlo[0] <= inner && r.x - qhi[0] >= -inner && r.y - qlo[1] <= inner &&
+                                           r.y - qhi[1] >= -inner && r.z - qlo[2] <= inner && r.z - qhi[2] >= -inner));
       if (wraps)
       {
 #pragma unroll 8
