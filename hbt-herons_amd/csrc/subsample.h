@@ -146,7 +146,7 @@ __global__ void k_init_mass_finish(SubArrays S, PartArrays Q, DevParams P, const
     S.warm[s] = WARM_PENDING;
     S.npro[s] = (int)v[1];
     // (periodic: the wrapped mean offset from the first proposed particle, added back)
-    const float4 r0 = P.periodic ? Q.posm[S.first_idx[s]] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 r0 = (P.periodic && v[1] > 0.) ? Q.posm[S.first_idx[s]] : make_float4(0.f, 0.f, 0.f, 0.f);
     const double o[3] = {r0.x, r0.y, r0.z};
     for (int k = 0; k < 3; k++)
     {

@@ -944,9 +944,12 @@ __global__ void k_round_finish_periodic(SubArrays S, PartArrays Q, DevParams P, 
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= S.nsub || S.mode[s] == MODE_IDLE || S.status[s] == ST_DISRUPTED)
     return;
+  const int first = S.first_idx[s];
+  if (first == 0x7fffffff)
+    return; // nothing is bound (after a warm round k_warm_reset_subs sets the frame)
   const double *v = red + (int64_t)s * RED_NV;
   const double M = v[0];
-  const float4 r0 = Q.posm[S.first_idx[s]];
+  const float4 r0 = Q.posm[first];
   S.ref[6 * s + 0] = (float)(v[1] / M + (double)r0.x);
   S.ref[6 * s + 1] = (float)(v[2] / M + (double)r0.y);
   S.ref[6 * s + 2] = (float)(v[3] / M + (double)r0.z);
