@@ -215,6 +215,7 @@ struct Batch
   DArr<uint32_t> bbox;
   DArr<int32_t> misc; // [0] active, [1] (unused), [2] overflow, [3] entry total, [4] max depth
   DArr<int32_t> wctr; // walk work counters
+  int small_loads = 0; // loads in a row that the entry buffers are far too large for
   DArr<char2> lev;                // per dense source: the level pair of its tree
   DArr<int32_t> mom_slots;        // moment passes: per window / group, the cells that end beyond it
   DArr<hbtx_sub_result> dres;
@@ -729,6 +730,28 @@ int64_t entry_bound(int64_t n)
 
 void grow_entries(Batch &B, int64_t need, bool slack);
 
+// Entry buffers (49 bytes an entry, some ten entries a particle where rounds are
+// replayed) serve the batches that follow: made anew at each load they cost a program of
+// large batches gigabytes of allocations and frees a call.  They are given back once ENTRY_SMALL_LOADS loads in
+// a row could do with an eighth of them, so that a small batch between large ones does
+// not cost the large ones theirs.
+#define ENTRY_SMALL_LOADS 16
+#define ENTRY_KEEP ((size_t)1 << 20) // entries that are kept in any case
+void bound_entries(Batch &B)
+{
+  const size_t need = (size_t)std::max<int64_t>(3 * B.n + 64, B.ent_bound);
+  const bool small = B.ent.n > ENTRY_KEEP && B.ent.n / 8 > need;
+  B.small_loads = small ? B.small_loads + 1 : 0;
+  if (B.small_loads < ENTRY_SMALL_LOADS)
+    return;
+  B.small_loads = 0;
+  B.ent.release();
+  B.eskip.release();
+  B.ent_depth.release();
+  B.wt.release();
+  B.cell_u.release();
+}
+
 void batch_reserve(hbtx_ctx *c, Batch &B)
 {
   const int64_t n = B.n;
@@ -766,6 +789,7 @@ void batch_reserve(hbtx_ctx *c, Batch &B)
   B.flag64.alloc(n + 1);
   B.keys.alloc(n);
   B.lev.alloc(n + 1);
+  bound_entries(B);
   grow_entries(B, std::min<int64_t>(3 * n + 64, WREC_MAX_ENTRIES), false);
   B.items.alloc(n / HBTX_WAVE + ns + 1);
   B.icnt.alloc(ns + 1);
