@@ -365,6 +365,45 @@ struct GraphKey
   }
 };
 
+// Workspaces of the calls that take host arrays, reused across calls.  Up to WS_KEEP_MAX
+// bytes together they stay (20 million targets of a tree, 30 million samples of the
+// classifier); a call that needed more gives them all back when it ends (WsUse).
+#define WS_KEEP_MAX ((size_t)1 << 30)
+struct Workspaces
+{
+  DArr<float> raw; // the arrays as uploaded
+  DArr<float4> tgt, posm;
+  DArr<double> phi;
+  DArr<uint64_t> keys;
+  DArr<int32_t> vals, seg, counter, off, sub_of, local;
+  DArr<hbtx_sub_result> res;
+  DArr<float> rc, mc, X;
+  DArr<uint8_t> y;
+  DArr<hbtx_sub_profile> prof;
+
+  template <class F>
+  void each(F &&f)
+  {
+    f(raw), f(tgt), f(posm), f(phi), f(keys), f(vals), f(seg), f(counter), f(off), f(sub_of), f(local), f(res), f(rc),
+      f(mc), f(X), f(y), f(prof);
+  }
+  void bound()
+  {
+    size_t bytes = 0;
+    each([&](auto &a) { bytes += a.n * sizeof(*a.p); });
+    if (bytes > WS_KEEP_MAX)
+      each([](auto &a) { a.release(); });
+  }
+};
+struct WsUse // of one call
+{
+  Workspaces &ws;
+  ~WsUse()
+  {
+    ws.bound();
+  }
+};
+
 struct hbtx_ctx
 {
   int device = 0;
@@ -402,20 +441,8 @@ struct hbtx_ctx
   int graph_rounds = 0, graph_captures = 0;
   int64_t tree_entries = 0, tree_entries_first = 0; // octree entries built, all rounds / first round
   Batch B;
-  // workspaces of the calls that take host arrays (grow-only, reused across calls)
-  struct
-  {
-    DArr<float> raw;            // the arrays as uploaded
-    DArr<float4> tgt, posm;
-    DArr<double> phi;
-    DArr<uint64_t> keys;
-    DArr<int32_t> vals, seg, counter, off, sub_of, local;
-    DArr<hbtx_sub_result> res;
-    DArr<float> rc, mc, X;
-    DArr<uint8_t> y;
-    DArr<hbtx_sub_profile> prof;
-  } ws;
-  // particle reassignment buffers (likewise)
+  Workspaces ws;
+  // particle reassignment buffers (grow-only, reused across calls)
   struct
   {
     DArr<float> pos, radii;
@@ -1854,6 +1881,7 @@ void tree_points(hbtx_ctx *c, hbtx_tree *T, int64_t nt, const float *tpos, const
     return;
   hipStream_t st = c->stream;
   auto &W = c->ws;
+  WsUse use{W};
   W.raw.alloc(4 * nt);
   W.tgt.alloc(nt);
   W.phi.alloc(nt);
@@ -2453,6 +2481,7 @@ int hbtx_profiles(hbtx_ctx *c, const hbtx_params *prm, int64_t n, const float *p
     }
     hoff[nsub] = (int32_t)n;
     auto &W = c->ws;
+    WsUse use{W};
     const int64_t n1 = std::max<int64_t>(n, 1);
     W.raw.alloc(4 * n1);
     W.posm.alloc(n1);
@@ -2830,6 +2859,7 @@ int hbtx_mlp_gradient(hbtx_ctx *c, hbtx_mlp *M, int64_t n, const float *X, const
   API_GUARD(c, {
     HIPCHK(hipSetDevice(c->device));
     hipStream_t st = c->stream;
+    WsUse use{c->ws};
     mlp_samples(c, n, X, y);
     auto &dX = c->ws.X;
     auto &dy = c->ws.y;
@@ -2853,6 +2883,7 @@ int hbtx_mlp_train(hbtx_ctx *c, hbtx_mlp *M, int64_t n, const float *X, const ui
     HIPCHK(hipSetDevice(c->device));
     REQUIRE(n < (int64_t)0x7fffffff, HBTX_E_INVALID, "too many training samples");
     hipStream_t st = c->stream;
+    WsUse use{c->ws};
     mlp_samples(c, n, X, y);
     auto &dX = c->ws.X;
     auto &dy = c->ws.y;
@@ -2907,6 +2938,7 @@ int hbtx_mlp_predict(hbtx_ctx *c, hbtx_mlp *M, int64_t n, const float *X, float 
     if (n == 0)
       return HBTX_OK;
     hipStream_t st = c->stream;
+    WsUse use{c->ws};
     mlp_samples(c, n, X, nullptr);
     auto &dX = c->ws.X;
     auto &dl = c->ws.rc;

@@ -37,3 +37,26 @@ def test_entry_buffers_after_a_large_batch():
             assert np.array_equal(got[k], want[k])
     finally:
         c.close()
+
+
+def test_workspaces_after_a_large_call():
+    src = np.random.default_rng(3).normal(0, 0.1, (200, 3)).astype(np.float32)
+    one = np.ones(200, np.float32)
+    tgt = np.tile(src, (110_000, 1))  # 22 million targets: 52 bytes each
+    c = hbtx.Context(0)
+    try:
+        tree = c.tree(src, one, hbtx.workload_params())
+        before = hbtx.device_bytes()
+        got = tree.potential(tgt)
+        # (the sort's scratch stays: 12 bytes a target and its tiles' counts, less than half as much)
+        assert hbtx.device_bytes() - before < (1 << 29)
+        # (another order of the terms in plain FP32 sums of about 16: 2^-24 each, both sides)
+        want = tree.potential(src)
+        assert np.allclose(got.reshape(-1, 200), want, rtol=3e-6)
+        # a small call keeps what it made
+        held = hbtx.device_bytes()
+        tree.potential(src)
+        assert hbtx.device_bytes() == held
+        tree.close()
+    finally:
+        c.close()
