@@ -1855,9 +1855,13 @@ void build_tree(hbtx_ctx *c, const hbtx_params &prm, int64_t n, const float *pos
 
 // Potentials at A's targets: the tree walk, or the exact sum over the records.
 // The exact sum takes several waves per 64 targets up to DS_ITEMS_PER_CU times 64
-// targets a CU; beyond that one wave per 64 targets keeps the chip as full, without
-// the exchange (20,011 sources, one wave against several: 30,001 targets 2087 and
-// 227 us, 131,072 targets 1382 and 957 us, 262,144 targets 1753 and 1971 us).
+// targets a CU (196,608 on 256 CUs); beyond that one wave per 64 targets keeps the chip as
+// full, without the exchange.  One wave against several, us:
+//   targets            30,001      131,072      196,608      262,144      400,000
+//   500 sources       71,   29     72,   56     85,   72     97,   87    122,  121
+//   2,000            233,   45    170,  126    180,  173    216,  221    289,  322
+//   20,011          2131,  241   1368,  968   1560, 1393   1781, 1834   2400, 2743
+// (30,001 targets are 469 waves' worth for 468 waves: one of them takes two.)
 #define DS_ITEMS_PER_CU 12
 template <bool PERIODIC, bool STATS>
 void launch_points(hbtx_ctx *c, const PointArgs &A)

@@ -114,6 +114,11 @@ __global__ __launch_bounds__(WALK_WG_THREADS, 8) void k_points_potential(PointAr
 #define DS_WAVES 8
 #define DS_GROUPS 8
 #define DS_THREADS (HBTX_WAVE * (DS_WAVES + 1))
+// Records from which on a block asks whether any of its pairs can wrap: the targets'
+// bounds (36 lane exchanges) cost more than they can save on fewer.  2,000 periodic
+// targets, asked and not: 10 sources away from the box faces 24.1 and 23.2 us (about a
+// face 24.9 and 23.5), 32 sources 25.5 and 26.1, 200 sources 26.4 and 27.9.
+#define DS_SCREEN_MIN 32
 template <bool PERIODIC, bool STATS>
 __global__ __launch_bounds__(DS_THREADS) void k_points_direct(PointArgs A)
 {
@@ -136,8 +141,9 @@ __global__ __launch_bounds__(DS_THREADS) void k_points_direct(PointArgs A)
       x = A.tgt[ti];
     Kahan acc;
     acc.init();
-    const bool wraps = PERIODIC && __syncthreads_or(records_may_wrap(ent, threadIdx.x, DS_THREADS, ee, valid, x.x, x.y,
-                                                                     x.z, A.P));
+    const bool wraps =
+      PERIODIC && (ee < DS_SCREEN_MIN || __syncthreads_or(records_may_wrap(ent, threadIdx.x, DS_THREADS, ee, valid, x.x,
+                                                                           x.y, x.z, A.P)));
     // stage st is formed in buffer st & 1 while stage st - 1 is added from the other
     for (int st = 0; st <= nstage; st++)
     {
