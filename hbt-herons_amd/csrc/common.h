@@ -83,20 +83,6 @@ struct DevParams
 // first entry after the cell's subtree; a particle's is its own index + 1).
 // The walk reads its own compact records, built alongside.
 
-// Loads through the constant address space: a wave-uniform index then becomes a
-// scalar (s_load) access.  Only for buffers that no kernel writes while it reads them.
-HBTX_DEV float4 const_load(const float4 *p, int i)
-{
-  typedef const __attribute__((address_space(4))) float cf;
-  const cf *q = (const cf *)(uintptr_t)(p + i);
-  return make_float4(q[0], q[1], q[2], q[3]);
-}
-HBTX_DEV int2 const_load(const int2 *p, int i)
-{
-  typedef const __attribute__((address_space(4))) int ci;
-  const ci *q = (const ci *)(uintptr_t)(p + i);
-  return make_int2(q[0], q[1]);
-}
 // Walk records: the walk's own copy of every tree, in the entries' depth-first
 // order but packed into 8-byte units.  A particle takes two units {x, y, z, m};
 // a cell three {x, y, z, m with the sign bit set, crit2, rskip}, rskip in bytes
@@ -105,7 +91,9 @@ HBTX_DEV int2 const_load(const int2 *p, int i)
 // is never opened.  Packing the particles into 16 bytes shrinks a tree's walk
 // footprint by almost half against the 32-byte entries.
 
-// a particle record (x, y, z, m) at an 8-byte aligned unit, through the scalar path
+// A particle record (x, y, z, m) at an 8-byte aligned unit, through the constant address
+// space: a wave-uniform address then becomes a scalar load.  Only for buffers that no kernel
+// writes while it reads them.
 HBTX_DEV float4 const_load_f4u(const uint2 *p)
 {
   typedef int v4i __attribute__((ext_vector_type(4)));

@@ -1129,7 +1129,6 @@ WalkArgs walk_args(hbtx_ctx *c, Batch &B, View &V, const DevParams &P)
   W.energy = V.Q.energy;
   W.esl = V.Q.esl;
   W.eref = B.eref.p + V.p0;
-  W.phi_out = nullptr;
   W.stats = c->stats.p;
   W.overflow = B.misc.p + 2;
   W.P = P;
@@ -1912,8 +1911,7 @@ void tree_points(hbtx_ctx *c, hbtx_tree *T, int64_t nt, const float *tpos, const
   A.treemode = T->treemode;
   A.cube = T->cube.p;
   A.wt = T->wt.p;
-  A.phi = nullptr;
-  A.phi_d = W.phi.p;
+  A.phi = W.phi.p;
   A.counter = W.counter.p;
   A.chunks = POINT_CHUNKS;
   A.stats = c->stats.p;
@@ -2417,8 +2415,7 @@ int hbtx_direct_potential_noalloc(hbtx_ctx *c, const hbtx_params *prm, int64_t n
       A.treemode = 0;
       A.cube = nullptr;
       A.wt = wt;
-      A.phi = nullptr;
-      A.phi_d = d_out_pot;
+      A.phi = d_out_pot;
       A.counter = counter; // (the scratch array holds one)
       A.chunks = 1;
       A.stats = nullptr;

@@ -15,8 +15,7 @@ struct PointArgs
   int32_t treemode;
   const double *cube;      // the tree's root cube (centre, half side)
   const uint2 *wt;         // walk records
-  float *phi;              // specific potential, scattered to the target's input index, or null
-  double *phi_d;           // optional double output
+  double *phi;             // specific potential, scattered to the target's input index
   int32_t *counter;        // work counters (ItemQueue), zeroed before launch
   int32_t chunks;          // item list split into this many contiguous chunks
   unsigned long long *stats;
@@ -29,11 +28,7 @@ HBTX_DEV void store_potential(const PointArgs &A, float tgt_mass, const Kahan &a
   if (!valid)
     return;
   const float self = tgt_mass / A.P.eps;
-  const double phi = ((double)self + (double)acc.s - (double)acc.c) * A.P.G_over_a;
-  if (A.phi)
-    A.phi[ti] = (float)phi;
-  if (A.phi_d)
-    A.phi_d[ti] = phi;
+  A.phi[ti] = ((double)self + (double)acc.s - (double)acc.c) * A.P.G_over_a;
 }
 
 template <bool PERIODIC, bool STATS>

@@ -156,16 +156,6 @@ __global__ void k_rs_groups(RsArgs A)
   }
 }
 
-HBTX_DEV void rs_wave_min_max(float &mn, float &mx)
-{
-#pragma unroll
-  for (int d = 1; d < HBTX_WAVE; d <<= 1)
-  {
-    mn = fminf(mn, __shfl_xor(mn, d, HBTX_WAVE));
-    mx = fmaxf(mx, __shfl_xor(mx, d, HBTX_WAVE));
-  }
-}
-
 // Pass 2 over particles: tracer / non-tracer lists (stable), box of the tracers'
 // offsets and largest |offset| per host halo.  A block takes RS_CHUNK consecutive
 // particles; every thread keeps running extrema for the host halo it is in and

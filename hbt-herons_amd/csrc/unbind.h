@@ -67,10 +67,6 @@ __global__ void k_publish(const int32_t *src, int32_t *dst, int n)
   if ((int)threadIdx.x < n)
     dst[threadIdx.x] = src[threadIdx.x];
 }
-__global__ void k_fill_u64(unsigned long long *p, int64_t n, unsigned long long v)
-{
-  GRID_STRIDE(i, n) p[i] = v;
-}
 
 // Batch start: every particle is a candidate, frame from the caller
 // (src/subhalo_unbind.cpp:503-541).

@@ -55,7 +55,6 @@ struct WalkArgs
   float *energy;
   float *esl;               // the same energies by slot (off[s] + target index)
   float *eref;              // refinement energies (MODE_REFINE targets)
-  float *phi_out;           // optional: specific potential per particle (float), may be null
   unsigned long long *stats;
   int32_t *overflow;        // the round's overflow word (WALK_STACK_OVERFLOW)
   DevParams P;
@@ -728,8 +727,6 @@ __global__ __launch_bounds__(WALK_WG_THREADS, 8) void k_walk_energy(WalkArgs A)
     const int md = A.mode[s];
     const float self = (md == MODE_FULL || md == MODE_REFINE || md == MODE_ADD) ? (A.selfm[p] / P.eps) : 0.f;
     const double phi = ((double)self + (double)acc.s - (double)acc.c) * P.G_over_a;
-    if (A.phi_out)
-      A.phi_out[p] = (float)phi;
     const float4 v = A.velu[p];
     const float *rf = A.ref + 6 * s;
     if (md == MODE_FULL || md == MODE_REFINE)
