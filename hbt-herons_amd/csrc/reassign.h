@@ -64,7 +64,7 @@ struct RsArgs
   int32_t *qtiles_n;     // [G+1] wave tiles per host halo, then their scan
   uint64_t *tkey, *qkey; // sorted keys
   int32_t *tval, *qval;  // particle index per sorted slot
-  int32_t *seg;          // [4G]: tracer begins | tracer counts | query begins | query counts
+  int32_t *seg;          // [6G]: tracer begins | tracer counts | query begins | query counts | the sort's ranges
   float4 *trec;          // [nt]
   float4 *nodes;         // 2 per node: lo, hi
   const int64_t *lbase;  // [RS_LEVELS] first node of every level

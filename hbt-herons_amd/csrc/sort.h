@@ -1,12 +1,12 @@
 // Segmented sort of (uint64 key, int32 value) pairs.
-//  * segments of <= SORT_WAVE_MAX elements: one wave each, bitonic sort in lanes;
+//  * segments of <= SORT_WAVE4_MAX elements: one wave each, bitonic sort in lanes;
 //  * segments of <= SORT_SMALL_MAX elements: one workgroup each, the same bitonic
-//    network in LDS;
+//    network in registers, lane moves and three steps through LDS;
 //  * where no segment is longer than SORT_BLOCK_MAX, those above: one workgroup each, a
 //    stable LSD radix sort whose passes stay in registers and LDS (the order of the next);
-//  * else the segments above SORT_SMALL_MAX: tiled LSD radix sort (8- or 9-bit digits, whichever needs
-//    fewer passes) where every tile of SORT_TILE elements ranks its keys stably
-//    with wave ballots (match of the digit bits) and LDS per-digit counters, so
+//  * else the segments above SORT_SMALL_MAX: tiled LSD radix sort (8- or 9-bit digits,
+//    whichever needs fewer passes) where every tile of SORT_TILE elements ranks its keys
+//    stably with wave ballots (match of the digit bits) and LDS per-digit counters, so
 //    all large segments advance together in one launch per pass.
 #pragma once
 #include "common.h"

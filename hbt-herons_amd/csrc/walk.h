@@ -79,11 +79,12 @@ constexpr int WALK_WG_THREADS = HBTX_WAVE * HBTX_WALK_WG_WAVES;
 // a tree, stay on one XCD's L2), then helps with the others.  The wave that finds a chunk
 // empty first sets its bit in the word after the counters, and a wave looking for
 // another chunk reads that word before it touches a counter.  With a failed addition on
-// each of eight counters a wave, which are served one after the other, 8,192 waves spent
-// longer on ending than a round of small items takes: walks of 1.2e6 particles in
-// subhaloes of at most 2,000, 0.89 ms, 0.47 so; in subhaloes up to a million, 2.1e6
-// particles 2.12 and 1.72 ms, 8e6 5.08 and 4.74.  (More counters than one an XCD made it worse, 5.9 ms of 8e6: a wave that
-// looks for work then reads them all, and they are what the others are adding to.)
+// every chunk's counter a wave, which are served one after the other, 8,192 waves spent
+// longer on ending than a round of small items takes: walks (16 chunks, the tuned number)
+// of 1.2e6 particles in subhaloes of at most 2,000, 0.89 ms, 0.47 so; in subhaloes up to a
+// million, 2.1e6 particles 2.12 and 1.72 ms, 8e6 5.08 and 4.74.  (Several counters a chunk
+// made it worse, 5.9 ms of 8e6: a wave that looks for work then reads them all, and they
+// are what the others are adding to.)
 #define QUEUE_STRIDE 32 // ints between counters: a cache line each
 struct ItemQueue
 {

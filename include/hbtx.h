@@ -5,6 +5,13 @@
  * Host arrays are owned by the caller; a context owns device buffers, its HIP
  * stream and its cached graphs.  One context per host thread.
  *
+ * Device buffers stay with the context from call to call and are given back by
+ * hbtx_destroy: the arrays of its largest batch and of its largest reassignment,
+ * the octree entries of its batches (given back earlier, after sixteen batches in a row
+ * that need an eighth of them), up to 1 GiB of workspaces of the other calls
+ * that take host arrays, the last freed tree's buffers (up to 512 MiB), and 32
+ * MiB of pinned host memory.  hbtx_device_bytes tells how much device memory that is.
+ *
  * Reference interfaces replaced (paths relative to the reference repository):
  *   hbtx_unbind_batch        Subhalo_t::Unbind(const Snapshot_t&)        src/subhalo.h:152, src/subhalo_unbind.cpp:463-808
  *                            (per subhalo, HBTX_PLAIN) and the batch loop of
